@@ -359,8 +359,9 @@ def run(state):
         p.run(c["iters"])
         return p.get_volume()
     if kind == "recon":
-        return mesolf_amd.recon_theory_phase_space_LFM_with_filter(
+        vol = mesolf_amd.recon_theory_phase_space_LFM_with_filter(
             state["image"], state["H"], state["Ht"], c["iters"], True, 1, precision=c["prec"])
+        return vol.astype(np.float32)  # the drop-in's doubles hold single-precision values
     if kind == "batch":
         for p, im in zip(state["patches"], state["images"]):
             p.set_image(im)
