@@ -166,21 +166,42 @@ hipError_t launch_postprocess(const float* X, int n1, int n2, int Z, double* coe
 // MEX operator (mex:43-266).
 hipError_t launch_mex_conv(const float* in, int64_t W, int64_t H, int64_t n, const float* K, int kw,
                            float* out, hipStream_t st);
-// MFMA form of the MEX operator for odd kw (clipping == zero padding); Kq is
-// a scratch of mex_kq_floats(kw) floats (the per-phase-row GEMM operand).
+// MFMA forms of the MEX operator for odd kw (clipping == zero padding): the
+// BF16 split form (mex_split.hip) where its 32-bit offsets reach, with the FP32
+// form behind it for bitmaps or kernels holding values that it leaves, or the
+// FP32 form alone.  One call has one scratch of mex_scratch_floats(kw) floats,
+// whose first kMexFlagFloats floats were zero when it was allocated and are
+// written by these launches only.
 constexpr int kMexMfmaMaxKw = 511;
-size_t mex_kq_floats(int kw);
-hipError_t launch_mex_mfma(const float* in, int64_t W, int64_t H, int64_t n, const float* K, int kw,
-                           float* Kq, float* out, hipStream_t st);
+constexpr int kMexFlagFloats = 64;
+size_t mex_scratch_floats(int kw);
+struct MexCall {
+  float* scratch = nullptr;     // operand table of the kernel set in use
+  int kw = 0;
+  const float* scan = nullptr;  // bitmaps still to be looked through
+  size_t nscan = 0;
+  int* flag = nullptr;          // null: the FP32 form alone
+  int gen = 0;                  // number of the call, stored in *flag to leave it to the FP32 form
+};
+// A call on `images` bitmaps [W, H] at `in`.
+MexCall mex_begin(int64_t W, int64_t H, int64_t images, int kw, const float* in, float* scratch);
+// out[j] = MEX(in[j], K) for j < n, or with lists out[dst[j]] += MEX(in[src[j]], K)
+// (dst distinct within a launch); new_kernel: K differs from the launch before.
+hipError_t launch_mex_mfma(MexCall& c, const float* in, int64_t W, int64_t H, int64_t n, const float* K,
+                           bool new_kernel, const int32_t* src, const int32_t* dst, float* out,
+                           hipStream_t st);
+// The split form (mex_split.hip).
+bool mex_split_takes(int64_t W, int64_t H, int64_t images, int kw);
+size_t mex_split_bytes(int kw);
+int mex_next_call();
+hipError_t launch_mex_split_prep(const float* K, int kw, void* Bt, const float* scan, size_t nscan, int* flag,
+                                 int gen, hipStream_t st);
+hipError_t launch_mex_split(const float* in, int64_t W, int64_t H, int64_t n, const void* Bt, int kw,
+                            const int32_t* src, const int32_t* dst, float* out, const int* flag, int gen,
+                            hipStream_t st);
 // Device address of the no-allocation MEX scratch on `device` (the device
 // must be current), resolved once per device at context creation.
 mlf_status noalloc_scratch_init(int device);
-// Kq of one kernel set K [kw][kw][15][15] (for launch_mex_mfma_list).
-hipError_t launch_mex_kq(const float* K, int kw, float* Kq, hipStream_t st);
-// out[dst[j]] += MEX(in[src[j]], K) for j < n (dst distinct within a launch).
-hipError_t launch_mex_mfma_list(const float* in, int64_t W, int64_t H, int64_t n, const float* Kq,
-                                int kw, const int32_t* src, const int32_t* dst, float* out,
-                                hipStream_t st);
 // out[s] = sum over j in [seg_ptr[s], seg_ptr[s+1]) of MEX(in[order[j]], K[plane[order[j]]]),
 // added in j order; K is [Z][15][15][kw][kw].
 hipError_t launch_mex_conv_segments(const float* in, int64_t W, int64_t H, const int32_t* plane,

@@ -5,6 +5,8 @@
 // h = kw/2, zero outside the bitmap; the tap window is clipped exactly as
 // mex_lfm_convolution_vec.cu:55-78 clips it (for even kw the last column/row
 // tap is dropped near the right/bottom edge).
+#include <algorithm>
+
 #include "internal.h"
 
 namespace mlf {
@@ -122,7 +124,9 @@ __global__ __launch_bounds__(kTileX* kTileY) void k_mex_conv_segments(
 // 32 lenslet columns (two M-tiles).  Per chunk of kMexCK input rows it stages
 // the images' rows and the chunk's Kq rows (T4 x 16 floats per row, read with
 // 16-byte loads, shared by every wave) in LDS; each Kq fragment read from LDS
-// feeds the MFMAs of both M-tiles.  Measured on the seed-library loop
+// feeds the MFMAs of both M-tiles.  This is the form for values that the BF16
+// split form (mex_split.hip) leaves and for bitmaps beyond its 32-bit offsets.
+// Measured on the seed-library loop
 // (396 x 396, kw = 241): 7.37 s with these settings (11.8 + 16 KB of LDS per
 // workgroup at kw = 241); Kq fragments from L2 instead: 9.60 s with one image
 // per wave, 8.27 s with two (three 9.52, four 10.76 s); two input rows per
@@ -134,7 +138,11 @@ constexpr int kMexThreads = 64 * kMexImg / kMexImgW;  // one wave per kMexImgW i
 constexpr int kMexCK = 1;
 constexpr int kMexCols = 32;  // lenslet columns per workgroup (2 M-tiles)
 
-__global__ void k_mex_kq(const float* __restrict__ K, int kw, int T4, float* __restrict__ Kq) {
+// flag != null: the launch does its work only if *flag == gen (the split form
+// of mex_split.hip has left the call to this one).
+__global__ void k_mex_kq(const float* __restrict__ K, int kw, int T4, float* __restrict__ Kq,
+                         const int* __restrict__ flag, int gen) {
+  if (flag && *flag != gen) return;
   const size_t total = (size_t)kN * kw * T4 * 16;
   for (size_t o = blockIdx.x * (size_t)blockDim.x + threadIdx.x; o < total;
        o += (size_t)gridDim.x * blockDim.x) {
@@ -156,7 +164,9 @@ __global__ __launch_bounds__(kMexThreads) void k_mex_mfma(const float* __restric
                                                   const float* __restrict__ Kq, int kw, int T4,
                                                   float* __restrict__ out,
                                                   const int32_t* __restrict__ src,
-                                                  const int32_t* __restrict__ dst) {
+                                                  const int32_t* __restrict__ dst,
+                                                  const int* __restrict__ flag, int gen) {
+  if (flag && *flag != gen) return;
   extern __shared__ float xs[];  // [kMexCK][kMexImg][XL], then the chunk's Kq rows [kMexCK][T4][16]
   const int y = blockIdx.x, ng = blockIdx.y, ib = blockIdx.z;
   const int q = y % kN, h = kw / 2;
@@ -223,20 +233,20 @@ __global__ __launch_bounds__(kMexThreads) void k_mex_mfma(const float* __restric
 
 }  // namespace
 
-size_t mex_kq_floats(int kw) {
+static size_t mex_kq_floats(int kw) {
   const int T4 = (kw + kN - 1 + 3) / 4 * 4;
   return (size_t)kN * kw * T4 * 16;
 }
 
-hipError_t launch_mex_kq(const float* K, int kw, float* Kq, hipStream_t st) {
+static hipError_t launch_kq(const float* K, int kw, float* Kq, const int* flag, int gen, hipStream_t st) {
   const int T4 = (kw + kN - 1 + 3) / 4 * 4;
-  hipLaunchKernelGGL(k_mex_kq, dim3(1024), dim3(256), 0, st, K, kw, T4, Kq);
+  hipLaunchKernelGGL(k_mex_kq, dim3(1024), dim3(256), 0, st, K, kw, T4, Kq, flag, gen);
   return hipGetLastError();
 }
 
-hipError_t launch_mex_mfma_list(const float* in, int64_t W, int64_t H, int64_t n, const float* Kq,
-                                int kw, const int32_t* src, const int32_t* dst, float* out,
-                                hipStream_t st) {
+static hipError_t launch_mfma(const float* in, int64_t W, int64_t H, int64_t n, const float* Kq, int kw,
+                              const int32_t* src, const int32_t* dst, float* out, const int* flag, int gen,
+                              hipStream_t st) {
   const int T4 = (kw + kN - 1 + 3) / 4 * 4;
   const int XL = kN * kMexCols + T4;
   const size_t shmem = sizeof(float) * kMexCK * (kMexImg * XL + T4 * 16);
@@ -246,24 +256,46 @@ hipError_t launch_mex_mfma_list(const float* in, int64_t W, int64_t H, int64_t n
   dim3 grid((unsigned)H, (unsigned)((n + kMexImg - 1) / kMexImg),
             (unsigned)((W / kN + 1 + kMexCols - 1) / kMexCols));
   hipLaunchKernelGGL(k_mex_mfma, grid, dim3(kMexThreads), shmem, st, in, (int)W, (int)H, (int)n, Kq, kw, T4,
-                     out, src, dst);
+                     out, src, dst, flag, gen);
   return hipGetLastError();
 }
 
-hipError_t launch_mex_mfma(const float* in, int64_t W, int64_t H, int64_t n, const float* K, int kw,
-                           float* Kq, float* out, hipStream_t st) {
-  const int T4 = (kw + kN - 1 + 3) / 4 * 4;
-  hipLaunchKernelGGL(k_mex_kq, dim3(1024), dim3(256), 0, st, K, kw, T4, Kq);
-  const int XL = kN * kMexCols + T4;
-  const size_t shmem = sizeof(float) * kMexCK * (kMexImg * XL + T4 * 16);
-  static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_mex_mfma),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-  if (attr != hipSuccess) return attr;
-  dim3 grid((unsigned)H, (unsigned)((n + kMexImg - 1) / kMexImg),
-            (unsigned)((W / kN + 1 + kMexCols - 1) / kMexCols));
-  hipLaunchKernelGGL(k_mex_mfma, grid, dim3(kMexThreads), shmem, st, in, (int)W, (int)H, (int)n, Kq, kw, T4,
-                     out, nullptr, nullptr);
-  return hipGetLastError();
+size_t mex_scratch_floats(int kw) {
+  return kMexFlagFloats + std::max(mex_kq_floats(kw), mex_split_bytes(kw) / sizeof(float));
+}
+
+MexCall mex_begin(int64_t W, int64_t H, int64_t images, int kw, const float* in, float* scratch) {
+  MexCall c;
+  c.scratch = scratch + kMexFlagFloats;
+  c.kw = kw;
+  c.scan = in;
+  c.nscan = (size_t)W * H * images;
+  if (mex_split_takes(W, H, images, kw)) {
+    c.flag = reinterpret_cast<int*>(scratch);
+    c.gen = mex_next_call();
+  }
+  return c;
+}
+
+hipError_t launch_mex_mfma(MexCall& c, const float* in, int64_t W, int64_t H, int64_t n, const float* K,
+                           bool new_kernel, const int32_t* src, const int32_t* dst, float* out,
+                           hipStream_t st) {
+  if (c.flag) {
+    if (new_kernel) {
+      const hipError_t e = launch_mex_split_prep(K, c.kw, c.scratch, c.scan, c.nscan, c.flag, c.gen, st);
+      if (e != hipSuccess) return e;
+      c.nscan = 0;  // the bitmaps are looked through once per call
+    }
+    const hipError_t e = launch_mex_split(in, W, H, n, c.scratch, c.kw, src, dst, out, c.flag, c.gen, st);
+    if (e != hipSuccess) return e;
+  }
+  // the whole call without the split form, and behind it for values that it
+  // leaves (the operand then takes the place of the split form's table)
+  if (new_kernel) {
+    const hipError_t e = launch_kq(K, c.kw, c.scratch, c.flag, c.gen, st);
+    if (e != hipSuccess) return e;
+  }
+  return launch_mfma(in, W, H, n, c.scratch, c.kw, src, dst, out, c.flag, c.gen, st);
 }
 
 hipError_t launch_mex_conv_segments(const float* in, int64_t W, int64_t H, const int32_t* plane,

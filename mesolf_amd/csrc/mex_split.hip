@@ -1,0 +1,436 @@
+// MEX operator for odd kernel widths on the BF16 matrix pipe at FP32 precision.
+//
+// As in k_mex_mfma (mex_kernels.hip), outputs grouped by phase make the operator a
+// GEMM: for output row y (q = y % 15), image n and x = 15 i + p
+//   out = sum_{ky, t} in[15 i + t - h, y - h + ky, n] * K[t - p, ky, p, q].
+// Every FP32 operand is split into three BF16 parts, x = x0 + x1 + x2 exactly
+// (8 + 8 + 8 significand bits, each part rounded to nearest), and a product
+// takes the six MFMAs x0 k0, x0 k1, x1 k0, x1 k1, x0 k2, x2 k0, all into one
+// FP32 accumulator; the three left out are below 2^-24 of the product.  Six
+// 16x16x32 BF16 MFMAs take 96 cycles where the FP32 pipe takes 256, and the
+// accumulator is rounded 6 times per 32 taps instead of 8 or more times.
+// Bound by the matrix pipe.  396 x 396 x 96, kw = 241: 8.85 ms, 1.19e15 BF16
+// flop/s issued for the products alone (FP32 MFMA, k_mex_mfma: 26.8 ms); 24
+// segments over 5 planes of that size: 7.9 ms (23.9); one 150 x 137 bitmap,
+// kw = 61: 35 us (229: one wave in eight had work).  Relative L2 error against
+// FP64 there: 5.7e-7 / 2.2e-7 / 7.2e-8 (FP32 MFMA 8.2e-7 / 7.9e-7 / 6.1e-7).
+//
+// Operand layout.  A lenslet's 15 pixels take 16 slots (slot 15 zero), so tap
+// t = 15 L + s - b sits at slot s of lenslet i - a + L (h = 15 a - b) and the
+// A fragment of a lane -- 8 consecutive slots of one lenslet -- is one aligned
+// 16-byte LDS read, for any alignment of h.  M rows are the cells (image, i)
+// counted through all images, so ragged widths waste no rows; the cells that a
+// workgroup's rows read are consecutive too and are staged once per input row
+// (split on the way).  N = 15 phases (16) of G output rows that share the
+// input row, each with its own kernel row: G rows reuse one A fragment.
+// The kernel side is a table of ready fragments built once per call
+// (k_mex_split_prep) and copied to LDS by buffer loads.
+//
+// A value that BF16 cannot round without overflow (infinities, NaN, the last
+// 2^-9 below FLT_MAX) would turn the products of its parts into NaN: the prep
+// kernel looks for one and stores the call's number in *flag, and then this
+// kernel leaves the call to k_mex_mfma, launched behind it.
+#include <algorithm>
+#include <atomic>
+
+#include "internal.h"
+
+namespace mlf {
+
+namespace {
+
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+
+constexpr int kMaxL = 40;  // lenslets (16 slots) per kernel row, even: kw <= kMexMfmaMaxKw
+constexpr int kDword3 = 0x00020000;  // raw buffer resource, 32-bit data format
+
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+__device__ __forceinline__ unsigned pk(float lo, float hi) {
+  const unsigned short a = __builtin_bit_cast(unsigned short, (__bf16)lo);
+  const unsigned short b = __builtin_bit_cast(unsigned short, (__bf16)hi);
+  return (unsigned)a | ((unsigned)b << 16);
+}
+// two values -> their three parts, packed in pairs
+__device__ __forceinline__ void split2(float x, float y, unsigned* w) {
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    w[k] = pk(x, y);
+    x -= __builtin_bit_cast(float, w[k] << 16);
+    y -= __builtin_bit_cast(float, w[k] & 0xFFFF0000u);
+  }
+}
+// |x| rounds to infinity in BF16 (or is not finite)
+__device__ __forceinline__ bool too_large(float x) {
+  return (__builtin_bit_cast(unsigned, x) & 0x7FFFFFFFu) >= 0x7F7F8000u;
+}
+
+struct SplitGeo {
+  int W, H, n;   // bitmap columns, rows, images of the launch
+  int kw, h;     // kernel width and half width
+  int nL;        // lenslets per bitmap row
+  int a;         // lenslets left of an output's own that its kernel reaches
+  int nks;       // K-steps (lenslet pairs) per kernel row
+  int nyg, nmb;  // output row groups, M blocks
+};
+
+// Fragment table Bt[q][ky][ks][part][lane][8]: lane (p = lane % 16, lg = lane / 16)
+// holds slots 8 (lg % 2) .. + 7 of lenslet L = 2 ks + lg / 2.  The blocks past
+// nbt look through `nscan` input values.
+__global__ __launch_bounds__(256) void k_mex_split_prep(const float* __restrict__ K, int kw, int b, int nks,
+                                                        uintx4* __restrict__ Bt, int nbt,
+                                                        const float* __restrict__ scan, size_t nscan,
+                                                        int* __restrict__ flag, int gen) {
+  bool bad = false;
+  if ((int)blockIdx.x < nbt) {
+    const size_t total = (size_t)kN * kw * nks * 64;
+    for (size_t o = blockIdx.x * (size_t)256 + threadIdx.x; o < total; o += (size_t)nbt * 256) {
+      const int lane = (int)(o & 63), p = lane & 15, lg = lane >> 4;
+      const size_t blk = o >> 6;  // (q kw + ky) nks + ks
+      const int ks = (int)(blk % nks);
+      const int ky = (int)((blk / nks) % kw);
+      const int q = (int)(blk / ((size_t)nks * kw));
+      const int kx0 = kN * (2 * ks + (lg >> 1)) + 8 * (lg & 1) - p - b;
+      const float* row = K + (size_t)kw * ky + (size_t)kw * kw * (min(p, kN - 1) + kN * q);
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int kx = kx0 + e;
+        const float t = row[min(max(kx, 0), kw - 1)];
+        bad = bad || too_large(t);
+        v[e] = (p < kN && kx >= 0 && kx < kw && 8 * (lg & 1) + e < kN) ? t : 0.f;
+      }
+      unsigned w[4][3];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) split2(v[2 * e], v[2 * e + 1], w[e]);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) Bt[(blk * 3 + k) * 64 + lane] = uintx4{w[0][k], w[1][k], w[2][k], w[3][k]};
+    }
+  } else {
+    const size_t nb = gridDim.x - nbt;
+    const size_t step = nb * 256;
+    size_t o = (blockIdx.x - nbt) * (size_t)256 + threadIdx.x;
+    for (; o + 3 * step < nscan; o += 4 * step) {
+      const float v0 = scan[o], v1 = scan[o + step], v2 = scan[o + 2 * step], v3 = scan[o + 3 * step];
+      bad = bad || too_large(v0) || too_large(v1) || too_large(v2) || too_large(v3);
+    }
+    for (; o < nscan; o += step) bad = bad || too_large(scan[o]);
+  }
+  if (bad) *flag = gen;
+}
+
+// WM waves along M times WK groups that share the input rows (row j goes to
+// group j % WK; the groups' accumulators are added in group order at the
+// end), MT M-tiles per wave, G output rows, SPB K-steps per barrier.
+template <int WM, int WK, int MT, int G, int SPB>
+struct SplitShape {
+  static constexpr int kThreads = 64 * WM * WK;
+  static constexpr int kRows = 16 * MT * WM;       // M rows (cells) per workgroup
+  static constexpr int kSlots = kRows + kMaxL + 1;  // staged cells, the last always zero
+  static constexpr int kHalf = kSlots * 16;         // bytes of one 8-slot half of all cells
+  static constexpr int kPart = 2 * kHalf;
+  static constexpr int kA = 3 * kPart;              // one input row, three parts
+  static constexpr int kB = SPB * G * 3 * 1024;     // one stage of kernel fragments
+  static constexpr int kGroup = 2 * kA + 2 * kB;
+  static constexpr int kLds = WK * kGroup;
+  static_assert(kLds <= 160 * 1024, "LDS");
+  static_assert((WK - 1) * WM * MT * G * 1024 <= kLds, "reduction buffer");
+};
+
+template <int WM, int WK, int MT, int G, int SPB>
+__global__ __launch_bounds__(64 * WM * WK) void k_mex_split(const float* __restrict__ in, SplitGeo g,
+                                                            const uintx4* __restrict__ Bt, float* __restrict__ out,
+                                                            const int32_t* __restrict__ src,
+                                                            const int32_t* __restrict__ dst,
+                                                            const int* __restrict__ flag, int gen) {
+  using S = SplitShape<WM, WK, MT, G, SPB>;
+  constexpr int NTH = 64 * WM;  // threads of a group
+  constexpr int NU = (S::kSlots * 8 + NTH - 1) / NTH;  // pixel pairs staged per thread and row
+  extern __shared__ __align__(16) char sm[];
+  if (uni(*flag) == gen) return;
+  const int W = g.W, H = g.H, nL = g.nL;
+  const int tid = threadIdx.x, lane = tid & 63, w = uni(tid >> 6), lr = lane & 15, lg = lane >> 4;
+  const int wk = w / WM, wm = w % WM, gt = tid - wk * NTH;
+  char* const Ab = sm + wk * S::kGroup;
+  char* const Bb = Ab + 2 * S::kA;
+  // Workgroups of one row group share its kernel fragments: blockIdx % 8 is
+  // the XCD, so they take consecutive turns on one XCD.  Groups in the middle
+  // of the bitmap, whose kernels are cut by no border, start first.
+  const int bx = blockIdx.x, turn = bx >> 3;
+  const int rank = (turn / g.nmb) * 8 + (bx & 7), mb = turn % g.nmb;
+  if (rank >= g.nyg) return;
+  const int yg = (rank & 1) ? g.nyg / 2 - (rank + 1) / 2 : g.nyg / 2 + rank / 2;
+  const int y0 = G * yg;
+  const int M0 = mb * S::kRows, NC = g.n * nL;
+
+  // staged pairs: pixels 15 lens + 2 k, + 1 (k = 7: pixel 14 and the zero slot)
+  const int pk8 = gt & 7;
+  const int ncell = S::kRows + 2 * g.nks - 1;
+  int off[NU];
+  unsigned ok = 0;
+#pragma unroll
+  for (int u = 0; u < NU; ++u) {
+    const int c = M0 - g.a + (gt >> 3) + u * (NTH / 8);
+    const bool in0 = (gt >> 3) + u * (NTH / 8) < ncell && c >= 0 && c < NC;
+    const int img = in0 ? c / nL : 0, x = kN * (in0 ? c - img * nL : 0) + 2 * pk8;
+    const bool ok0 = in0 && x < W, ok1 = ok0 && pk8 < 7 && x + 1 < W;
+    off[u] = ok0 ? (src ? src[img] : img) * W * H + x : 0;
+    ok |= (unsigned)ok0 << u | (unsigned)ok1 << (u + 16);
+  }
+  static_assert(NU <= 16, "mask bits");
+  float v0[NU], v1[NU];
+  auto load_row = [&](int r) {
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      const float* s = in + (size_t)(off[u] + r * W);
+      v0[u] = s[0];
+      v1[u] = s[(ok >> (u + 16)) & 1];
+    }
+  };
+  auto store_row = [&](char* A) {
+    char* d = A + (pk8 >> 2) * S::kHalf + (gt >> 3) * 16 + (pk8 & 3) * 4;
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      if ((gt >> 3) + u * (NTH / 8) >= ncell) continue;
+      unsigned p[3];
+      split2((ok >> u) & 1 ? v0[u] : 0.f, (ok >> (u + 16)) & 1 ? v1[u] : 0.f, p);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) *reinterpret_cast<unsigned*>(d + u * (NTH / 8) * 16 + k * S::kPart) = p[k];
+    }
+  };
+  if (gt < 12)  // the zero slot of each buffer, part and half
+    *reinterpret_cast<uintx4*>(Ab + (gt / 6) * S::kA + (gt % 6) * S::kHalf + (S::kSlots - 1) * 16) = uintx4{0, 0, 0, 0};
+
+  // this lane's A rows
+  int lens[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) lens[m] = (M0 + 16 * (wm * MT + m) + lr) % nL - g.a + (lg >> 1);
+  const int slot0 = 16 * wm * MT + lr + (lg >> 1);
+
+  floatx4 acc[MT][G];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int i = 0; i < G; ++i) acc[m][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+  const int rlo = max(0, y0 - g.h), rhi = min(H - 1, y0 + G - 1 + g.h);
+  const int nj = (rhi - rlo + WK) / WK;       // rows per group
+  const int ns = (g.nks + SPB - 1) / SPB;     // stages per row
+  const __amdgpu_buffer_rsrc_t br = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uintx4*>(Bt), 0, kN * g.kw * g.nks * 3 * 1024, kDword3);
+  int q15[G];
+#pragma unroll
+  for (int i = 0; i < G; ++i) q15[i] = (y0 + i) % kN;
+  auto issue_b = [&](int r, int s, char* buf) {
+#pragma unroll
+    for (int c0 = 0; c0 < SPB * G * 3; c0 += WM) {
+      const int c = c0 + wm;
+      if (c >= SPB * G * 3) break;  // wave-uniform
+      const int part = c % 3, i = (c / 3) % G, kk = c / (3 * G);
+      const int ky = min(max(r - y0 - i + g.h, 0), g.kw - 1);  // rows outside the kernel are copied, not used
+      const int ks = min(s * SPB + kk, g.nks - 1);
+      const int o = (((q15[i] * g.kw + ky) * g.nks + ks) * 3 + part) * 1024;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(br, (__attribute__((address_space(3))) void*)(buf + c * 1024), 16,
+                                               lane * 16, uni(o), 0, 0);
+    }
+  };
+
+  issue_b(rlo + wk, 0, Bb);
+  load_row(min(rlo + wk, H - 1));
+  store_row(Ab);
+  int t = 0;
+  for (int j = 0; j < nj; ++j) {
+    const int r = rlo + j * WK + wk;
+    const char* A = Ab + (j & 1) * S::kA;
+    unsigned use = 0;  // output rows whose kernel holds this input row
+#pragma unroll
+    for (int i = 0; i < G; ++i) {
+      const int ky = r - y0 - i + g.h;
+      use |= (unsigned)(r <= rhi && y0 + i < H && ky >= 0 && ky < g.kw) << i;
+    }
+    use = uni(use);
+    for (int s = 0; s < ns; ++s, ++t) {
+      // this stage's copies and the row's staged cells are in LDS, and every
+      // wave is done with the buffers that are written next
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
+      const bool lastrow = j + 1 >= nj;
+      if (!(lastrow && s + 1 >= ns)) issue_b(s + 1 < ns ? r : r + WK, s + 1 < ns ? s + 1 : 0, Bb + ((t + 1) & 1) * S::kB);
+      if (s == 0 && !lastrow) load_row(min(r + WK, H - 1));
+      if (s == 1 && !lastrow) store_row(Ab + ((j + 1) & 1) * S::kA);
+      const char* B = Bb + (t & 1) * S::kB + lane * 16;
+#pragma unroll
+      for (int kk = 0; kk < SPB; ++kk) {
+        const int ks = s * SPB + kk;
+        if (ks >= g.nks || !use) continue;
+        bf16x8 a[MT][3];
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          const bool v = (unsigned)(lens[m] + 2 * ks) < (unsigned)nL;
+          const char* p = A + (lg & 1) * S::kHalf + (v ? slot0 + 16 * m + 2 * ks : S::kSlots - 1) * 16;
+#pragma unroll
+          for (int k = 0; k < 3; ++k) a[m][k] = *reinterpret_cast<const bf16x8*>(p + k * S::kPart);
+        }
+#pragma unroll
+        for (int i = 0; i < G; ++i) {
+          if (!((use >> i) & 1)) continue;
+          bf16x8 b[3];
+#pragma unroll
+          for (int k = 0; k < 3; ++k) b[k] = *reinterpret_cast<const bf16x8*>(B + ((kk * G + i) * 3 + k) * 1024);
+          constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+          for (int q = 0; q < 6; ++q)
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+              acc[m][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m][pa[q]], b[pb[q]], acc[m][i], 0, 0, 0);
+        }
+      }
+      if (ns == 1 && !lastrow) store_row(Ab + ((j + 1) & 1) * S::kA);
+    }
+  }
+
+  if constexpr (WK > 1) {
+    __syncthreads();
+    floatx4* red = reinterpret_cast<floatx4*>(sm);
+    if (wk > 0) {
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int i = 0; i < G; ++i) red[((((wk - 1) * WM + wm) * MT + m) * G + i) * 64 + lane] = acc[m][i];
+    }
+    __syncthreads();
+    if (wk > 0) return;
+#pragma unroll
+    for (int k = 0; k < WK - 1; ++k)
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int i = 0; i < G; ++i) acc[m][i] += red[(((k * WM + wm) * MT + m) * G + i) * 64 + lane];
+  }
+  if (lr >= kN) return;
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int c = M0 + 16 * (wm * MT + m) + 4 * lg + j;
+      if (c >= NC) continue;
+      const int img = c / nL, x = kN * (c - img * nL) + lr;
+      if (x >= W) continue;
+      float* o = out + (size_t)(dst ? dst[img] : img) * W * H + x;
+#pragma unroll
+      for (int i = 0; i < G; ++i) {
+        if (y0 + i >= H) continue;
+        float* d = o + (size_t)(y0 + i) * W;
+        *d = dst ? *d + acc[m][i][j] : acc[m][i][j];
+      }
+    }
+}
+
+typedef void (*SplitKernel)(const float*, SplitGeo, const uintx4*, float*, const int32_t*, const int32_t*, const int*,
+                            int);
+struct SplitVariant {
+  SplitKernel fn;
+  int wm, wk, mt, g, spb, lds;
+};
+template <int WM, int WK, int MT, int G, int SPB>
+SplitVariant variant() {
+  return {&k_mex_split<WM, WK, MT, G, SPB>, WM, WK, MT, G, SPB, SplitShape<WM, WK, MT, G, SPB>::kLds};
+}
+
+}  // namespace
+
+static int split_lenslets(int kw, int* a, int* b) {
+  const int h = kw / 2;
+  *a = (h + kN - 1) / kN;
+  *b = kN * *a - h;
+  return (kw + 13 + *b) / kN + 1;
+}
+
+static int split_nks(int kw) {
+  int a, b;
+  return (split_lenslets(kw, &a, &b) + 1) / 2;
+}
+
+bool mex_split_takes(int64_t W, int64_t H, int64_t images, int kw) {
+  // 32-bit element offsets into the bitmaps and the M row count
+  return kw % 2 == 1 && kw <= kMexMfmaMaxKw && (double)W * H * images < 2147483648.0 && split_nks(kw) * 2 <= kMaxL;
+}
+
+size_t mex_split_bytes(int kw) { return (size_t)kN * kw * split_nks(kw) * 3 * 1024; }
+
+int mex_next_call() {
+  static std::atomic<int> calls{0};
+  return ++calls;
+}
+
+hipError_t launch_mex_split_prep(const float* K, int kw, void* Bt, const float* scan, size_t nscan, int* flag,
+                                 int gen, hipStream_t st) {
+  int a, b;
+  split_lenslets(kw, &a, &b);
+  const int nks = split_nks(kw);
+  const size_t total = (size_t)kN * kw * nks * 64;
+  const int nbt = (int)std::min<size_t>((total + 255) / 256, 4096);
+  const int nbs = nscan ? (int)std::min<size_t>((nscan + 1023) / 1024, 2048) : 0;
+  hipLaunchKernelGGL(k_mex_split_prep, dim3(nbt + nbs), dim3(256), 0, st, K, kw, b, nks, (uintx4*)Bt, nbt, scan,
+                     nscan, flag, gen);
+  return hipGetLastError();
+}
+
+// The shape with the least estimated time: matrix or LDS cycles of a
+// workgroup's longest group, times the rounds that 256 CUs need (every shape
+// fills a CU's LDS).  396 x 396, kw = 241: 96 bitmaps take <8, 1, 3, 4, 2> (162
+// M-tiles in blocks of 24: 693 workgroups, 2.7 rounds; blocks of 32 would pad
+// them by a fifth), 17 bitmaps <2, 4, 2, 2, 1> or <4, 2, 2, 4, 1>, one small
+// bitmap <1, 8, 1, 1, 1> (eight waves share the kernel's rows).
+hipError_t launch_mex_split(const float* in, int64_t W, int64_t H, int64_t n, const void* Bt, int kw,
+                            const int32_t* src, const int32_t* dst, float* out, const int* flag, int gen,
+                            hipStream_t st) {
+  static const SplitVariant variants[] = {
+      variant<8, 1, 4, 4, 2>(), variant<8, 1, 3, 4, 2>(), variant<8, 1, 2, 4, 2>(), variant<4, 2, 4, 4, 1>(),
+      variant<4, 2, 3, 4, 1>(), variant<4, 2, 2, 4, 1>(), variant<2, 4, 2, 2, 1>(), variant<1, 8, 2, 1, 1>(),
+      variant<1, 8, 1, 1, 1>(),
+  };
+  static const hipError_t attr = [] {
+    for (const SplitVariant& v : variants) {
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(v.fn),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }();
+  if (attr != hipSuccess) return attr;
+  SplitGeo g;
+  int b;
+  g.W = (int)W;
+  g.H = (int)H;
+  g.n = (int)n;
+  g.kw = kw;
+  g.h = kw / 2;
+  g.nL = (int)((W + kN - 1) / kN);
+  (void)split_lenslets(kw, &g.a, &b);
+  g.nks = split_nks(kw);
+  const int64_t cells = n * g.nL;
+  const SplitVariant* best = nullptr;
+  double best_t = 0.0;
+  for (const SplitVariant& v : variants) {
+    const int64_t wgs = (H + v.g - 1) / v.g * ((cells + 16 * v.mt * v.wm - 1) / (16 * v.mt * v.wm));
+    const double rows = (double)std::min<int64_t>(H, kw + v.g - 1) / v.wk;
+    const double mfma = 2.0 * 6 * 16 * v.mt * v.g, lds = 8.0 * 8 * 3 * (v.mt + v.g);
+    const double t = (double)((wgs + 255) / 256) * (rows * (g.nks * std::max(mfma, lds) + 400.0 * ((g.nks + v.spb - 1) / v.spb)) + 4000.0);
+    if (!best || t < best_t) {
+      best = &v;
+      best_t = t;
+    }
+  }
+  g.nyg = (int)((H + best->g - 1) / best->g);
+  g.nmb = (int)((cells + 16 * best->mt * best->wm - 1) / (16 * best->mt * best->wm));
+  const int64_t grid = (int64_t)((g.nyg + 7) / 8) * 8 * g.nmb;
+  if (grid > 0x7fffffff) return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL(best->fn, dim3((unsigned)grid), dim3(64 * best->wm * best->wk), best->lds, st, in, g,
+                     (const uintx4*)Bt, out, src, dst, flag, gen);
+  return hipGetLastError();
+}
+
+}  // namespace mlf

@@ -1,19 +1,20 @@
 // MEX operator without device allocation: mlf_lfm_convolution_vec_noalloc.
 //
-// mlf_lfm_convolution_vec_device keeps the MFMA form's GEMM operand (Kq,
-// mex_kq_floats(kw) floats, 59 MB at the production kernel width 241) in a
-// buffer the library allocates on first use.  Callers that cannot allocate
+// mlf_lfm_convolution_vec_device keeps the MFMA forms' kernel operand
+// (mex_scratch_floats(kw) floats, 100 MB at the production kernel width 241) in
+// a buffer the library allocates on first use.  Callers that cannot allocate
 // device memory (code under graph capture, tight serving loops) use this
-// variant instead: Kq lives in `scratch`, a file-scope device array of
-// kNoAllocFloats floats (64 MiB, odd kw <= 257) that every GPU the library
+// variant instead: the operand lives in `scratch`, a file-scope device array of
+// kNoAllocFloats floats (116 MiB, odd kw <= 257) that every GPU the library
 // runs on holds until the process ends.
 //
 // On the host the name `scratch` is a stand-in, not a device address: its
 // address on a device is resolved once per device by hipGetSymbolAddress at
 // context creation (mlf_context_create, with that device current) and only
 // that address is passed to kernels.  Every call on one GPU shares its
-// array, which keeps the last call's contents: the Kq build writes every
-// element a launch reads, so nothing needs clearing.  Calls on one context
+// array, which keeps the last call's contents: the operand build writes every
+// element a launch reads, and the flag words at its start (zero at load) hold
+// numbers of past calls, which no later call has; so nothing needs clearing.  Calls on one context
 // are ordered by its stream; calls that overlap on one GPU from different
 // contexts race on the array.
 #include <mutex>
@@ -24,8 +25,8 @@
 namespace mlf {
 
 namespace {
-constexpr size_t kNoAllocFloats = (size_t)16 << 20;  // 64 MiB
-constexpr int kNoAllocMaxKw = 257;                   // largest odd kw whose Kq fits
+constexpr size_t kNoAllocFloats = (size_t)29 << 20;  // 116 MiB
+constexpr int kNoAllocMaxKw = 257;                   // largest odd kw whose operand fits
 constexpr int kMaxDevices = 64;
 
 static __device__ __align__(256) float scratch[kNoAllocFloats];
@@ -82,9 +83,11 @@ extern "C" mlf_status mlf_lfm_convolution_vec_noalloc(mlf_context ctx, const flo
       kq = ctx->device >= 0 && ctx->device < kMaxDevices ? g_scratch_ptr[ctx->device] : nullptr;
     }
     if (!kq) return set_error(MLF_ERR_INTERNAL, "scratch of device %d not resolved", ctx->device);
-    if (mex_kq_floats((int)kw) > kNoAllocFloats)
+    if (mex_scratch_floats((int)kw) > kNoAllocFloats)
       return set_error(MLF_ERR_INTERNAL, "scratch too small for kw %lld", (long long)kw);
-    MLF_LAUNCH(launch_mex_mfma(d_bitmap, width, height, n, d_kernels, (int)kw, kq, d_out, ctx->stream));
+    MexCall c = mex_begin(width, height, n, (int)kw, d_bitmap, kq);
+    MLF_LAUNCH(launch_mex_mfma(c, d_bitmap, width, height, n, d_kernels, true, nullptr, nullptr, d_out,
+                               ctx->stream));
     return MLF_OK;
   }
   // even kw: the scalar kernel, which uses no scratch

@@ -1830,6 +1830,16 @@ mlf_status mlf_recon_phase_space(const float* lfimg, int64_t I1, int64_t I2, con
   return MLF_OK;
 }
 
+// Operand scratch of the context for kernels kw wide (called with ctx->mu held).
+static mlf_status ctx_mex_scratch(mlf_context ctx, int kw) {
+  const size_t need = mex_scratch_floats(kw);
+  if (ctx->mex_kq.count >= need) return MLF_OK;
+  MLF_HIP(hipStreamSynchronize(ctx->stream));  // earlier calls may still read it
+  MLF_CHECK(ctx->mex_kq.alloc(need));
+  MLF_LAUNCH(launch_fill(ctx->mex_kq.ptr, kMexFlagFloats, 0.f, ctx->stream));
+  return MLF_OK;
+}
+
 mlf_status mlf_lfm_convolution_vec_device(mlf_context ctx, const float* d_bitmap, int64_t width,
                                           int64_t height, int64_t n, const float* d_kernels,
                                           int64_t kw, int64_t nphase, float* d_out) {
@@ -1847,13 +1857,10 @@ mlf_status mlf_lfm_convolution_vec_device(mlf_context ctx, const float* d_bitmap
   if (kw % 2 == 1 && kw <= kMexMfmaMaxKw) {
     // odd kernels: the MFMA form; its operand scratch lives in the context
     std::lock_guard<std::mutex> lk(ctx->mu);
-    const size_t need = mex_kq_floats((int)kw);
-    if (ctx->mex_kq.count < need) {
-      MLF_HIP(hipStreamSynchronize(ctx->stream));  // earlier calls may still read it
-      MLF_CHECK(ctx->mex_kq.alloc(need));
-    }
-    MLF_LAUNCH(launch_mex_mfma(d_bitmap, width, height, n, d_kernels, (int)kw, ctx->mex_kq.ptr,
-                               d_out, ctx->stream));
+    MLF_CHECK(ctx_mex_scratch(ctx, (int)kw));
+    MexCall c = mex_begin(width, height, n, (int)kw, d_bitmap, ctx->mex_kq.ptr);
+    MLF_LAUNCH(launch_mex_mfma(c, d_bitmap, width, height, n, d_kernels, true, nullptr, nullptr, d_out,
+                               ctx->stream));
     return MLF_OK;
   }
   MLF_LAUNCH(launch_mex_conv(d_bitmap, width, height, n, d_kernels, (int)kw, d_out, ctx->stream));
@@ -2322,17 +2329,13 @@ static mlf_status segments_device(mlf_context ctx, const float* d_in, int64_t W,
     MLF_CHECK(upload_vec(d_dst, dst));
     MLF_LAUNCH(launch_fill(d_out, img * nseg, 0.f, st));
     std::lock_guard<std::mutex> lk(ctx->mu);
-    const size_t need = mex_kq_floats(kw);
-    if (ctx->mex_kq.count < need) {
-      MLF_HIP(hipStreamSynchronize(st));  // earlier calls may still read it
-      MLF_CHECK(ctx->mex_kq.alloc(need));
-    }
+    MLF_CHECK(ctx_mex_scratch(ctx, kw));
+    MexCall c = mex_begin(W, H, nslices, kw, d_in, ctx->mex_kq.ptr);
     int64_t zprev = -1;
     for (const Launch& l : launches) {
-      if (l.z != zprev) MLF_LAUNCH(launch_mex_kq(d_K + (size_t)l.z * kplane, kw, ctx->mex_kq.ptr, st));
+      MLF_LAUNCH(launch_mex_mfma(c, d_in, W, H, l.n, d_K + (size_t)l.z * kplane, l.z != zprev,
+                                 d_src.ptr + l.off, d_dst.ptr + l.off, d_out, st));
       zprev = l.z;
-      MLF_LAUNCH(launch_mex_mfma_list(d_in, W, H, l.n, ctx->mex_kq.ptr, kw, d_src.ptr + l.off,
-                                      d_dst.ptr + l.off, d_out, st));
     }
     // the index lists are freed on return: wait for the launches that read them
     MLF_HIP(hipStreamSynchronize(st));
