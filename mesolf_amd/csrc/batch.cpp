@@ -144,7 +144,7 @@ mlf_status enqueue_views(mlf_batch_s* b, hipStream_t st, int nviews = 0) {
   for (int k = 0; k < nv; ++k) {
     const FwdGeo g{b->d_slots.ptr, ps->d_rf.ptr, pk.d_woff.ptr, pk.d_nchunk.ptr, b->d_fsched.ptr,
                    b->d_counts.ptr + 0,
-                   pk.d_finv.ptr ? pk.d_finv.ptr + (size_t)k * ps->Z : nullptr};
+                   pk.d_finv.ptr ? pk.d_finv.ptr + (size_t)k * ps->Z : nullptr, pk.d_tap_inf.ptr};
     const int u = ps->uv[2 * k], v = ps->uv[2 * k + 1];
     const void* Wk = pk.fwd.ptr + (size_t)k * pk.pvf * eb;
     if (b->tpz) {

@@ -99,6 +99,7 @@ struct FwdGeo {
   const int32_t* sched;   // [entries][4] = (slot, z, b1, b2)
   const int32_t* count;   // number of entries
   const float* finv;      // FP16: [Z] inverse PSF scale of the view (null otherwise)
+  const int32_t* tap_inf; // FP32 Toeplitz: not 0 if a tap of the PSF is infinite
 };
 
 struct RatioGeo {
@@ -177,8 +178,11 @@ hipError_t launch_block_scale(const float* src, const int64_t* off, const int32_
 // (non-finite -> 0) into each slot's R; y_out (single-slot launches) gets y.
 hipError_t launch_ratio_gather_tpz(FwdGeo g, RatioGeo rg, int grid, int Z, int cw, int u, int v,
                                    int use_lf, float* y_out, hipStream_t st);
-hipError_t launch_pack_fwd_tpz(Precision p, const float* src, void* dst, PackGeo pg, int Z, int V,
+// tap_inf (FP32): a zeroed word that becomes 1 if a tap is infinite.
+hipError_t launch_pack_fwd_tpz(Precision p, const float* src, void* dst, PackGeo pg, int Z, int V, int* tap_inf,
                                hipStream_t st);
+// elements (of elem_bytes) of one plane's packed Toeplitz taps
+int64_t fwd_tpz_elems(Precision p, int r);
 size_t bwd_smem_bytes(Precision p, int rmax, int epad_max, int nt, int occ);
 
 hipError_t launch_fwd_mfma(Precision p, const void* W, FwdGeo g, int grid, size_t smem, int nbuf,

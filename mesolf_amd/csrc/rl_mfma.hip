@@ -358,17 +358,10 @@ void k_fwd_mfma(const T* __restrict__ W, FwdGeo g) {
 // the final P tile is scattered, once per entry, by in-register diagonal sums
 // and plain LDS stores.
 constexpr int kTpzNT = 3;      // N-tiles (taps along axis 1): K <= 48, i.e. r <= 23
-// Zero source for injection-ring rows outside the grid (read by the DMA, never
-// written), so the shift needs no per-element select.
-__device__ __align__(16) float g_zero_row[256] = {};  // >= one ring row (FP32: 225 floats)
-
-// W/ring buffers: the DMA runs NB-1 steps ahead.  Two buffers keep the BF16
-// kernel at 75 KB of LDS (two workgroups per CU, which measured 1.9x faster
-// than three buffers at one workgroup per CU); FP32 W buffers are 45 KB each.
-template <typename T>
-struct TpzBufs {
-  static constexpr int value = 2;
-};
+// W/ring buffers: the DMA runs one step ahead (two buffers keep the kernel at
+// 75 KB of LDS, two workgroups per CU, which measured 1.9x faster than three
+// buffers at one workgroup per CU).
+constexpr int kTpzBufs = 2;
 constexpr int kRingRow = 256;  // elements per lenslet row of the injection ring (phases >= 225 stay 0)
 
 template <typename T, int MT>
@@ -381,11 +374,11 @@ void k_fwd_tpz(const T* __restrict__ W, FwdGeo g) {
   constexpr int VEC = 16 / sizeof(T);
   constexpr int RV = PHI / VEC;
   constexpr bool SWZ = (RV == 32);
-  constexpr int NB = TpzBufs<T>::value;                        // buffers; DMA runs NB-1 steps ahead
+  constexpr int NB = kTpzBufs;
   constexpr int WSLOT = ((16 * kTpzNT * RV + 255) / 256) * 256;  // 16-byte slots per W buffer
   extern __shared__ __align__(16) char smem[];
   T* Wb = reinterpret_cast<T*>(smem);                                        // [NB][WSLOT*VEC]
-  // injection ring: FP32 volume rows (FP32) or BF16 shadow rows (BF16), kRingRow elements each
+  // injection ring: shadow rows, kRingRow elements each
   T* ring = reinterpret_cast<T*>(smem + (size_t)NB * WSLOT * 16);            // [NB][CW][kRingRow]
   float* ywin = reinterpret_cast<float*>(ring + NB * CW * kRingRow);         // [4 waves][16][MT + 2r]
 
@@ -393,7 +386,6 @@ void k_fwd_tpz(const T* __restrict__ W, FwdGeo g) {
   for (int ent = blockIdx.x; ent < nent; ent += gridDim.x) {
     const int* s = g.sched + 4 * ent;
     const SlotDesc sd = load_slot(g.slots, uni(cload(s)));
-    const float* __restrict__ X = sd.X;
     const T* __restrict__ Xb = reinterpret_cast<const T*>(sd.Xb);
     const int n1 = sd.n1, n2 = sd.n2;
     const int z = uni(cload(s + 1)), b1 = uni(cload(s + 2)), b2 = uni(cload(s + 3));
@@ -411,11 +403,10 @@ void k_fwd_tpz(const T* __restrict__ W, FwdGeo g) {
         sd.partial + uni64(cload(sd.poff + z)) + (size_t)(b2 * ceil_div(n1, 16) + b1) * 16 * (CW + 2 * r);
     float unscale = 1.f;
     if constexpr (is_f16<T>()) unscale = cload(g.finv + z) * sd.xs_inv;
-    const float* Xz = X + (size_t)z * n2 * n1 * kXRow;
-    const T* Xbz = KPL > 1 ? Xb + (size_t)z * n2 * n1 * kShadowRow : nullptr;  // BF16 / FP16 shadow plane
+    const T* Xbz = Xb + (size_t)z * n2 * n1 * kShadowRow;  // shadow plane
     // the shadow plane as a buffer (a plane is below 2^31 bytes, checked at patch creation)
     const __amdgpu_buffer_rsrc_t shr = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<T*>(Xbz), 0, KPL > 1 ? (int)((size_t)n2 * n1 * kShadowRow * sizeof(T)) : 0, kBufferDword3);
+        const_cast<T*>(Xbz), 0, (int)((size_t)n2 * n1 * kShadowRow * sizeof(T)), kBufferDword3);
     float* yw = ywin + w * 16 * WW;  // every cell is written by the flush
     for (int o = tid; o < NB * CW * kRingRow; o += 256) ring[o] = (T)0.f;  // pads stay zero
 
@@ -429,26 +420,18 @@ void k_fwd_tpz(const T* __restrict__ W, FwdGeo g) {
       const size_t lens = ((size_t)z * n2 + (ok ? c2 : 0)) * n1 + (ok ? i1 : 0);
   #pragma unroll
       for (int ks = 0; ks < NKS; ++ks) {
-        if constexpr (KPL == 1) {
-          const int ph = ks * KSTEP + lg;
-          const float v = gload(X + lens * kXRow + (ph < kP ? ph : kP - 1));
-          a[mt][ks] = (ok && ph < kP) ? v : 0.f;
-        } else {
-          // BF16 shadow rows are 256 phases (zero beyond 225), 16-byte aligned
-          const typename M::frag v =
-              gload(reinterpret_cast<const typename M::frag*>(Xb + lens * kShadowRow + ks * KSTEP + lg * KPL));
-          a[mt][ks] = ok ? v : typename M::frag{};
-        }
+        // shadow rows are 256 phases (zero beyond 225), 16-byte aligned
+        const typename M::frag v =
+            gload(reinterpret_cast<const typename M::frag*>(Xb + lens * kShadowRow + ks * KSTEP + lg * KPL));
+        a[mt][ks] = ok ? v : typename M::frag{};
       }
     }
     __syncthreads();  // ring zeroed before any DMA lands
 
     const T* Wz = W + uni64(cload(g.woff + z));  // [K][nrow][PHI]
-    // Every wave issues the same number of DMA instructions per step (W: the
-    // entry's nw_inst; ring: CW*RPASS passes / 4 waves), so a step can wait
-    // for an earlier batch with a fixed vmcnt.  Only the K tap rows e2 < K
-    // are copied: rows K..16*NT-1 of the buffer feed accumulator columns that
-    // the flush drops, so whatever they hold does not matter.
+    // Only the K tap rows e2 < K are copied: rows K..16*NT-1 of the buffer feed
+    // accumulator columns that the flush drops, so whatever they hold does not
+    // matter.
     const int nslot = K * RV;
     const int nw_inst = (nslot + 255) / 256;
     // Copy addresses: a wave-uniform (scalar) base plus the lane's 32-bit byte
@@ -474,66 +457,26 @@ void k_fwd_tpz(const T* __restrict__ W, FwdGeo g) {
                                          16, 0, 0);
       }
     };
-    // injection row needed when entering step t (t >= 1): i1 = 16*b1 + r - t
-    // (rows outside the grid are loaded clamped and zeroed at the shift)
-    // FP32: 225 floats per lenslet in 4 passes of 64 dwords; BF16: the 512-byte
-    // shadow row in 2 passes of 64 dwords.
-    constexpr int RPASS = (KPL == 1) ? 4 : 2;
-    auto issue_inj = [&](int t, int slot_buf) {
-      const int i1r = 16 * b1 + r - t;
-      const bool rowok = i1r >= 0 && i1r < n1;
-      const int i1 = min(max(i1r, 0), n1 - 1);
-      char* dst = reinterpret_cast<char*>(ring + slot_buf * CW * kRingRow);
-      for (int q = w; q < CW * RPASS; q += 4) {
-        const int c = q / RPASS, part = q - c * RPASS;
-        const bool ok = rowok && c2_0 + c < n2;
-        const int c2 = min(c2_0 + c, n2 - 1);
-        const size_t lens = (size_t)c2 * n1 + i1;  // within the plane
-        const int d = part * 64 + lane;          // dword within the row
-        if constexpr (KPL == 1) {
-          if (d >= kP) continue;
-        }
-        const char* row = ok ? (KPL == 1 ? reinterpret_cast<const char*>(Xz + lens * kXRow)
-                                         : reinterpret_cast<const char*>(Xbz + lens * kShadowRow))
-                             : reinterpret_cast<const char*>(g_zero_row);
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(row + 4 * d),
-                                         (__attribute__((address_space(3))) void*)(dst + (c * kRingRow) * (int)sizeof(T) + 4 * part * 64),
-                                         4, 0, 0);
-      }
-    };
-    // DMA instructions per wave of a batch t >= 1 (16-bit: every W slot copy is issued)
-    const int n_batch = (KPL == 1 ? nw_inst : kWInst) + CW * RPASS / 4;
-
+    constexpr int RPASS = 2;  // passes of 64 dwords per 512-byte shadow row
     floatx4 acc[MT][kTpzNT];
   #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
   #pragma unroll
       for (int nt = 0; nt < kTpzNT; ++nt) acc[mt][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    // batch t = W column t (+ injection row t for t >= 1); batches with index
-    // >= 1 are n_batch instructions per wave
+    // batch t = W column t and, for t >= 1, injection row t (i1 = 16 b1 + r - t)
     issue_w(0, 0);
-    for (int t = 1; t < NB - 1 && t < K; ++t) {
-      issue_w(t, t % NB);
-      issue_inj(t, t % NB);
-    }
-    wait_vm_le(max(0, min(K, NB - 1) - 1) * n_batch);  // batch 0 landed
+    wait_vm<0>();  // batch 0 landed
     __syncthreads();
-    // 16-bit: the copies of batch t + NB - 1 are spread over tile 0's K-steps
+    // The copies of batch t + 1 are spread over tile 0's K-steps
     // (one injection copy and at most one W copy per K-step, no branches), so
     // the eight waves of a CU do not queue their copies at the address unit
     // all at once.  The last step re-copies the last column and a row past the
     // grid (zeros) into the free buffer, which nothing reads.
     constexpr int kInj = CW * RPASS / 4;  // injection copies per wave and step
-    static_assert(KPL == 1 || (kInj <= NKS && kWInst <= NKS), "one copy of each kind per K-step");
+    static_assert(kInj <= NKS && kWInst <= NKS, "one copy of each kind per K-step");
     for (int t = 0; t < K; ++t) {
       const int tn = min(t + NB - 1, K - 1), bn = (t + NB - 1) % NB;
-      if constexpr (KPL == 1) {
-        if (t + NB - 1 < K) {
-          issue_w(tn, bn);
-          issue_inj(tn, bn);
-        }
-      }
       const char* w_src = reinterpret_cast<const char*>(Wz + (size_t)tn * nrow * PHI);
       char* w_dst = reinterpret_cast<char*>(Wb) + (size_t)bn * WSLOT * 16;
       const int i1r_n = 16 * b1 + r - tn;
@@ -541,23 +484,21 @@ void k_fwd_tpz(const T* __restrict__ W, FwdGeo g) {
       const int i1_n = min(max(i1r_n, 0), n1 - 1);
       char* inj_dst = reinterpret_cast<char*>(ring + bn * CW * kRingRow);
       auto issue_piece = [&](int k) __attribute__((always_inline)) {
-        if constexpr (KPL > 1) {
-          if (k < kWInst)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(w_src + woff[k]),
-                                             (__attribute__((address_space(3))) void*)(w_dst + (256 * k + 64 * w) * 16),
-                                             16, 0, 0);
-          if (k < kInj) {
-            // rows outside the grid: an offset past the plane, which the
-            // buffer load returns as zeros (no branch, no zero-row pointer)
-            const int q = w + 4 * k, c = q / RPASS, part = q - c * RPASS;
-            const bool ok = rowok_n && c2_0 + c < n2;
-            const int c2 = min(c2_0 + c, n2 - 1);
-            const unsigned voff = ok ? (unsigned)(((c2 * n1 + i1_n) * kShadowRow + part * 128) * 2) + 4u * lane
-                                     : 0x80000000u;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                shr, (__attribute__((address_space(3))) void*)(inj_dst + (c * kRingRow) * (int)sizeof(T) + 4 * part * 64),
-                4, voff, 0, 0, 0);
-          }
+        if (k < kWInst)
+          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(w_src + woff[k]),
+                                           (__attribute__((address_space(3))) void*)(w_dst + (256 * k + 64 * w) * 16),
+                                           16, 0, 0);
+        if (k < kInj) {
+          // rows outside the grid: an offset past the plane, which the
+          // buffer load returns as zeros (no branch, no zero-row pointer)
+          const int q = w + 4 * k, c = q / RPASS, part = q - c * RPASS;
+          const bool ok = rowok_n && c2_0 + c < n2;
+          const int c2 = min(c2_0 + c, n2 - 1);
+          const unsigned voff = ok ? (unsigned)(((c2 * n1 + i1_n) * kShadowRow + part * 128) * 2) + 4u * lane
+                                   : 0x80000000u;
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(
+              shr, (__attribute__((address_space(3))) void*)(inj_dst + (c * kRingRow) * (int)sizeof(T) + 4 * part * 64),
+              4, voff, 0, 0, 0);
         }
       };
       const T* Wc = Wb + (size_t)(t % NB) * WSLOT * VEC;
@@ -598,12 +539,9 @@ void k_fwd_tpz(const T* __restrict__ W, FwdGeo g) {
       tile(std::integral_constant<int, 0>{});
       if (NT > 1) tile(std::integral_constant<int, 1>{});
       if (NT > 2) tile(std::integral_constant<int, 2>{});
-      // batch t+1 landed; later batches may still be in flight
-      wait_vm_le(max(0, min(K, t + NB) - t - 2) * n_batch);
+      wait_vm<0>();  // batch t + 1 landed
       __syncthreads();
       if (t + 1 < K) {
-        const int i1n = 16 * b1 + r - (t + 1);
-        (void)i1n;
         const T* rg = ring + ((t + 1) % NB) * CW * kRingRow;
   #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
@@ -614,24 +552,16 @@ void k_fwd_tpz(const T* __restrict__ W, FwdGeo g) {
           // arrived as zeros
   #pragma unroll
           for (int ks = 0; ks < NKS; ++ks) {
-            if constexpr (KPL == 1) {
-              a[mt][ks] = __builtin_bit_cast(
-                  float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, a[mt][ks]), 0x111, 0xF, 0xF, true));
-            } else {
-              typedef int intx4 __attribute__((ext_vector_type(4)));
-              intx4 cv = __builtin_bit_cast(intx4, a[mt][ks]);
+            typedef int intx4 __attribute__((ext_vector_type(4)));
+            intx4 cv = __builtin_bit_cast(intx4, a[mt][ks]);
   #pragma unroll
-              for (int q = 0; q < 4; ++q) cv[q] = __builtin_amdgcn_mov_dpp(cv[q], 0x111, 0xF, 0xF, true);
-              a[mt][ks] = __builtin_bit_cast(typename M::frag, cv);
-            }
+            for (int q = 0; q < 4; ++q) cv[q] = __builtin_amdgcn_mov_dpp(cv[q], 0x111, 0xF, 0xF, true);
+            a[mt][ks] = __builtin_bit_cast(typename M::frag, cv);
           }
           if (lr == 0) {
             const T* rp = rg + c * kRingRow + lg * KPL;
   #pragma unroll
-            for (int ks = 0; ks < NKS; ++ks) {
-              if constexpr (KPL == 1) a[mt][ks] = rp[ks * KSTEP];
-              else a[mt][ks] = *reinterpret_cast<const typename M::frag*>(rp + ks * KSTEP);
-            }
+            for (int ks = 0; ks < NKS; ++ks) a[mt][ks] = *reinterpret_cast<const typename M::frag*>(rp + ks * KSTEP);
           }
         }
       }
@@ -687,6 +617,328 @@ void k_fwd_tpz(const T* __restrict__ W, FwdGeo g) {
       gstore(out + o, sum);
     }
     __syncthreads();  // LDS is reused by the next entry
+  }
+}
+
+// ------------------------------------------- forward (Toeplitz, split FP32)
+// The FP32 forward on the BF16 matrix pipe.  Same GEMM, register window over
+// i1 and partial windows as k_fwd_tpz; every operand is split exactly into
+// three BF16 parts (x = x0 + x1 + x2, each rounded to nearest) and a product
+// takes the six MFMAs of the parts whose orders add up to at most two (left
+// out: below 2^-24 of the product).  Six 16x16x32 BF16 MFMAs take 96 cycles
+// where the FP32 pipe takes 256.  The matrix pipe cuts low bits of what it
+// adds to a large accumulator, so a step's 24 MFMAs per tile start from zero
+// and their sum is added to the accumulator by the vector unit: with one chain
+// over all steps the sums came out 1.2e-6 low, with one per step the error
+// against FP64 is 5.9e-8 (FP32 pipe 8.7e-8; 81 x 81 x 51).
+// Bound by the matrix pipe: 81 x 81 x 51, 177 views 127.6 ms (FP32 pipe 302), 0.72 ms
+// per view, 1.2e15 flop/s issued.
+// The A parts of 16 lenslets x 256 phases would fill 192 registers per wave
+// for two columns, so the phases go in two halves of 128 (96 registers, two
+// workgroups per CU), each half a whole walk over e1, summed in the same
+// accumulators.  The taps are stored as ready B fragments, [half][e1][N-tile]
+// [K-step][part][lane][8], so that a step's copy is contiguous and its LDS
+// reads are free of conflicts.
+// Infinities of the volume or the taps would turn into NaN between the parts:
+// an entry that meets one is summed again directly in FP32.
+constexpr int kSplitKS = 4;       // K-steps (32 phases) per half
+constexpr int kSplitFrag = 1024;  // bytes of one fragment of a wave
+
+__device__ __forceinline__ unsigned pack_bf16(float lo, float hi) {
+  return (unsigned)__builtin_bit_cast(unsigned short, (__bf16)lo) |
+         ((unsigned)__builtin_bit_cast(unsigned short, (__bf16)hi) << 16);
+}
+// x, y -> their three BF16 parts, packed in pairs.  A finite value that BF16
+// would round to infinity takes the largest BF16 as its first part.
+__device__ __forceinline__ void split_bf16(float x, float y, unsigned* w) {
+  constexpr float kMax = 3.3895314e38f;
+  w[0] = pack_bf16(fmaxf(fminf(x, kMax), -kMax), fmaxf(fminf(y, kMax), -kMax));
+#pragma unroll
+  for (int k = 1; k < 3; ++k) {
+    x -= __builtin_bit_cast(float, w[k - 1] << 16);
+    y -= __builtin_bit_cast(float, w[k - 1] & 0xFFFF0000u);
+    w[k] = pack_bf16(x, y);
+  }
+}
+__device__ __forceinline__ bool is_inf(float x) { return __builtin_amdgcn_classf(x, 0x204); }
+
+template <int MT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+void k_fwd_tps(const char* __restrict__ W, FwdGeo g) {
+  typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+  typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
+  constexpr int CW = 4 * MT;  // input columns c2 per workgroup
+  constexpr int WBUF = kTpzNT * kSplitKS * 3 * kSplitFrag;
+  extern __shared__ __align__(16) char smem[];
+  // [2][WBUF] tap fragments; then per wave the entering lenslets
+  // [MT][part][128 phases].  The flush's windows reuse the tap buffers.
+  const int nent = uni(cload(g.count));
+  for (int ent = blockIdx.x; ent < nent; ent += gridDim.x) {
+    const int* s = g.sched + 4 * ent;
+    const SlotDesc sd = load_slot(g.slots, uni(cload(s)));
+    const int n1 = sd.n1, n2 = sd.n2;
+    const int z = uni(cload(s + 1)), b1 = uni(cload(s + 2)), b2 = uni(cload(s + 3));
+    const int r = uni(cload(g.r + z));
+    const int K = 2 * r + 1;
+    const int NT = (K + 15) / 16;
+    const int WW = MT + 2 * r;
+    const int tid = threadIdx.x, lane = tid & 63, w = uni(tid >> 6), lr = lane & 15, lg = lane >> 4;
+    const int c2_0 = CW * b2;
+    float* const out =
+        sd.partial + uni64(cload(sd.poff + z)) + (size_t)(b2 * ceil_div(n1, 16) + b1) * 16 * (CW + 2 * r);
+    // one plane of the volume and one plane's taps as buffers: reads past the
+    // end (lenslets outside the grid, padded tap rows) return zeros
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+        sd.X + (size_t)z * n2 * n1 * kXRow, 0, (int)((size_t)n2 * n1 * kXRow * 4), kBufferDword3);
+    const int step_bytes = NT * kSplitKS * 3 * kSplitFrag;
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char*>(W) + 4 * uni64(cload(g.woff + z)), 0, 2 * K * step_bytes, kBufferDword3);
+    char* const ring = smem + 2 * WBUF + w * MT * 768;
+    bool inf = cload(g.tap_inf) != 0;
+
+    bf16x8 a[MT][kSplitKS][3];
+    auto load_a = [&](int h) {
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        const int c2 = c2_0 + MT * w + mt, i1 = 16 * b1 + lr + r;
+        const unsigned o = c2 < n2 && i1 < n1 ? (unsigned)(4 * ((c2 * n1 + i1) * kXRow + 128 * h + 8 * lg))
+                                              : 0x80000000u;
+#pragma unroll
+        for (int ks = 0; ks < kSplitKS; ++ks) {
+          const floatx4 v0 = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(xr, o, 128 * ks, 0));
+          const floatx4 v1 = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(xr, o, 128 * ks + 16, 0));
+          unsigned p[4][3];
+          split_bf16(v0[0], v0[1], p[0]);
+          split_bf16(v0[2], v0[3], p[1]);
+          split_bf16(v1[0], v1[1], p[2]);
+          split_bf16(v1[2], v1[3], p[3]);
+#pragma unroll
+          for (int q = 0; q < 3; ++q)
+            a[mt][ks][q] = __builtin_bit_cast(bf16x8, uintx4{p[0][q], p[1][q], p[2][q], p[3][q]});
+#pragma unroll
+          for (int j = 0; j < 4; ++j) inf = inf || is_inf(v0[j]) || is_inf(v1[j]);
+        }
+      }
+    };
+    // piece q of step st's taps: this wave's share of N-tile q / 3
+    const unsigned tap_lane = 16 * lane;
+    auto issue_w = [&](int st, int q) __attribute__((always_inline)) {
+      const unsigned vo = 16 * (q / 3) + lr < K ? tap_lane : 0x80000000u;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          wr, (__attribute__((address_space(3))) void*)(smem + (st & 1) * WBUF + (4 * q + w) * kSplitFrag), 16, vo,
+          st * step_bytes + (4 * q + w) * kSplitFrag, 0, 0);
+    };
+    for (int q = 0; q < 3 * NT; ++q) issue_w(0, q);
+    load_a(0);
+
+    floatx4 acc[MT][kTpzNT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < kTpzNT; ++nt) acc[mt][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    wait_vm<0>();
+    lds_barrier();
+
+    // the lenslet that enters column `inj_mt` of this wave: 4 of its phases per lane
+    const int inj_mt = MT == 2 ? lane >> 5 : 0, inj_ph = 4 * (lane & 31), inj_c2 = c2_0 + MT * w + inj_mt;
+    const bool inj_on = MT == 2 || lane < 32;
+    const int nst = 2 * K;
+    int t = 0, h = 0;  // step st = h K + t
+    for (int st = 0; st < nst; ++st) {
+      const bool last_t = t + 1 == K;
+      floatx4 inj = {0.f, 0.f, 0.f, 0.f};
+      if (!last_t) {
+        const int i1 = 16 * b1 + r - (t + 1);
+        const unsigned o = i1 >= 0 && i1 < n1 && inj_c2 < n2 && inj_on
+                               ? (unsigned)(4 * ((inj_c2 * n1 + i1) * kXRow + 128 * h + inj_ph))
+                               : 0x80000000u;
+        inj = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(xr, o, 0, 0));
+      }
+      const char* Wc = smem + (st & 1) * WBUF + 16 * lane;
+      const bool more = st + 1 < nst;
+      bf16x8 bn[3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) bn[p] = *reinterpret_cast<const bf16x8*>(Wc + p * kSplitFrag);
+      auto tile = [&](auto ntc) __attribute__((always_inline)) {
+        constexpr int nt = decltype(ntc)::value;
+        floatx4 c[MT];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) c[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < kSplitKS; ++ks) {
+          constexpr int kLastQ = kTpzNT * kSplitKS - 1;
+          const int q = nt * kSplitKS + ks, qn = q < kLastQ ? q + 1 : kLastQ;
+          bf16x8 b[3];
+#pragma unroll
+          for (int p = 0; p < 3; ++p) b[p] = bn[p];
+          // the next K-step's fragments (past the plane's tiles: unused)
+#pragma unroll
+          for (int p = 0; p < 3; ++p) bn[p] = *reinterpret_cast<const bf16x8*>(Wc + (3 * qn + p) * kSplitFrag);
+          if (more && q < 3 * NT) issue_w(st + 1, q);
+          // smallest products first
+          constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+          for (int i = 0; i < 6; ++i)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+              c[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt][ks][pa[i]], b[pb[i]], c[mt], 0, 0, 0);
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[mt][nt] += c[mt];
+      };
+      static_assert(kTpzNT == 3, "three N-tiles");
+      tile(std::integral_constant<int, 0>{});
+      if (NT > 1) tile(std::integral_constant<int, 1>{});
+      if (NT > 2) tile(std::integral_constant<int, 2>{});
+      if (!last_t && inj_on) {
+        unsigned p0[3], p1[3];
+        split_bf16(inj[0], inj[1], p0);
+        split_bf16(inj[2], inj[3], p1);
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+          *reinterpret_cast<uintx2*>(ring + inj_mt * 768 + q * 256 + 2 * inj_ph) = uintx2{p0[q], p1[q]};
+        inf = inf || is_inf(inj[0]) || is_inf(inj[1]) || is_inf(inj[2]) || is_inf(inj[3]);
+      }
+      wait_vm<0>();   // the next step's taps
+      lds_barrier();  // ... of every wave, and every wave is done with this step's
+      if (last_t) {
+        t = 0;
+        ++h;
+        if (h < 2) load_a(h);
+        continue;
+      }
+      ++t;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+        for (int ks = 0; ks < kSplitKS; ++ks)
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            uintx4 c = __builtin_bit_cast(uintx4, a[mt][ks][q]);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) c[j] = __builtin_amdgcn_mov_dpp(c[j], 0x111, 0xF, 0xF, true);
+            a[mt][ks][q] = __builtin_bit_cast(bf16x8, c);
+          }
+        if (lr == 0) {
+#pragma unroll
+          for (int ks = 0; ks < kSplitKS; ++ks)
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+              a[mt][ks][q] = *reinterpret_cast<const bf16x8*>(ring + mt * 768 + q * 256 + 64 * ks + 16 * lg);
+        }
+      }
+    }
+
+    // flush as in k_fwd_tpz (the last barrier has freed the tap buffers)
+    float* const ywin = reinterpret_cast<float*>(smem);
+    float* const yw = ywin + w * 16 * WW;
+    floatx4 carry = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int nt = 0; nt <= kTpzNT; ++nt) {
+      if (nt > NT) continue;
+      floatx4 col = carry;
+      carry = floatx4{0.f, 0.f, 0.f, 0.f};
+      if (nt < kTpzNT && nt < NT) {
+        const bool ev = nt * 16 + lr < K;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float x = row_ror(ev ? acc[mt][nt < kTpzNT ? nt : 0][j] : 0.f, mt);
+            col[j] += lr >= mt ? x : 0.f;
+            carry[j] += lr >= mt ? 0.f : x;
+          }
+      }
+      const int c = nt * 16 + lr;
+      if (c < WW) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) yw[(4 * lg + j) * WW + c] = col[j];
+      }
+    }
+    if (lane == 0) *reinterpret_cast<int*>(ring) = 0;
+    if (inf) *reinterpret_cast<int*>(ring) = 1;
+    __syncthreads();
+    int any = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) any |= *reinterpret_cast<const int*>(smem + 2 * WBUF + q * MT * 768);
+    any = uni(any);
+    const int Wc2 = CW + 2 * r;
+    for (int o = tid; o < 16 * Wc2; o += 256) {
+      const int c = o >> 4, i = o & 15;
+      float sum = 0.f;
+      if (!any) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int cc = c - MT * q;
+          if (cc >= 0 && cc < WW) sum += ywin[(q * 16 + i) * WW + cc];
+        }
+      } else {
+        // y[i][c] = sum over e1, columns and phases of X * taps, FP32
+        for (int cc = max(0, c - K + 1); cc < CW && cc <= c; ++cc)
+          for (int e1 = 0; e1 < K; ++e1) {
+            const int i1 = 16 * b1 + i - (e1 - r), c2 = c2_0 + cc, e2 = c - cc;
+            const bool in = i1 >= 0 && i1 < n1 && c2 < n2;
+            for (int ph = 0; ph < kP; ++ph) {
+              const unsigned xo = in ? (unsigned)(4 * ((c2 * n1 + i1) * kXRow + ph)) : 0x80000000u;
+              const float x = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xr, xo, 0, 0));
+              const int f = ((((ph >> 7) * K + e1) * NT + (e2 >> 4)) * kSplitKS + ((ph >> 5) & 3)) * 3;
+              const int wo = f * kSplitFrag + (((ph >> 3) & 3) * 16 + (e2 & 15)) * 16 + (ph & 7) * 2;
+              float tap = 0.f;
+#pragma unroll
+              for (int q = 0; q < 3; ++q)
+                tap += __builtin_bit_cast(
+                    float, (unsigned)(unsigned short)__builtin_amdgcn_raw_buffer_load_b16(wr, wo + q * kSplitFrag, 0, 0) << 16);
+              sum = fmaf(x, tap, sum);
+            }
+          }
+      }
+      gstore(out + o, sum);
+    }
+    __syncthreads();  // LDS is reused by the next entry
+  }
+}
+
+// ABI block [e2][e1][phase] -> the fragments of k_fwd_tps, [half][e1][N-tile]
+// [K-step][part][lane][8]: lane (lr, lg) holds tap row e2 = 16 nt + lr, phases
+// 128 half + 32 ks + 8 lg .. + 7.  *tap_inf becomes 1 if a tap is infinite
+// (its parts are then itself, 0, 0).
+__global__ void k_pack_fwd_split(const float* __restrict__ src, char* __restrict__ dst, PackGeo pg,
+                                 int* __restrict__ tap_inf) {
+  typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+  const int z = blockIdx.y, v = blockIdx.z;
+  const int K = 2 * pg.r[z] + 1, NT = (K + 15) / 16;
+  const float* s = src + (size_t)v * pg.src_view + pg.src_off[z];
+  char* d = dst + 4 * ((size_t)v * pg.dst_view + pg.dst_off[z]);
+  const size_t total = (size_t)2 * K * NT * kSplitKS * 64;
+  for (size_t o = blockIdx.x * (size_t)blockDim.x + threadIdx.x; o < total; o += (size_t)gridDim.x * blockDim.x) {
+    const int lane = (int)(o & 63), lr = lane & 15, lg = lane >> 4;
+    const size_t f = o >> 6;
+    const int ks = (int)(f % kSplitKS), nt = (int)((f / kSplitKS) % NT);
+    const int he = (int)(f / ((size_t)kSplitKS * NT)), h = he / K, e1 = he - h * K;
+    const int e2 = 16 * nt + lr, ph = 128 * h + 32 * ks + 8 * lg;
+    unsigned p[4][3];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float x[2];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int pj = ph + 2 * j + q;
+        x[q] = e2 < K && pj < kP ? s[((size_t)e2 * K + e1) * kP + pj] : 0.f;
+      }
+      split_bf16(x[0], x[1], p[j]);
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        if (is_inf(x[q])) {
+          const unsigned m = q ? 0xFFFF0000u : 0xFFFFu;
+          p[j][0] = (p[j][0] & ~m) | (pack_bf16(x[0], x[1]) & m);
+          p[j][1] &= ~m;
+          p[j][2] &= ~m;
+          *tap_inf = 1;
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      *reinterpret_cast<uintx4*>(d + (f * 3 + q) * kSplitFrag + 16 * lane) = uintx4{p[0][q], p[1][q], p[2][q], p[3][q]};
   }
 }
 
@@ -1642,12 +1894,17 @@ hipError_t launch_fwd_mfma(Precision p, const void* W, FwdGeo g, int grid, size_
 }
 
 size_t tpz_smem_bytes(Precision p, int rmax, int MT) {
-  const bool f32 = p == Precision::kF32;
-  const int RV = f32 ? Mma<float>::PHI / 4 : Mma<__bf16>::PHI / 8;
-  const int NB = f32 ? TpzBufs<float>::value : TpzBufs<__bf16>::value;
+  if (p == Precision::kF32) return (size_t)2 * kTpzNT * kSplitKS * 3 * kSplitFrag + 4 * MT * 768;
+  const int RV = Mma<__bf16>::PHI / 8;
   const size_t wslot = ((16 * kTpzNT * RV + 255) / 256) * 256;
-  return (size_t)NB * wslot * 16 + elem_bytes(p) * NB * 4 * MT * kRingRow +
+  return (size_t)kTpzBufs * wslot * 16 + elem_bytes(p) * kTpzBufs * 4 * MT * kRingRow +
          sizeof(float) * 4 * 16 * (MT + 2 * rmax);
+}
+
+int64_t fwd_tpz_elems(Precision p, int r) {
+  const int64_t K = 2 * r + 1, nt = (K + 15) / 16;
+  if (p == Precision::kF32) return 2 * K * nt * kSplitKS * 3 * (kSplitFrag / 4);
+  return K * 16 * nt * fwd_phi(p);
 }
 
 int tpz_max_radius() { return (16 * kTpzNT - 1) / 2; }
@@ -1656,9 +1913,9 @@ hipError_t launch_fwd_tpz(Precision p, int mt, const void* W, FwdGeo g, int grid
                           hipStream_t st) {
   if (p == Precision::kF32) {
     if (mt == 1)
-      hipLaunchKernelGGL((k_fwd_tpz<float, 1>), dim3(grid), dim3(256), smem, st, (const float*)W, g);
+      hipLaunchKernelGGL(k_fwd_tps<1>, dim3(grid), dim3(256), smem, st, (const char*)W, g);
     else
-      hipLaunchKernelGGL((k_fwd_tpz<float, 2>), dim3(grid), dim3(256), smem, st, (const float*)W, g);
+      hipLaunchKernelGGL(k_fwd_tps<2>, dim3(grid), dim3(256), smem, st, (const char*)W, g);
   } else if (p == Precision::kF16) {
     if (mt == 2)
       hipLaunchKernelGGL((k_fwd_tpz<_Float16, 2>), dim3(grid), dim3(256), smem, st, (const _Float16*)W, g);
@@ -1779,11 +2036,11 @@ hipError_t launch_ratio_gather_tpz(FwdGeo g, RatioGeo rg, int grid, int Z, int c
   return hipGetLastError();
 }
 
-hipError_t launch_pack_fwd_tpz(Precision p, const float* src, void* dst, PackGeo pg, int Z, int V,
+hipError_t launch_pack_fwd_tpz(Precision p, const float* src, void* dst, PackGeo pg, int Z, int V, int* tap_inf,
                                hipStream_t st) {
   dim3 grid(64, Z, V);
   if (p == Precision::kF32)
-    hipLaunchKernelGGL(k_pack_fwd_tpz<float>, grid, dim3(256), 0, st, src, (float*)dst, pg);
+    hipLaunchKernelGGL(k_pack_fwd_split, grid, dim3(256), 0, st, src, (char*)dst, pg, tap_inf);
   else if (p == Precision::kF16)
     hipLaunchKernelGGL(k_pack_fwd_tpz<_Float16>, grid, dim3(256), 0, st, src, (_Float16*)dst, pg);
   else
@@ -1882,8 +2139,8 @@ hipError_t mfma_kernel_attributes() {
       reinterpret_cast<const void*>(&k_fwd_mfma<float, kFwdMTF32, 2>),
       reinterpret_cast<const void*>(&k_fwd_mfma<__bf16, kFwdMTBF16, 1>),
       reinterpret_cast<const void*>(&k_fwd_mfma<__bf16, kFwdMTBF16, 2>),
-      reinterpret_cast<const void*>(&k_fwd_tpz<float, 1>),
-      reinterpret_cast<const void*>(&k_fwd_tpz<float, 2>),
+      reinterpret_cast<const void*>(&k_fwd_tps<1>),
+      reinterpret_cast<const void*>(&k_fwd_tps<2>),
       reinterpret_cast<const void*>(&k_fwd_tpz<__bf16, 2>),
       reinterpret_cast<const void*>(&k_fwd_tpz<__bf16, 4>),
       reinterpret_cast<const void*>(&k_bwd_mfma<float, 3, 2, false>),

@@ -307,15 +307,14 @@ static mlf_status psf_ensure_pack(mlf_psf_s* ps, Precision prec) {
     const int nt_f = (2 * ps->rf[z] + 1) * (2 * ps->rf[z] + 1);
     const int nt_b = (2 * ps->rb[z] + 1) * (2 * ps->rb[z] + 1);
     pk.nchunk[z] = (nt_f + kFwdChunk - 1) / kFwdChunk;
-    const int Kf = 2 * ps->rf[z] + 1;
-    rows_f[z] = pk.tpz ? Kf * 16 * ((Kf + 15) / 16) : pk.nchunk[z] * kFwdChunk;
+    rows_f[z] = pk.nchunk[z] * kFwdChunk;
     const int Kb = 2 * ps->rb[z] + 1;
     const int nt_b_pad = prec != Precision::kF32 ? 32 * bwd_quad_steps(Kb) : nt_b;
     const int tpad = prec != Precision::kF32 ? kBwdTapPad16 : kBwdTapPad;
     pk.epad[z] = (nt_b_pad + tpad - 1) / tpad * tpad;
     rows_b[z] = pk.epad[z];
     pk.woff[z] = of;
-    of += (int64_t)rows_f[z] * phi;
+    of += pk.tpz ? fwd_tpz_elems(prec, ps->rf[z]) : (int64_t)rows_f[z] * phi;
     pk.boff[z] = ob;
     ob += (int64_t)kPhiPadBwd * pk.epad[z];
   }
@@ -345,7 +344,8 @@ static mlf_status psf_ensure_pack(mlf_psf_s* ps, Precision prec) {
   }
   PackGeo gf{ps->d_rf.ptr, d_rows_f.ptr, ps->d_offf.ptr, pk.d_woff.ptr, ps->per_view_f, pk.pvf, 0,
              pk.d_fscale.ptr};
-  hipError_t e = pk.tpz ? launch_pack_fwd_tpz(prec, ps->fwd.ptr, pk.fwd.ptr, gf, Z, V, st)
+  MLF_CHECK(upload_vec(pk.d_tap_inf, std::vector<int32_t>{0}));
+  hipError_t e = pk.tpz ? launch_pack_fwd_tpz(prec, ps->fwd.ptr, pk.fwd.ptr, gf, Z, V, pk.d_tap_inf.ptr, st)
                         : launch_pack_fwd(prec, ps->fwd.ptr, pk.fwd.ptr, gf, Z, V, st);
   if (e != hipSuccess) return set_error(MLF_ERR_DEVICE, "pack_fwd: %s", hipGetErrorString(e));
   PackGeo gb{ps->d_rb.ptr, d_rows_b.ptr, ps->d_offb.ptr, pk.d_boff.ptr, ps->per_view_b, pk.pvb,
@@ -963,7 +963,7 @@ static FwdGeo fwd_geo(mlf_patch_s* p, int k) {
   const PrecPack& pk = ps->pack[(int)p->kp];
   return FwdGeo{p->d_slot.ptr, ps->d_rf.ptr, pk.d_woff.ptr, pk.d_nchunk.ptr, p->d_fsched.ptr,
                 p->d_counts.ptr + 0,
-                pk.d_finv.ptr ? pk.d_finv.ptr + (size_t)k * ps->Z : nullptr};
+                pk.d_finv.ptr ? pk.d_finv.ptr + (size_t)k * ps->Z : nullptr, pk.d_tap_inf.ptr};
 }
 
 static BwdGeo bwd_geo(mlf_patch_s* p, int k) {

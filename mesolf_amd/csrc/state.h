@@ -41,13 +41,15 @@ mlf_status upload_vec(DevBuf<T>& d, const std::vector<T>& h) {
 // PSF tables re-laid out for the MFMA kernels of one precision.
 struct PrecPack {
   bool built = false;
-  bool tpz = false;                   // forward tables in the Toeplitz layout [z][e1][e2pad][PHI]
+  bool tpz = false;                   // forward tables for the Toeplitz kernels (16-bit: [z][e1][e2pad][PHI],
+                                      // FP32: split fragments, k_pack_fwd_split)
   DevBuf<uint8_t> fwd, bwd;           // [V][z][e_pad64][PHI], [V][z][kPhiPadBwd][e_pad32]
   int64_t pvf = 0, pvb = 0;           // elements per view
   std::vector<int64_t> woff, boff;    // per-plane element offsets inside a view
   std::vector<int32_t> nchunk, epad;
   DevBuf<int64_t> d_woff, d_boff;
   DevBuf<int32_t> d_nchunk, d_epad;
+  DevBuf<int32_t> d_tap_inf;          // FP32 Toeplitz: FwdGeo::tap_inf
   DevBuf<float> d_fscale, d_finv, d_bscale;  // FP16: [V][Z] tap scales (empty otherwise)
 };
 
