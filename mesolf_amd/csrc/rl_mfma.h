@@ -53,8 +53,7 @@ inline __host__ __device__ int bwd_row_cells(int Wd, int nt, int occ) {
 }
 constexpr int kRatioLens = 32;    // lenslets per ratio work entry
 constexpr int kRatioSlices = 8;   // plane slices summed in parallel per entry (x kRatioLens = 256 threads)
-constexpr int kBwdTapPad = 32;    // FP32 backward taps padded to a multiple of 32
-constexpr int kBwdTapPad16 = 64;  // 16-bit: an even number of K-steps of 32 (the K loop runs in pairs)
+constexpr int kBwdTapPad = 64;    // an even number of K-steps of 32 taps (the K loop runs in pairs)
 constexpr int kTpzMTF32 = 2;      // Toeplitz forward: default input columns per wave, f32 (1 also built)
 constexpr int kTpzMTBF16 = 4;     // Toeplitz forward: default input columns per wave, bf16 (2 also built)
 constexpr int kShadowRow = 256;   // BF16 volume shadow: phases per lenslet (zero beyond 225)
@@ -111,7 +110,7 @@ struct BwdGeo {
   const SlotDesc* slots;
   const int32_t* r;       // [Z] backward radius
   const int64_t* boff;    // [Z] element offset of the plane block in the packed view
-  const int32_t* epad;    // [Z] padded tap count (multiple of kBwdTapPad / kBwdTapPad16)
+  const int32_t* epad;    // [Z] padded tap count (multiple of kBwdTapPad)
   const int32_t* sched;   // [entries][5] = (slot, z, b1, b2, first phase group)
   const int32_t* count;
   int view;               // selects the normaliser table of the view
@@ -124,8 +123,6 @@ struct PackGeo {
   const int64_t* src_off;  // [Z] offset in the ABI view block
   const int64_t* dst_off;  // [Z] offset in the packed view block
   int64_t src_view, dst_view;
-  int quad;                // backward pack (16-bit types): taps in K-steps of four 8-tap pieces
-                           // from four consecutive rows (bwd_quad_tap)
   const float* scale;      // [V][Z] factor applied to the taps (FP16), or null
 };
 
@@ -183,7 +180,9 @@ hipError_t launch_pack_fwd_tpz(Precision p, const float* src, void* dst, PackGeo
                                hipStream_t st);
 // elements (of elem_bytes) of one plane's packed Toeplitz taps
 int64_t fwd_tpz_elems(Precision p, int r);
-size_t bwd_smem_bytes(Precision p, int rmax, int epad_max, int nt, int occ);
+size_t bwd_smem_bytes(Precision p, int rmax, int nt, int occ);
+// elements (of elem_bytes) of one plane's packed backprojection taps
+int64_t bwd_plane_elems(Precision p, int epad);
 
 hipError_t launch_fwd_mfma(Precision p, const void* W, FwdGeo g, int grid, size_t smem, int nbuf,
                            hipStream_t st);

@@ -648,17 +648,26 @@ __device__ __forceinline__ unsigned pack_bf16(float lo, float hi) {
   return (unsigned)__builtin_bit_cast(unsigned short, (__bf16)lo) |
          ((unsigned)__builtin_bit_cast(unsigned short, (__bf16)hi) << 16);
 }
-// x, y -> their three BF16 parts, packed in pairs.  A finite value that BF16
-// would round to infinity takes the largest BF16 as its first part.
-__device__ __forceinline__ void split_bf16(float x, float y, unsigned* w) {
-  constexpr float kMax = 3.3895314e38f;
-  w[0] = pack_bf16(fmaxf(fminf(x, kMax), -kMax), fmaxf(fminf(y, kMax), -kMax));
+constexpr float kBF16Max = 3.3895314e38f;
+// x, y -> their three BF16 parts, packed in pairs; w[0] holds the first ones.
+__device__ __forceinline__ void split_rest(float x, float y, unsigned* w) {
 #pragma unroll
   for (int k = 1; k < 3; ++k) {
     x -= __builtin_bit_cast(float, w[k - 1] << 16);
     y -= __builtin_bit_cast(float, w[k - 1] & 0xFFFF0000u);
     w[k] = pack_bf16(x, y);
   }
+}
+// A finite value that BF16 would round to infinity takes the largest BF16 as
+// its first part.
+__device__ __forceinline__ void split_bf16(float x, float y, unsigned* w) {
+  w[0] = pack_bf16(fmaxf(fminf(x, kBF16Max), -kBF16Max), fmaxf(fminf(y, kBF16Max), -kBF16Max));
+  split_rest(x, y, w);
+}
+// Values known to lie within the BF16 range.
+__device__ __forceinline__ void split_finite(float x, float y, unsigned* w) {
+  w[0] = pack_bf16(x, y);
+  split_rest(x, y, w);
 }
 __device__ __forceinline__ bool is_inf(float x) { return __builtin_amdgcn_classf(x, 0x204); }
 
@@ -1150,7 +1159,7 @@ void k_bwd_mfma(const T* __restrict__ Wb, BwdGeo g, float wgt) {
   // none, the epilogue loads each tile one tile ahead.  16-bit with 3 N-tiles
   // has the registers to load every tile's X and 1/B1 rows before the K loop,
   // so its epilogue waits for no load; with 4, every tile's X.
-  constexpr int PRE = OCC >= 3 ? 0 : ((NT == 3 || NT == 4) && M::KPL > 1 ? MT : MT - 1);
+  constexpr int PRE = OCC >= 3 ? 0 : (NT == 3 || NT == 4 ? MT : MT - 1);
   // 3 N-tiles: every tile's 1/B1 rows before the K loop too
   constexpr bool TPRE = PRE == MT && NT == 3;
   static_assert(!SPL || __is_same(T, __bf16), "the split volume is a BF16 form");
@@ -1207,31 +1216,16 @@ void k_bwd_mfma(const T* __restrict__ Wb, BwdGeo g, float wgt) {
     const bool ok1 = a1 < n1;
     const int a1c = ok1 ? a1 : n1 - 1;
     const int c1 = norm_class(a1c, n1, r);
-    // window cell of this lane's lenslet in M-tile mt: base + mt * Wr (16-bit
-    // windows have rows of Wr = bwd_row_cells(Wd) cells; FP32: Wd)
-    const int Wr = KPL > 1 ? bwd_row_cells(Wd, NT, OCC) : Wd;
+    // window cell of this lane's lenslet in M-tile mt: base + mt * Wr
+    const int Wr = bwd_row_cells(Wd, NT, OCC);
     const int base = (lr + r) + (4 * w + r) * Wr;
 
     // ratio window
-    float* Rw = reinterpret_cast<float*>(smem);  // FP32: [Wd][Wd]
-    int* toff = reinterpret_cast<int*>(smem + sizeof(float) * ((Wd * Wd + 7) & ~7));  // FP32: [epad]
     using frag_t = typename M::frag;
-    // 16-bit: [Wd][Wr] after the staging window Rs / tap ring (which alias)
+    // [Wd][Wr] after the staging window Rs / tap ring (which alias)
     frag_t* Rv = reinterpret_cast<frag_t*>(smem + bwd_ring_bytes(Wd, NT, (int)sizeof(T), OCC));
-    if constexpr (KPL == 1) {
-      // FP32: scalar im2col reads, taps e1-fastest
-      gather_window(R, n1, n2, 16 * b1 - r, 16 * b2 - r, Wd, Rw);
-      for (int e = tid; e < epad; e += 256) {
-        int off = 0;  // padded taps have zero weights; any in-window read is fine
-        if (e < ntaps) {
-          const int e2 = e / K, e1 = e - e2 * K;
-          off = -(e1 - r) - (e2 - r) * Wd;
-        }
-        toff[e] = off;
-      }
-      lds_barrier();
-    } else {
-      // 16-bit: a lane's 8 taps of a K-step are 8 consecutive e1 in one row
+    {
+      // a lane's 8 taps of a K-step are 8 consecutive e1 in one row
       // (bwd_quad_tap).  Cell (x, y) of the pre-shifted window holds R(x-j, y)
       // for j = 0..7, so each A fragment is a single 16-byte LDS read.
       float* Rs = reinterpret_cast<float*>(smem);  // [Wd][Wd]
@@ -1430,49 +1424,14 @@ void k_bwd_mfma(const T* __restrict__ Wb, BwdGeo g, float wgt) {
       // issued once every wave is done with the ring, so that they land
       // while this group's update runs (16-bit)
       auto prefetch_next = [&]() {
-        if constexpr (KPL > 1) {
-          if (gi + 1 < g.groups) {
-            lds_barrier();
+        if (gi + 1 < g.groups) {
+          lds_barrier();
   #pragma unroll
-            for (int q = 0; q < STG - SPB; ++q) issue_taps_g(grp + 1, q, q);
-            pref = true;
-          }
+          for (int q = 0; q < STG - SPB; ++q) issue_taps_g(grp + 1, q, q);
+          pref = true;
         }
       };
-      if constexpr (KPL == 1) {
-        load_x(0, MT - 1);
-        load_t(0);
-        // taps in chunks of four K-steps (the pack's chunk order): a lane's
-        // taps of a chunk are one 16-byte load, issued a chunk ahead
-        static_assert(KSTEP == 4, "FP32 K-step of 4 taps");
-        const float* Bl = Bz + (size_t)lr * epad + 4 * lg;
-        floatx4_t bc[NT];
-  #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) bc[nt] = gload(reinterpret_cast<const floatx4_t*>(Bl + (size_t)nt * 16 * epad));
-        const int nc4 = nks / 4;  // epad is a multiple of 32
-        for (int c = 0; c < nc4; ++c) {
-          floatx4_t bx[NT];
-          if (c + 1 < nc4) {
-  #pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-              bx[nt] = gload(reinterpret_cast<const floatx4_t*>(Bl + (size_t)nt * 16 * epad + 16 * (c + 1)));
-          }
-  #pragma unroll
-          for (int s4 = 0; s4 < 4; ++s4) {
-            const int o = toff[(4 * c + s4) * KSTEP + lg];
-  #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-              const typename M::frag af = Rw[base + mt * Wr + o];
-  #pragma unroll
-              for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = M::mma(bc[nt][s4], af, acc[mt][nt]);
-            }
-          }
-          if (c + 1 < nc4) {
-  #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) bc[nt] = bx[nt];
-          }
-        }
-      } else {
+      {
         // the first slices came from the previous group's prefetch: the
         // update's operations issued since are younger than them
         const int upd = pref ? kUpdOps : 0;
@@ -1627,8 +1586,7 @@ void k_bwd_mfma(const T* __restrict__ Wb, BwdGeo g, float wgt) {
               }
             } else {
               __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uintx4, xn), xr, (int)(xbase + 4u * ph), 0, 0);
-              // the 16-bit paths always carry the shadow
-              if constexpr (KPL > 1) __builtin_amdgcn_raw_buffer_store_b64(hi, sr, (int)(sbase + 2u * ph), 0, 0);
+              __builtin_amdgcn_raw_buffer_store_b64(hi, sr, (int)(sbase + 2u * ph), 0, 0);
             }
             continue;
           }
@@ -1750,6 +1708,258 @@ void k_bwd_mfma(const T* __restrict__ Wb, BwdGeo g, float wgt) {
   }
 }
 
+// ------------------------------------------------ backward (split FP32)
+// The FP32 backprojection and update on the BF16 matrix pipe: the GEMM, tap
+// order (bwd_quad_tap) and entries of k_bwd_mfma, with every operand split
+// exactly into three BF16 parts and six MFMAs per product as in k_fwd_tps.
+// The ratio window stays FP32 in LDS, mirrored along axis 0 so that a lane's 8
+// taps are 8 ascending floats, and is split in registers: a window of ready
+// parts would need eight shifted copies to be read 16 bytes at a time (125 KB
+// at radius 17 instead of 16 KB, one workgroup per CU instead of two).  The
+// taps are stored as ready fragments, [16-phase tile][K-step][part][lane][8],
+// and copied into a ring of four K-steps, two per barrier.  The sums of a
+// K-step start from zero and are added by the vector unit (k_fwd_tps): one
+// chain over the K loop left B 2e-7 low, which the view steps compounded to
+// 1.3e-6 of the volume (now 6.1e-7, the FP32 pipe 6.2e-7; 61 x 67 x 51, 3
+// iterations).  Bound by the matrix pipe: 407 us per view at 61 x 67 x 51 (FP32
+// pipe 641), 1.1e15 flop/s issued.  Phase groups of 80: 240 of 225 phases in
+// three groups; groups of 48 measured 580 us (each group splits the window again).
+constexpr int kBwdSplitStages = 4;
+// Floats per window row: room for the 8-tap pieces past the last column, and
+// 16 modulo 32 so that the four rows of a fragment read fall on different banks.
+inline __host__ __device__ constexpr int bwd_split_row(int Wd) { return 16 + 32 * ((Wd + 7 - 16 + 31) / 32); }
+
+template <int NT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+void k_bwd_split(const char* __restrict__ Wb, BwdGeo g, float wgt) {
+  typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+  constexpr int MT = 4;
+  constexpr int PRE = NT == 3 ? MT : 2;  // M-tiles whose X is loaded before the K loop (registers)
+  constexpr int kSlice = NT * 3 * kSplitFrag;
+  extern __shared__ __align__(16) char smem[];
+  const int nent = uni(cload(g.count));
+  for (int ent = blockIdx.x; ent < nent; ent += gridDim.x) {
+    const int* s = g.sched + 5 * ent;
+    const SlotDesc sd = load_slot(g.slots, uni(cload(s)));
+    const int n1 = sd.n1, n2 = sd.n2;
+    const int z = uni(cload(s + 1)), b1 = uni(cload(s + 2)), b2 = uni(cload(s + 3)), grp0 = uni(cload(s + 4));
+    const int r = uni(cload(g.r + z));
+    const int K = 2 * r + 1, nch = (K + 7) / 8;
+    const int nks = uni(cload(g.epad + z)) / 32;
+    const int Wd = 16 + 2 * r, Wr = bwd_split_row(Wd);
+    const int tid = threadIdx.x, lane = tid & 63, w = uni(tid >> 6), lr = lane & 15, lg = lane >> 4;
+    float* const Rw = reinterpret_cast<float*>(smem);  // [Wd][Wr]
+    char* const ring = smem + 4 * Wd * Wr;
+
+    const int C1 = uni(cload(sd.C1 + z)), C2 = norm_classes(n2, r);
+    const size_t nlp = (size_t)n2 * n1;
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+        sd.X + z * nlp * kXRow, 0, (int)(nlp * kXRow * 4), kBufferDword3);
+    const __amdgpu_buffer_rsrc_t tr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(sd.Tn + (size_t)g.view * sd.pvt + uni64(cload(sd.toffT + z))), 0, C2 * C1 * kNormRow * 4,
+        kBufferDword3);
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char*>(Wb) + 4 * uni64(cload(g.boff + z)), 0, kPhiPadBwd / 16 * nks * 3 * kSplitFrag, kBufferDword3);
+    const int a1 = 16 * b1 + lr;
+    const bool ok1 = a1 < n1;
+    const int a1c = ok1 ? a1 : n1 - 1;
+    const int c1 = norm_class(a1c, n1, r);
+
+    // copies of K-step ks of phase group gx into ring slot ks % stages
+    auto issue_taps = [&](int gx, int ks) {
+      if (ks >= nks) return;  // wave-uniform
+      char* dst = ring + (ks % kBwdSplitStages) * kSlice;
+#pragma unroll
+      for (int i = 0; i < (NT * 3 + 3) / 4; ++i) {
+        const int c = 4 * i + w;  // fragment: tile c / 3, part c % 3
+        if (c >= NT * 3) break;
+        const int so = ((gx * NT + c / 3) * nks + ks) * 3 * kSplitFrag + (c % 3) * kSplitFrag;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (__attribute__((address_space(3))) void*)(dst + c * kSplitFrag), 16,
+                                                 16 * lane, so, 0, 0);
+      }
+    };
+    issue_taps(grp0, 0);
+    issue_taps(grp0, 1);
+    // window: column x of row y at Wd - 1 - x, the rest of a row zero; ratios
+    // past the largest BF16 (never reached by photon counts) are cut to it
+    {
+      const __amdgpu_buffer_rsrc_t rr = __builtin_amdgcn_make_buffer_rsrc(sd.R, 0, (int)(nlp * 4), kBufferDword3);
+      constexpr int kPer = 8;
+      for (int c0 = 0; c0 < Wd * Wr; c0 += 256 * kPer) {
+        float v[kPer];
+#pragma unroll
+        for (int q = 0; q < kPer; ++q) {
+          const int o = c0 + tid + 256 * q, y = o / Wr, x = Wd - 1 - (o - y * Wr);
+          const int i1 = 16 * b1 - r + x, i2 = 16 * b2 - r + y;
+          const bool in = x >= 0 && i1 >= 0 && i1 < n1 && i2 >= 0 && i2 < n2;
+          v[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                               rr, in ? 4u * (unsigned)(i2 * n1 + i1) : 0x80000000u, 0, 0));
+        }
+#pragma unroll
+        for (int q = 0; q < kPer; ++q) {
+          const int o = c0 + tid + 256 * q;
+          if (o < Wd * Wr) Rw[o] = fminf(v[q], kBF16Max);
+        }
+      }
+    }
+
+    for (int gi = 0; gi < g.groups; ++gi) {
+      const int grp = grp0 + gi;
+      const int gbase = grp * 16 * NT;
+      floatx4 acc[MT][NT];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
+      floatx4 xv[MT][NT], bv[NT];
+      auto lens_of = [&](int mt) {
+        const int a2 = 16 * b2 + 4 * w + mt;
+        return (a2 < n2 ? a2 : n2 - 1) * n1 + a1c;
+      };
+      auto load_x = [&](int mt) {
+        const int o = 4 * (lens_of(mt) * kXRow + gbase + 4 * lg);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+          xv[mt][nt] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(xr, o, 64 * nt, 0));
+      };
+      auto load_t = [&](int mt, floatx4* d) {
+        const int a2 = 16 * b2 + 4 * w + mt;
+        const int o = 4 * ((norm_class(a2 < n2 ? a2 : n2 - 1, n2, r) * C1 + c1) * kNormRow + gbase + 4 * lg);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+          d[nt] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(tr, o, 64 * nt, 0));
+      };
+#pragma unroll
+      for (int mt = 0; mt < PRE; ++mt) load_x(mt);
+
+      int qb = 0, qc = 0;
+      for (int ks = 0; ks < nks; ks += 2) {
+        // this pair's copies have landed.  The first pair's are older than the
+        // X loads and (after a group) the previous update's stores.
+        if (ks > 0) wait_vm<0>();
+        else if (gi > 0) wait_vm<(PRE + MT) * NT>();
+        else wait_vm<PRE * NT>();
+        lds_barrier();
+        issue_taps(grp, ks + 2);
+        issue_taps(grp, ks + 3);
+#pragma unroll 1
+        for (int h = 0; h < 2; ++h) {
+          const char* T = ring + ((ks + h) % kBwdSplitStages) * kSlice + 16 * lane;
+          const int e2 = min(4 * qb + lg, K - 1);
+          const float* R0 = Rw + (4 * w + 2 * r - e2) * Wr + 15 - lr + 8 * qc;
+          if (++qc == nch) {
+            qc = 0;
+            ++qb;
+          }
+          bf16x8 wn[MT][3];
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt) {
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = R0[mt * Wr + j];
+            unsigned p[4][3];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) split_finite(v[2 * j], v[2 * j + 1], p[j]);
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+              wn[mt][q] = __builtin_bit_cast(bf16x8, uintx4{p[0][q], p[1][q], p[2][q], p[3][q]});
+          }
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) {
+            bf16x8 b[3];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) b[q] = *reinterpret_cast<const bf16x8*>(T + (3 * nt + q) * kSplitFrag);
+            constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+            floatx4 c[MT];
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) c[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < 6; ++i)
+#pragma unroll
+              for (int mt = 0; mt < MT; ++mt)
+                c[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[pb[i]], wn[mt][pa[i]], c[mt], 0, 0, 0);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) acc[mt][nt] += c[mt];
+          }
+        }
+      }
+
+      // fused multiplicative update (recon:130-137): the remaining X and the 1/B1
+      // rows of two tiles first, then the next group's first tap slices, then
+      // tile by tile, the rows of tile mt + 2 requested behind tile mt's stores
+      auto update_tile = [&](int mt, const floatx4* x4, const floatx4* b4) {
+        const bool ok = ok1 && 16 * b2 + 4 * w + mt < n2;
+        const unsigned base = ok ? 4u * (unsigned)(lens_of(mt) * kXRow) : 0x80000000u;
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+          const int ph = gbase + 16 * nt + 4 * lg;
+          floatx4 xn;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float x = x4[nt][j];
+            float C = x * acc[mt][nt][j] * b4[nt][j];
+            C = __builtin_amdgcn_classf(C, 0x1E0) ? C : 0.f;  // NaN, infinities and negatives -> 0
+            const float v = C * wgt + (1.f - wgt) * x;
+            xn[j] = v < 0.f ? 0.f : v;
+          }
+          if (gbase + 16 * nt + 16 <= kP) {  // wave-uniform
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uintx4, xn), xr, (int)(base + 4u * ph), 0, 0);
+          } else {  // the tile that reaches past phase 224 (and empty ones)
+            const unsigned o4 = ok && ph + 4 <= kP ? base + 4u * ph : 0x80000000u;
+            const unsigned o1 = ok && ph < kP && ph + 4 > kP ? base + 4u * ph : 0x80000000u;
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uintx4, xn), xr, (int)o4, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, xn[0]), xr, (int)o1, 0, 0);
+          }
+        }
+      };
+      floatx4 bt[2][NT];
+#pragma unroll
+      for (int mt = PRE; mt < MT; ++mt) load_x(mt);
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt) load_t(mt, bt[mt]);
+      lds_barrier();  // every wave is done with the ring (and, after the last group, the window)
+      if (gi + 1 < g.groups) {
+        issue_taps(grp + 1, 0);
+        issue_taps(grp + 1, 1);
+      }
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        update_tile(mt, xv[mt], bt[mt & 1]);
+        if (mt < 2) load_t(mt + 2, bt[mt & 1]);
+      }
+    }
+  }
+}
+
+// ABI block [e][phase] -> the fragments of k_bwd_split.
+__global__ void k_pack_bwd_split(const float* __restrict__ src, char* __restrict__ dst, PackGeo pg) {
+  typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+  const int z = blockIdx.y, v = blockIdx.z;
+  const int K = 2 * pg.r[z] + 1;
+  const int nks = (int)(pg.rows[z] / 32);
+  const float* s = src + (size_t)v * pg.src_view + pg.src_off[z];
+  char* d = dst + 4 * ((size_t)v * pg.dst_view + pg.dst_off[z]);
+  const size_t total = (size_t)(kPhiPadBwd / 16) * nks * 64;
+  for (size_t o = blockIdx.x * (size_t)blockDim.x + threadIdx.x; o < total; o += (size_t)gridDim.x * blockDim.x) {
+    const int lane = (int)(o & 63);
+    const size_t f = o >> 6;  // tile nks + ks
+    const int ks = (int)(f % nks), ph = 16 * (int)(f / nks) + (lane & 15);
+    float x[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      int e2, e1;
+      bwd_quad_tap(32 * ks + 8 * (lane >> 4) + j, K, &e2, &e1);
+      x[j] = ph < kP && e2 < K && e1 < K ? s[((size_t)e2 * K + e1) * kP + ph] : 0.f;
+    }
+    unsigned p[4][3];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) split_bf16(x[2 * j], x[2 * j + 1], p[j]);
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      *reinterpret_cast<uintx4*>(d + (f * 3 + q) * kSplitFrag + 16 * lane) = uintx4{p[0][q], p[1][q], p[2][q], p[3][q]};
+  }
+}
+
 // ------------------------------------------------------------ table packing
 // ABI block [e][phase] (phase fastest, 225) -> forward pack [e_pad][PHI].
 template <typename T>
@@ -1776,7 +1986,7 @@ template <typename T>
 __global__ void k_pack_bwd(const float* __restrict__ src, T* __restrict__ dst, PackGeo pg) {
   const int z = blockIdx.y, v = blockIdx.z;
   const float sc = pg.scale ? pg.scale[(size_t)v * gridDim.y + z] : 1.f;
-  const int K = 2 * pg.r[z] + 1, ntaps = K * K;
+  const int K = 2 * pg.r[z] + 1;
   const size_t epad = (size_t)pg.rows[z];
   const float* s = src + (size_t)v * pg.src_view + pg.src_off[z];
   T* d = dst + (size_t)v * pg.dst_view + pg.dst_off[z];
@@ -1784,19 +1994,10 @@ __global__ void k_pack_bwd(const float* __restrict__ src, T* __restrict__ dst, P
        o += (size_t)gridDim.x * blockDim.x) {
     const int ph = (int)(o / epad), t = (int)(o % epad);
     int e2, e1;
-    if (pg.quad) {
-      bwd_quad_tap(t, K, &e2, &e1);
-    } else {
-      // FP32: taps e1-fastest, dense, stored in chunks of 16 (four K-steps of
-      // 4) lane-group-major: position 16 c + 4 g + s holds tap 16 c + 4 s + g,
-      // so lane group g reads its taps of the four steps with one 16-byte load
-      const int lt = (t & ~15) | ((t & 3) << 2) | ((t >> 2) & 3);
-      e2 = lt / K;
-      e1 = lt - e2 * K;
-    }
+    bwd_quad_tap(t, K, &e2, &e1);
     const bool ok = ph < kP && e2 < K && e1 < K;
-    // 16-bit: tile-major, [16-row tile][K-step of 32 taps][16 rows][32 taps]
-    const size_t od = pg.quad ? (size_t)(ph >> 4) * 16 * epad + (size_t)(t >> 5) * 512 + (ph & 15) * 32 + (t & 31) : o;
+    // tile-major, [16-row tile][K-step of 32 taps][16 rows][32 taps]
+    const size_t od = (size_t)(ph >> 4) * 16 * epad + (size_t)(t >> 5) * 512 + (ph & 15) * 32 + (t & 31);
     d[od] = (T)(ok ? s[((size_t)e2 * K + e1) * kP + ph] * sc : 0.f);
   }
 }
@@ -1868,9 +2069,10 @@ size_t fwd_smem_bytes(Precision p, int rmax, int bm2) {
   return fwd_smem_nbuf(p, rmax, bm2, fwd_nbuf(p, rmax, bm2));
 }
 
-size_t bwd_smem_bytes(Precision p, int rmax, int epad_max, int nt, int occ) {
+size_t bwd_smem_bytes(Precision p, int rmax, int nt, int occ) {
   const int Wd = 16 + 2 * rmax;
-  if (p == Precision::kF32) return sizeof(float) * ((Wd * Wd + 7) & ~7) + sizeof(int) * epad_max;
+  if (p == Precision::kF32)
+    return sizeof(float) * (size_t)Wd * bwd_split_row(Wd) + (size_t)kBwdSplitStages * nt * 3 * kSplitFrag;
   return bwd_ring_bytes(Wd, nt, 2, occ) + 16 * (size_t)Wd * bwd_row_cells(Wd, nt, occ);
 }
 
@@ -2081,9 +2283,9 @@ hipError_t launch_bwd_mfma(Precision p, int nt, int occ, bool split, const void*
   if (split && p != Precision::kBF16) return hipErrorInvalidValue;
   if (p == Precision::kF32) {
     if (nt == 3)
-      hipLaunchKernelGGL((k_bwd_mfma<float, 3, 2, false>), dim3(grid), dim3(256), smem, st, (const float*)Wb, g, w);
+      hipLaunchKernelGGL(k_bwd_split<3>, dim3(grid), dim3(256), smem, st, (const char*)Wb, g, w);
     else
-      hipLaunchKernelGGL((k_bwd_mfma<float, 5, 2, false>), dim3(grid), dim3(256), smem, st, (const float*)Wb, g, w);
+      hipLaunchKernelGGL(k_bwd_split<5>, dim3(grid), dim3(256), smem, st, (const char*)Wb, g, w);
   } else if (p == Precision::kF16) {
     launch_bwd_t<_Float16, false>(nt, occ, Wb, g, grid, smem, w, st);
   } else if (split) {
@@ -2104,11 +2306,16 @@ hipError_t launch_pack_fwd(Precision p, const float* src, void* dst, PackGeo pg,
   return hipGetLastError();
 }
 
+int64_t bwd_plane_elems(Precision p, int epad) {
+  return p == Precision::kF32 ? (int64_t)(kPhiPadBwd / 16) * (epad / 32) * 3 * (kSplitFrag / 4)
+                              : (int64_t)kPhiPadBwd * epad;
+}
+
 hipError_t launch_pack_bwd(Precision p, const float* src, void* dst, PackGeo pg, int Z, int V,
                            hipStream_t st) {
   dim3 grid(64, Z, V);
   if (p == Precision::kF32)
-    hipLaunchKernelGGL(k_pack_bwd<float>, grid, dim3(256), 0, st, src, (float*)dst, pg);
+    hipLaunchKernelGGL(k_pack_bwd_split, grid, dim3(256), 0, st, src, (char*)dst, pg);
   else if (p == Precision::kF16)
     hipLaunchKernelGGL(k_pack_bwd<_Float16>, grid, dim3(256), 0, st, src, (_Float16*)dst, pg);
   else
@@ -2143,8 +2350,8 @@ hipError_t mfma_kernel_attributes() {
       reinterpret_cast<const void*>(&k_fwd_tps<2>),
       reinterpret_cast<const void*>(&k_fwd_tpz<__bf16, 2>),
       reinterpret_cast<const void*>(&k_fwd_tpz<__bf16, 4>),
-      reinterpret_cast<const void*>(&k_bwd_mfma<float, 3, 2, false>),
-      reinterpret_cast<const void*>(&k_bwd_mfma<float, 5, 2, false>),
+      reinterpret_cast<const void*>(&k_bwd_split<3>),
+      reinterpret_cast<const void*>(&k_bwd_split<5>),
       reinterpret_cast<const void*>(&k_fwd_tpz<_Float16, 2>),
       reinterpret_cast<const void*>(&k_fwd_tpz<_Float16, 4>),
       reinterpret_cast<const void*>(&k_bwd_mfma<_Float16, 3, 2, false>),

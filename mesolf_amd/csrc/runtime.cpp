@@ -305,18 +305,15 @@ static mlf_status psf_ensure_pack(mlf_psf_s* ps, Precision prec) {
   int64_t of = 0, ob = 0;
   for (int z = 0; z < Z; ++z) {
     const int nt_f = (2 * ps->rf[z] + 1) * (2 * ps->rf[z] + 1);
-    const int nt_b = (2 * ps->rb[z] + 1) * (2 * ps->rb[z] + 1);
     pk.nchunk[z] = (nt_f + kFwdChunk - 1) / kFwdChunk;
     rows_f[z] = pk.nchunk[z] * kFwdChunk;
     const int Kb = 2 * ps->rb[z] + 1;
-    const int nt_b_pad = prec != Precision::kF32 ? 32 * bwd_quad_steps(Kb) : nt_b;
-    const int tpad = prec != Precision::kF32 ? kBwdTapPad16 : kBwdTapPad;
-    pk.epad[z] = (nt_b_pad + tpad - 1) / tpad * tpad;
+    pk.epad[z] = (32 * bwd_quad_steps(Kb) + kBwdTapPad - 1) / kBwdTapPad * kBwdTapPad;
     rows_b[z] = pk.epad[z];
     pk.woff[z] = of;
     of += pk.tpz ? fwd_tpz_elems(prec, ps->rf[z]) : (int64_t)rows_f[z] * phi;
     pk.boff[z] = ob;
-    ob += (int64_t)kPhiPadBwd * pk.epad[z];
+    ob += bwd_plane_elems(prec, pk.epad[z]);
   }
   pk.pvf = of;
   pk.pvb = ob;
@@ -342,14 +339,14 @@ static mlf_status psf_ensure_pack(mlf_psf_s* ps, Precision prec) {
     MLF_LAUNCH(launch_block_scale(ps->bwd.ptr, ps->d_offb.ptr, ps->d_rb.ptr, ps->per_view_b, Z, V,
                                   pk.d_bscale.ptr, nullptr, ps->ctx->stream));
   }
-  PackGeo gf{ps->d_rf.ptr, d_rows_f.ptr, ps->d_offf.ptr, pk.d_woff.ptr, ps->per_view_f, pk.pvf, 0,
+  PackGeo gf{ps->d_rf.ptr, d_rows_f.ptr, ps->d_offf.ptr, pk.d_woff.ptr, ps->per_view_f, pk.pvf,
              pk.d_fscale.ptr};
   MLF_CHECK(upload_vec(pk.d_tap_inf, std::vector<int32_t>{0}));
   hipError_t e = pk.tpz ? launch_pack_fwd_tpz(prec, ps->fwd.ptr, pk.fwd.ptr, gf, Z, V, pk.d_tap_inf.ptr, st)
                         : launch_pack_fwd(prec, ps->fwd.ptr, pk.fwd.ptr, gf, Z, V, st);
   if (e != hipSuccess) return set_error(MLF_ERR_DEVICE, "pack_fwd: %s", hipGetErrorString(e));
   PackGeo gb{ps->d_rb.ptr, d_rows_b.ptr, ps->d_offb.ptr, pk.d_boff.ptr, ps->per_view_b, pk.pvb,
-             prec != Precision::kF32 ? 1 : 0, pk.d_bscale.ptr};
+             pk.d_bscale.ptr};
   e = launch_pack_bwd(prec, ps->bwd.ptr, pk.bwd.ptr, gb, Z, V, st);
   if (e != hipSuccess) return set_error(MLF_ERR_DEVICE, "pack_bwd: %s", hipGetErrorString(e));
   MLF_HIP(hipStreamSynchronize(st));
@@ -1108,11 +1105,10 @@ mlf_status mlf::patch_setup_tiles(mlf_patch_s* p) {
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return ps->rf[a] > ps->rf[b]; });
   std::vector<int64_t> poff(Z);
   const int64_t po = partial_elems(ps, p->tpz, p->cw, p->bm2, p->n1, p->n2, &poff);
-  int rfmax = 0, rbmax = 0, epmax = 0;
+  int rfmax = 0, rbmax = 0;
   for (int z = 0; z < Z; ++z) {
     rfmax = std::max(rfmax, ps->rf[z]);
     rbmax = std::max(rbmax, ps->rb[z]);
-    epmax = std::max(epmax, ps->pack[(int)p->kp].epad[z]);
   }
   p->fent.clear();
   for (int z : order)
@@ -1190,7 +1186,7 @@ mlf_status mlf::patch_setup_tiles(mlf_patch_s* p) {
   MLF_CHECK(upload_vec(p->d_slot, std::vector<SlotDesc>{sd}));
   p->smem_f = p->tpz ? tpz_smem_bytes(p->kp, rfmax, p->fwd_mt) : fwd_smem_bytes(p->kp, rfmax, p->bm2);
   p->fwd_nbuf = fwd_nbuf(p->kp, rfmax, p->bm2);
-  p->smem_b = bwd_smem_bytes(p->kp, rbmax, epmax, p->bwd_nt, p->bwd_occ);
+  p->smem_b = bwd_smem_bytes(p->kp, rbmax, p->bwd_nt, p->bwd_occ);
   if (p->smem_f > 160 * 1024 || p->smem_b > 160 * 1024)
     return set_error(MLF_ERR_UNSUPPORTED,
                      "PSF radius too large for the LDS tiles (rf_max=%d, rb_max=%d)", rfmax, rbmax);
