@@ -150,8 +150,10 @@ size_t summary_scratch_doubles(size_t npix, int T);
 // global != 0: the 'global' detrend (std image with the rank-1 background,
 // summary_image_generation_module.m:43-60); dbuf, w1, w2 and p are unused.
 hipError_t launch_summary(const float* Y, size_t npix, int T, int w1, int w2, int p, int bg_iter,
-                          int global, double* scratch, float* dbuf, double* img, double* s,
+                          int global, double* scratch, float* dbuf, double* img, double* s, int cus,
                           hipStream_t st);
+// whether launch_summary keeps a detrended movie in dbuf [npix, T] ('pixelwise')
+bool summary_needs_movie(size_t npix, int T);
 const double* summary_temporal(const double* scratch);
 // Bilinear (griddedInterpolant 'linear', extrapolating) resample of n frames
 // [H, W] at yq [Hq] x xq [Wq] (device arrays, 1-based pixel coordinates).

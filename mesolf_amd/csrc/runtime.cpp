@@ -2191,14 +2191,16 @@ static mlf_status summary_device(mlf_context ctx, const float* d_movie, int64_t 
   DevBuf<double> scratch, s_own;
   DevBuf<float> dbuf;
   MLF_CHECK(scratch.alloc(summary_scratch_doubles(npix, T)));
-  if (!global) MLF_CHECK(dbuf.alloc(npix * (size_t)T));
+  if (!global && summary_needs_movie(npix, T)) MLF_CHECK(dbuf.alloc(npix * (size_t)T));
   double* s = d_bg_spatial;
   if (!s) {
     MLF_CHECK(s_own.alloc(npix));
     s = s_own.ptr;
   }
+  int cus = 0;
+  MLF_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
   MLF_LAUNCH(launch_summary(d_movie, npix, T, window_1, window_2, poly_index, bg_iter, global,
-                            scratch.ptr, dbuf.ptr, d_summary, s, ctx->stream));
+                            scratch.ptr, dbuf.ptr, d_summary, s, cus, ctx->stream));
   if (d_bg_temporal)
     MLF_HIP(hipMemcpyAsync(d_bg_temporal, summary_temporal(scratch.ptr), sizeof(double) * T,
                            hipMemcpyDeviceToDevice, ctx->stream));

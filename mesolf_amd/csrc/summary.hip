@@ -13,6 +13,8 @@
 // a = b = (k-1)/2 for odd k, a = k/2, b = k/2 - 1 for even k, kept as a
 // running FP64 sum (one sample enters and one leaves per frame; the leaving
 // sample is read again, from cache).
+#include <algorithm>
+
 #include "internal.h"
 
 namespace mlf {
@@ -360,6 +362,425 @@ __global__ __launch_bounds__(kThreads) void k_rectify(const float* __restrict__ 
   }
 }
 
+// ---------------------------------------------------------------- tile passes
+// Movies whose tiles fit LDS (up to about 950 frames): every pass over the movie holds one tile
+// of P pixels x T frames in LDS, so a rank-1 round (Y t, then s'Y) reads the
+// movie once instead of twice, the first pass takes the maximum along, and the
+// last round's Y t, the detrend, the smoothing and the std image share one
+// read with no detrended movie in memory: 6 reads of the movie for 5 rounds
+// instead of 13 and a write.  765 x 750 x 400: 2.26 ms a call (the passes above:
+// 4.15), 0.24 ms per round (3.8 TB/s; k_r1_tdot + k_r1_sdot 0.48).  A workgroup
+// requests its next tile into registers before it computes on the one in LDS
+// (tiles of 64 pixels x 400 frames leave room for one workgroup per CU; 1024
+// threads rather than 512: 0.28 ms per round).  Tile passes go to
+// consecutive workgroups of one XCD, so that the cache lines that two tiles
+// share are read once.
+//
+// The rounds keep s unscaled: t is divided by its norm anyway, and a positive
+// factor of s changes nothing before that.
+struct TileArgs {
+  const float* Y;
+  size_t npix;
+  int T;
+  const double* mx;     // movie maximum
+  const double* tt;     // unscaled temporal component [T]
+  double* tparts;       // [T][workgroups]: partial s'Y
+  double* parts;        // [workgroups]: partial maxima (movie, or image)
+  // last pass
+  double* s;            // spatial component
+  double* img;
+  double* t_out;        // tt / |tt|
+  int w1, w2, p;
+};
+
+constexpr size_t kTileLds = 160 * 1024;
+constexpr int kTileThreads = 1024;
+constexpr int kRun = 8;  // frames per run of the last pass
+enum TileMode { kTileFirst, kTileRound, kTileLast, kTileLastGlobal };
+inline __host__ __device__ size_t tile_rows_bytes(int P, int T) { return ((size_t)T * (P + 1) * 4 + 15) / 16 * 16; }
+size_t tile_lds(int P, int T, int mode) {
+  const size_t common = tile_rows_bytes(P, T) + 8 * ((size_t)T + 2 * kTileThreads + P);
+  return mode <= kTileRound
+             ? common
+             : common + tile_rows_bytes(P, T) + 8 * ((size_t)((T + kRun - 1) / kRun) * P + 2 * (size_t)T);
+}
+
+__device__ __forceinline__ double tile_reduce(double v, double* sh, bool max) {
+  for (int off = 32; off > 0; off >>= 1) {
+    const double o = __shfl_down(v, off, 64);
+    v = max ? nmax(v, o) : v + o;
+  }
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  __syncthreads();
+  if (lane == 0) sh[wid] = v;
+  __syncthreads();
+  double r = sh[0];
+  for (int k = 1; k < kTileThreads / 64; ++k) r = max ? nmax(r, sh[k]) : r + sh[k];
+  return r;
+}
+
+// Registers of one tile's samples: thread (i, q) holds pixel i of frames q,
+// q + G, ...  A wave's rows are uniform neighbours, so a load takes a scalar row
+// address and a 32-bit lane offset.  Past the last frame or pixel a load
+// repeats a valid one (its value is not used).
+template <int P, int R>
+struct TileRegs {
+  static constexpr int G = kTileThreads / P;
+  float v[R];
+  __device__ __forceinline__ void load(const float* __restrict__ Y, size_t npix, int T, size_t tile) {
+    const int tid = threadIdx.x;
+    const size_t px = tile * P + tid % P;
+    const unsigned vo = 4u * (unsigned)(px < npix ? px : npix - 1);
+    const int sub = (tid & 63) / P;
+    const unsigned vs = vo + 4u * (unsigned)npix * sub;
+    int row = __builtin_amdgcn_readfirstlane(tid >> 6) * (64 / P);
+    asm volatile("" : "+s"(row));  // else every row address is kept over the tile loop, in spilled registers
+    const char* base = reinterpret_cast<const char*>(Y) + 4 * npix * (size_t)row;
+#pragma unroll
+    for (int k = 0; k < R; k += 8) {
+      if (k * G < T) {
+#pragma unroll
+        for (int h = 0; h < 8; ++h) {
+          const char* b = row < T ? base : reinterpret_cast<const char*>(Y);
+          v[k + h] = *reinterpret_cast<const float*>(b + (P == 64 || row + sub < T ? vs : vo));
+          row += G;
+          base += 4 * npix * G;
+        }
+      }
+    }
+  }
+};
+
+// first tile of a workgroup: 32 consecutive tiles per XCD (blockIdx % 8) and round
+__device__ __forceinline__ size_t first_tile() {
+  const unsigned n = gridDim.x;
+  return n % 8 == 0 ? (blockIdx.x & 7) * (n / 8) + (blockIdx.x >> 3) : blockIdx.x;
+}
+
+// tile -> LDS; `t` (null: not wanted): this thread's part of Y t
+template <int P, int R, typename F>
+__device__ __forceinline__ void tile_store(const TileRegs<P, R>& regs, float* Yt, int T, bool in, F&& each) {
+  constexpr int G = kTileThreads / P, LD = P + 1;
+  const int i = threadIdx.x % P, q = threadIdx.x / P;
+#pragma unroll
+  for (int k = 0; k < R; k += 8) {
+    if (k * G < T) {
+#pragma unroll
+      for (int h = 0; h < 8; ++h) {
+        const int j = q + (k + h) * G;
+        const float x = in ? regs.v[k + h] : 0.f;
+        if (j < T) {
+          Yt[j * LD + i] = x;
+          each(j, x);
+        }
+      }
+    }
+  }
+}
+
+// t = tt / |tt| in LDS
+__device__ __forceinline__ void tile_temporal(const TileArgs& g, double* td, double* red, bool write) {
+  double ss = 0.0;
+  for (int j = threadIdx.x; j < g.T; j += kTileThreads) ss = fma(g.tt[j], g.tt[j], ss);
+  const double nrm = sqrt(tile_reduce(ss, red, false));
+  for (int j = threadIdx.x; j < g.T; j += kTileThreads) {
+    const double t = g.tt[j] / nrm;
+    td[j] = t;
+    if (write) g.t_out[j] = t;
+  }
+  __syncthreads();
+}
+
+// kTileFirst: partial maxima and s'Y of the constant s; kTileRound: s = Y t, then s'Y
+template <int P, int R, int MODE>
+__global__ __launch_bounds__(kTileThreads) void k_summary_round(TileArgs g) {
+  constexpr int NT = kTileThreads, G = NT / P;
+  constexpr int LD = P + 1;                      // odd: lanes along the frames fall on different banks
+  constexpr int kFrames = (1200 + NT - 1) / NT;  // frames per thread of s'Y
+  extern __shared__ __align__(16) char lds[];
+  const int T = g.T, tid = threadIdx.x;
+  float* Yt = reinterpret_cast<float*>(lds);  // [T][LD]
+  double* td = reinterpret_cast<double*>(lds + tile_rows_bytes(P, T));
+  double* red = td + T;        // [2 NT]
+  double* vs = red + 2 * NT;   // [P]
+  const size_t npix = g.npix, ntile = (npix + P - 1) / P, nwg = gridDim.x;
+  TileRegs<P, R> regs;
+  size_t tile = first_tile();
+  if (tile < ntile) regs.load(g.Y, npix, T, tile);
+  const double mx = MODE == kTileFirst ? 1.0 : *g.mx;
+  if constexpr (MODE == kTileFirst) {
+    if (tid < P) vs[tid] = 1.0 / sqrt((double)npix);
+  } else {
+    tile_temporal(g, td, red, false);
+  }
+  double acc[kFrames];
+#pragma unroll
+  for (int k = 0; k < kFrames; ++k) acc[k] = 0.0;
+  float mf = __builtin_nanf("");
+  for (; tile < ntile; tile += nwg) {
+    const bool in = tile * P + tid % P < npix;
+    double a = 0.0;
+    tile_store(regs, Yt, T, in, [&](int j, float x) {
+      if constexpr (MODE == kTileFirst) mf = in ? fmaxf(mf, x) : mf;  // NaN ignored
+      else a = fma((double)x, td[j], a);
+    });
+    if constexpr (MODE == kTileRound) red[tid] = a;
+    __syncthreads();
+    if (tile + nwg < ntile) regs.load(g.Y, npix, T, tile + nwg);  // in flight while this tile is worked on
+    if constexpr (MODE == kTileRound) {
+      if (tid < P) {
+        double r = red[tid];
+#pragma unroll
+        for (int k = 1; k < G; ++k) r += red[tid + k * P];
+        vs[tid] = r / mx;
+      }
+      __syncthreads();
+    }
+#pragma unroll
+    for (int k = 0; k < kFrames; ++k) {
+      const int j = tid + k * NT;
+      if (j < T) {
+        double r0 = 0.0, r1 = 0.0;
+#pragma unroll 8
+        for (int c = 0; c < P; c += 2) {
+          r0 = fma((double)Yt[j * LD + c], vs[c], r0);
+          r1 = fma((double)Yt[j * LD + c + 1], vs[c + 1], r1);
+        }
+        acc[k] += r0 + r1;
+      }
+    }
+    __syncthreads();  // the tile, red and vs are rewritten
+  }
+#pragma unroll
+  for (int k = 0; k < kFrames; ++k) {
+    const int j = tid + k * NT;
+    if (j < T) g.tparts[(size_t)j * nwg + blockIdx.x] = acc[k];
+  }
+  if constexpr (MODE == kTileFirst) {
+    const double m = tile_reduce((double)mf, red, true);
+    if (tid == 0) g.parts[blockIdx.x] = m;
+  }
+}
+
+// sums of whole runs of kRun rows of pixel i, by threads (i, q)
+template <int P>
+__device__ __forceinline__ void run_sums(const float* rows, double* runs, int T) {
+  for (int c = threadIdx.x / P; c < T / kRun; c += kTileThreads / P) {
+    const float* y = rows + c * kRun * (P + 1) + threadIdx.x % P;
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < kRun; ++k) s += (double)y[k * (P + 1)];
+    runs[c * P + threadIdx.x % P] = s;
+  }
+}
+// sum of rows lo .. hi of this thread's pixel, whole runs from their sums
+template <int P>
+__device__ __forceinline__ double window_sum(const float* y, const double* runs, int lo, int hi) {
+  double s = 0.0;
+  const int c0 = (lo + kRun - 1) / kRun, c1 = (hi + 1) / kRun;
+  if (c0 >= c1) {
+    for (int k = lo; k <= hi; ++k) s += (double)y[k * (P + 1)];
+    return s;
+  }
+  for (int k = lo; k < c0 * kRun; ++k) s += (double)y[k * (P + 1)];
+  for (int c = c0; c < c1; ++c) s += runs[c * P];
+  for (int k = c1 * kRun; k <= hi; ++k) s += (double)y[k * (P + 1)];
+  return s;
+}
+
+// The last round's s = Y t and the image.  'pixelwise': the detrended tile
+// (FP32, as k_detrend stores it) in LDS beside the samples; a thread walks runs
+// of 8 frames, each window sum started from the sums of whole runs.  0.90 ms at
+// 765 x 750 x 400 (k_r1_sdot + k_detrend + k_smooth_std: 1.23 ms), bound by the
+// LDS reads and FP64 chains of the windows; one running sum over a quarter of
+// the frames per thread took 2.4 ms, 512 threads instead of 1024 1.15 ms.
+template <int P, int R, int MODE>
+__global__ __launch_bounds__(kTileThreads) void k_summary_last(TileArgs g) {
+  constexpr int NT = kTileThreads, G = NT / P, LD = P + 1;
+  extern __shared__ __align__(16) char lds[];
+  const int T = g.T, tid = threadIdx.x, i = tid % P, q = tid / P;
+  float* Yt = reinterpret_cast<float*>(lds);                            // [T][LD]
+  float* Dt = reinterpret_cast<float*>(lds + tile_rows_bytes(P, T));    // [T][LD]
+  double* td = reinterpret_cast<double*>(lds + 2 * tile_rows_bytes(P, T));
+  double* red = td + T;        // [2 NT]
+  double* vs = red + 2 * NT;   // [P]
+  double* rk1 = vs + P;        // [T] 1 / (samples in the window of frame j), window_1
+  double* rk2 = rk1 + T;       // [T] window_2
+  double* runs = rk2 + T;      // [T / kRun][P]
+  const size_t npix = g.npix, ntile = (npix + P - 1) / P, nwg = gridDim.x;
+  TileRegs<P, R> regs;
+  size_t tile = first_tile();
+  if (tile < ntile) regs.load(g.Y, npix, T, tile);
+  const double mx = *g.mx, minv = 1.0 / mx;
+  tile_temporal(g, td, red, blockIdx.x == 0);
+  double tc = 0.0;  // 'global': mean of t
+  if constexpr (MODE == kTileLastGlobal) {
+    for (int j = 0; j < T; ++j) tc += td[j];
+    tc /= (double)T;
+  }
+  int a1, b1, a2, b2;
+  window_of(g.w1, &a1, &b1);
+  window_of(g.w2, &a2, &b2);
+  for (int j = tid; j < T; j += NT) {
+    rk1[j] = 1.0 / (double)(min(j + b1, T - 1) - max(j - a1, 0) + 1);
+    rk2[j] = 1.0 / (double)(min(j + b2, T - 1) - max(j - a2, 0) + 1);
+  }
+  double m = __builtin_nan("");
+  for (; tile < ntile; tile += nwg) {
+    const size_t px = tile * P + i;
+    const bool in = px < npix;
+    double a = 0.0;
+    tile_store(regs, Yt, T, in, [&](int j, float x) { a = fma((double)x, td[j], a); });
+    red[tid] = a;
+    __syncthreads();
+    if (tile + nwg < ntile) regs.load(g.Y, npix, T, tile + nwg);
+    if (tid < P) {
+      double r = red[tid];
+#pragma unroll
+      for (int k = 1; k < G; ++k) r += red[tid + k * P];
+      r /= mx;
+      vs[tid] = r;
+      if (in) g.s[px] = r;
+    }
+    double A = 0.0, B = 0.0;
+    if constexpr (MODE == kTileLast) {
+      run_sums<P>(Yt, runs, T);
+      __syncthreads();
+      const float* y = Yt + i;
+      float* d = Dt + i;
+      for (int j0 = q * kRun; j0 < T; j0 += G * kRun) {
+        double S = window_sum<P>(y, runs + i, max(j0 - a1, 0), min(j0 + b1, T - 1));
+        const float* yc = y + j0 * LD;
+        if (j0 >= a1 && j0 + kRun + b1 < T) {  // every window of the run is whole
+          float c[kRun], n[kRun], o[kRun];
+#pragma unroll
+          for (int k = 0; k < kRun; ++k) {
+            c[k] = yc[k * LD];
+            n[k] = yc[(k + b1 + 1) * LD];
+            o[k] = yc[(k - a1) * LD];
+          }
+#pragma unroll
+          for (int k = 0; k < kRun; ++k) {
+            d[(j0 + k) * LD] = (float)(((double)c[k] - S * rk1[j0 + k]) * minv);
+            S += (double)n[k];
+            S -= (double)o[k];
+          }
+        } else {
+          for (int j = j0; j < min(j0 + kRun, T); ++j) {
+            d[j * LD] = (float)(((double)y[j * LD] - S * rk1[j]) * minv);
+            if (j + b1 + 1 <= T - 1) S += (double)y[(j + b1 + 1) * LD];
+            if (j - a1 >= 0) S -= (double)y[(j - a1) * LD];
+          }
+        }
+      }
+      __syncthreads();
+      run_sums<P>(Dt, runs, T);
+      __syncthreads();
+      for (int j0 = q * kRun; j0 < T; j0 += G * kRun) {
+        double S = window_sum<P>(d, runs + i, max(j0 - a2, 0), min(j0 + b2, T - 1));
+        auto add = [&](double sm) {
+          double v = 1.0;
+          for (int n = 0; n < g.p; ++n) v *= sm;
+          A = fma(v, v, A);
+          B += v;
+        };
+        const float* dc = d + j0 * LD;
+        if (j0 >= a2 && j0 + kRun + b2 < T) {
+          float n[kRun], o[kRun];
+#pragma unroll
+          for (int k = 0; k < kRun; ++k) {
+            n[k] = dc[(k + b2 + 1) * LD];
+            o[k] = dc[(k - a2) * LD];
+          }
+#pragma unroll
+          for (int k = 0; k < kRun; ++k) {
+            add(S * rk2[j0 + k]);
+            S += (double)n[k];
+            S -= (double)o[k];
+          }
+        } else {
+          for (int j = j0; j < min(j0 + kRun, T); ++j) {
+            add(S * rk2[j]);
+            if (j + b2 + 1 <= T - 1) S += (double)d[(j + b2 + 1) * LD];
+            if (j - a2 >= 0) S -= (double)d[(j - a2) * LD];
+          }
+        }
+      }
+    } else {
+      __syncthreads();
+      for (int j = q; j < T; j += G) {
+        const double x = (double)Yt[j * LD + i] / mx;
+        A = fma(x, x, A);
+        B += x;
+      }
+    }
+    red[tid] = A;
+    red[NT + tid] = B;
+    __syncthreads();
+    if (tid < P && in) {
+      for (int k = 1; k < G; ++k) {
+        A += red[tid + k * P];
+        B += red[NT + tid + k * P];
+      }
+      const double mean = B / (double)T;
+      double r;
+      if constexpr (MODE == kTileLast) {
+        r = sqrt(A / (double)T - mean * mean);
+      } else {
+        const double y1 = vs[tid];
+        r = sqrt((A - y1 * y1) / (double)T - mean * mean + 2.0 * mean * y1 * tc - y1 * y1 * (tc * tc));
+      }
+      g.img[px] = r;
+      m = nmax(m, r);
+    }
+    __syncthreads();  // the tiles, red and vs are rewritten
+  }
+  m = tile_reduce(m, red, true);
+  if (tid == 0) g.parts[blockIdx.x] = m;
+}
+
+typedef void (*TileKernel)(TileArgs);
+
+// Pixels per tile of a movie of T frames: the widest rows that fit LDS (0: no
+// tile does, the movie goes through the passes above).
+int tile_pixels(size_t npix, int T, int mode) {
+  if (npix >= (size_t)1 << 28) return 0;  // 32-bit byte offsets within four rows
+  for (int P : {64, 32, 16})
+    if (!(P == 64 && mode >= kTileLast) && !(P == 16 && mode <= kTileRound) && tile_lds(P, T, mode) <= kTileLds)
+      return P;
+  return 0;
+}
+bool tiled(size_t npix, int T) { return tile_pixels(npix, T, kTileRound) && tile_pixels(npix, T, kTileLast); }
+
+template <int P>
+TileKernel pick_round(int T, int mode) {
+  const bool small = T <= 16 * (kTileThreads / P);
+  if (mode == kTileFirst) return small ? &k_summary_round<P, 16, kTileFirst> : &k_summary_round<P, 40, kTileFirst>;
+  return small ? &k_summary_round<P, 16, kTileRound> : &k_summary_round<P, 40, kTileRound>;
+}
+template <int P>
+TileKernel pick_last(int mode) {
+  return mode == kTileLast ? &k_summary_last<P, 16, kTileLast> : &k_summary_last<P, 16, kTileLastGlobal>;
+}
+
+constexpr int kTileWgs = 1024;  // most workgroups of a pass
+
+hipError_t launch_tile(const TileArgs& g, int mode, int cus, int* nwg, hipStream_t st) {
+  const int P = tile_pixels(g.npix, g.T, mode);
+  const size_t lds = tile_lds(P, g.T, mode);
+  const TileKernel fn = mode <= kTileRound ? (P == 64 ? pick_round<64>(g.T, mode) : pick_round<32>(g.T, mode))
+                                           : (P == 32 ? pick_last<32>(mode) : pick_last<16>(mode));
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTileLds);
+  if (e != hipSuccess) return e;
+  const size_t ntile = (g.npix + P - 1) / P;
+  const size_t per_cu = std::min<size_t>(kTileLds / lds, 2);
+  *nwg = (int)std::min<size_t>(ntile, std::min<size_t>(kTileWgs, per_cu * cus));
+  if (*nwg > 8) *nwg = *nwg / 8 * 8;
+  hipLaunchKernelGGL(fn, dim3(*nwg), dim3(kTileThreads), lds, st, g);
+  return hipGetLastError();
+}
+
 inline unsigned blocks_for(size_t n) { return (unsigned)((n + kThreads - 1) / kThreads); }
 
 }  // namespace
@@ -367,13 +788,40 @@ inline unsigned blocks_for(size_t n) { return (unsigned)((n + kThreads - 1) / kT
 size_t summary_scratch_doubles(size_t npix, int T) {
   const size_t nchunk = (npix + kChunk - 1) / kChunk;
   const size_t nblk = (npix + kThreads - 1) / kThreads;
+  if (tiled(npix, T)) return 2 + 2 * (size_t)T + (size_t)T * kTileWgs + kTileWgs;
   // mx, norm, t[T], tdot parts[T * nchunk], per-block parts[max(nblk, 1024)]
   return 2 + (size_t)T + (size_t)T * nchunk + (nblk > 1024 ? nblk : 1024);
 }
 
+bool summary_needs_movie(size_t npix, int T) { return !tiled(npix, T); }
+
+static hipError_t launch_summary_tiled(const float* Y, size_t npix, int T, int w1, int w2, int p, int bg_iter,
+                                       int global, double* scratch, double* img, double* s, int cus,
+                                       hipStream_t st) {
+  double* mx = scratch;
+  double* nrm = scratch + 1;
+  double* t = scratch + 2;   // the result (summary_temporal)
+  double* tt = t + T;        // unscaled
+  TileArgs g{Y, npix, T, mx, tt, tt + T, tt + T + (size_t)T * kTileWgs, s, img, t, w1, w2, p};
+  int nwg = 0;
+  for (int it = 0; it < bg_iter; ++it) {
+    const hipError_t e = launch_tile(g, it == 0 ? kTileFirst : kTileRound, cus, &nwg, st);
+    if (e != hipSuccess) return e;
+    if (it == 0) hipLaunchKernelGGL(k_fold_max, dim3(1), dim3(kThreads), 0, st, g.parts, nwg, mx);
+    hipLaunchKernelGGL(k_r1_tsum, dim3(T), dim3(kThreads), 0, st, g.tparts, nwg, T, mx, tt);
+  }
+  const hipError_t e = launch_tile(g, global ? kTileLastGlobal : kTileLast, cus, &nwg, st);
+  if (e != hipSuccess) return e;
+  const unsigned nblk = blocks_for(npix);
+  hipLaunchKernelGGL(k_fold_max, dim3(1), dim3(kThreads), 0, st, g.parts, nwg, nrm);
+  hipLaunchKernelGGL(k_scale_div, dim3(nblk < 65535 ? nblk : 65535), dim3(kThreads), 0, st, img, npix, nrm);
+  return hipGetLastError();
+}
+
 hipError_t launch_summary(const float* Y, size_t npix, int T, int w1, int w2, int p, int bg_iter,
-                          int global, double* scratch, float* dbuf, double* img, double* s,
+                          int global, double* scratch, float* dbuf, double* img, double* s, int cus,
                           hipStream_t st) {
+  if (tiled(npix, T)) return launch_summary_tiled(Y, npix, T, w1, w2, p, bg_iter, global, scratch, img, s, cus, st);
   const size_t nchunk = (npix + kChunk - 1) / kChunk;
   const unsigned nblk = blocks_for(npix);
   double* mx = scratch;
