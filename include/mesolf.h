@@ -231,7 +231,8 @@ mlf_status mlf_batch_last_run_ms(mlf_batch b, double* ms);
  * the backprojection's 16-phase tiles per phase group (5 or 3, and 4 for
  * BF16: 3, 5 or 4 groups of 80, 48 or 64 phases cover the 225 phases) and its
  * phase groups per work entry (0: all groups
- * of a lenslet tile in one entry, which builds the tile's ratio window once;
+ * of a lenslet tile in one entry, which builds the tile's ratio window once,
+ * or fewer where the grid has too few tiles to fill the card;
  * 1: one group per entry).
  * Autotuning times every shape on `views` view steps of the patch (or of all
  * patches of the batch, in its shared launches), restores the volumes, and

@@ -38,6 +38,7 @@ struct mlf_batch_s {
   int cus = 0;
   size_t smem_f = 0, smem_b = 0;
   int fwd_nbuf = 2;
+  int bwd_gpe = 1;  // phase groups per backprojection entry (backward_split)
   // one RL iteration's view loop as a graph
   bool use_graph = true;
   hipGraph_t graph = nullptr;
@@ -87,16 +88,25 @@ mlf_status rebuild(mlf_batch_s* b) {
   };
   std::vector<Ent> fe, be;
   std::vector<int32_t> rs;
+  // the groups of a lenslet tile are split over entries by the batch's tile count
+  const int ngrp = kPhiPadBwd / (16 * std::max(1, b->bwd_nt));
+  int tiles = 0;
+  for (const mlf_patch_s* p : b->slots) tiles += (int)(p->bent.size() / 4) * p->bwd_gpe / ngrp;
+  const int gpe = backward_split(tiles, ngrp, bwd_groups_per_entry(b->bwd_nt, b->bwd_grp));
+  if (gpe != b->bwd_gpe) drop_graph(b);
+  b->bwd_gpe = gpe;
   for (size_t i = 0; i < b->slots.size(); ++i) {
     mlf_patch_s* p = b->slots[i];
     sd.push_back(p->slot);
-    for (size_t e = 0; e + 3 <= p->fent.size(); e += 3) {
+    for (size_t e = 0; e + 4 <= p->fent.size(); e += 4) {
       const int z = p->fent[e];
-      fe.push_back(Ent{ps->rf[z], {(int32_t)i, z, p->fent[e + 1], p->fent[e + 2], 0}});
+      fe.push_back(Ent{ps->rf[z], {(int32_t)i, z, p->fent[e + 1], p->fent[e + 2], p->fent[e + 3]}});
     }
     for (size_t e = 0; e + 4 <= p->bent.size(); e += 4) {
       const int z = p->bent[e];
-      be.push_back(Ent{ps->rb[z], {(int32_t)i, z, p->bent[e + 1], p->bent[e + 2], p->bent[e + 3]}});
+      if (p->bent[e + 3] != 0) continue;  // one visit per tile
+      for (int gq = 0; gq < ngrp; gq += gpe)
+        be.push_back(Ent{ps->rb[z], {(int32_t)i, z, p->bent[e + 1], p->bent[e + 2], gq}});
     }
     for (int j = 0; j < p->nblk_r; ++j) {
       rs.push_back((int32_t)i);
@@ -108,16 +118,15 @@ mlf_status rebuild(mlf_batch_s* b) {
   std::stable_sort(be.begin(), be.end(), by_r);
   std::vector<int32_t> fs, bs;
   std::vector<int> fg, bg;  // XCD groups: (slot, plane) and (slot, plane, phase group)
-  const int ngrp = kPhiPadBwd / (16 * std::max(1, b->bwd_nt));  // XCD groups: entries start at a phase group
   for (const Ent& e : fe) {
-    fs.insert(fs.end(), e.v, e.v + 4);
+    fs.insert(fs.end(), e.v, e.v + 5);
     fg.push_back(e.v[0] * ps->Z + e.v[1]);
   }
   for (const Ent& e : be) {
     bs.insert(bs.end(), e.v, e.v + 5);
     bg.push_back((e.v[0] * ps->Z + e.v[1]) * ngrp + e.v[4]);
   }
-  xcd_interleave(fs, 4, fg);
+  xcd_interleave(fs, 5, fg);
   xcd_interleave(bs, 5, bg);
   b->n_f = (int)fe.size();
   b->n_b = (int)be.size();
@@ -155,7 +164,7 @@ mlf_status enqueue_views(mlf_batch_s* b, hipStream_t st, int nviews = 0) {
       MLF_LAUNCH(launch_ratio_gather(g, rg, b->grid_r, ps->Z, b->bm2, u, v, 1, nullptr, st));
     }
     const BwdGeo bg{b->d_slots.ptr, ps->d_rb.ptr, pk.d_boff.ptr, pk.d_epad.ptr, b->d_bsched.ptr,
-                    b->d_counts.ptr + 1, k, bwd_groups_per_entry(b->bwd_nt, b->bwd_grp)};
+                    b->d_counts.ptr + 1, k, b->bwd_gpe};
     // every slot of a BF16 Toeplitz batch holds its volume in the split form
     const bool split = b->tpz && b->kp == Precision::kBF16;
     MLF_LAUNCH(launch_bwd_mfma(b->kp, b->bwd_nt, b->bwd_occ, split, pk.bwd.ptr + (size_t)k * pk.pvb * eb, bg,

@@ -85,6 +85,7 @@ struct SlotDesc {
   const int32_t* C1;      // [Z] normaliser classes along axis 0
   int n1, n2;
   float xs, xs_inv;       // FP16 shadow scale (1 otherwise)
+  int fparts;             // Toeplitz forward: runs of e1 per block, each with its own partial windows
 };
 
 // Work entries are processed by a grid-stride loop over *count entries, so a
@@ -95,7 +96,7 @@ struct FwdGeo {
   const int32_t* r;       // [Z] forward radius
   const int64_t* woff;    // [Z] element offset of the plane block in the packed view
   const int32_t* nchunk;  // [Z] number of 64-tap chunks (Q-scatter kernel)
-  const int32_t* sched;   // [entries][4] = (slot, z, b1, b2)
+  const int32_t* sched;   // [entries][5] = (slot, z, b1, b2, run of e1)
   const int32_t* count;   // number of entries
   const float* finv;      // FP16: [Z] inverse PSF scale of the view (null otherwise)
   const int32_t* tap_inf; // FP32 Toeplitz: not 0 if a tap of the PSF is infinite

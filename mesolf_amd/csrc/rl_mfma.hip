@@ -158,6 +158,7 @@ __device__ __forceinline__ SlotDesc load_slot(const SlotDesc* slots, int i) {
   o.n2 = uni(cload(&d->n2));
   o.xs = __builtin_bit_cast(float, uni(__builtin_bit_cast(int, cload(&d->xs))));
   o.xs_inv = __builtin_bit_cast(float, uni(__builtin_bit_cast(int, cload(&d->xs_inv))));
+  o.fparts = uni(cload(&d->fparts));
   return o;
 }
 // s_waitcnt vmcnt(<= n) without waiting on LDS/export counters (gfx9 encoding:
@@ -210,7 +211,7 @@ void k_fwd_mfma(const T* __restrict__ W, FwdGeo g) {
 
   const int nent = uni(cload(g.count));
   for (int ent = blockIdx.x; ent < nent; ent += gridDim.x) {
-    const int* s = g.sched + 4 * ent;
+    const int* s = g.sched + 5 * ent;
     const SlotDesc sd = load_slot(g.slots, uni(cload(s)));
     const float* __restrict__ X = sd.X;
     const int n1 = sd.n1, n2 = sd.n2;
@@ -352,47 +353,50 @@ void k_fwd_mfma(const T* __restrict__ W, FwdGeo g) {
 // input column c2 (one M-tile per c2), N = e2 (16 * ceil(K/16)), K = (e1, phase).
 // The A operand is a register window over i1: stepping e1 shifts it by one
 // lane (DPP row_shr:1 within each 16-lane row) and lane 0 takes the next
-// lenslet from an LDS ring filled by direct-to-LDS loads.  The B operand (one
-// e1 column of taps) is copied global -> LDS while the previous column's
-// MFMAs run.  The sum over e1 happens inside the MFMA accumulators, so only
+// lenslet from a ring in LDS.  The B operand (one e1 column of taps) is stored
+// as ready fragments, [e1][N-tile][K-step][lane][8].  Both are copied global ->
+// LDS by buffer loads, spread over a step's MFMAs, kTpzDepth(NT) - 1 steps ahead:
+// narrow planes have little matrix work per step, and with one step ahead
+// their steps waited for the copies (NT = 1: 4 columns of 8 KB in flight, NT = 3: 2
+// of 24 KB).  Per view, against row-major taps copied by FLAT loads one step
+// ahead: 101 x 101 x 51 BF16 227 -> 207 us, 81 x 73 x 31 FP16 68.5 -> 61.7 us,
+// 33 x 33 x 11 BF16 19.0 -> 16.7 us, the same bits.  The sum over e1 happens inside the MFMA accumulators, so only
 // the final P tile is scattered, once per entry, by in-register diagonal sums
 // and plain LDS stores.
 constexpr int kTpzNT = 3;      // N-tiles (taps along axis 1): K <= 48, i.e. r <= 23
-// W/ring buffers: the DMA runs one step ahead (two buffers keep the kernel at
-// 75 KB of LDS, two workgroups per CU, which measured 1.9x faster than three
-// buffers at one workgroup per CU).
-constexpr int kTpzBufs = 2;
-constexpr int kRingRow = 256;  // elements per lenslet row of the injection ring (phases >= 225 stay 0)
+constexpr int kFrag = 1024;    // bytes of one 16 x 32 16-bit fragment of a wave
+constexpr int kTpzKS = kPhiPadBF16 / 32;  // K-steps per column
+inline __host__ __device__ constexpr int tpz_depth(int nt) { return nt == 1 ? 4 : nt == 2 ? 3 : 2; }
+inline __host__ __device__ constexpr int tpz_step_bytes(int nt, int mt) {
+  return nt * kTpzKS * kFrag + 4 * mt * kShadowRow * 2;
+}
+// LDS: the widest of the tap and lenslet rings over the tile counts (the flush's windows reuse it)
+inline __host__ __device__ constexpr int tpz_lds(int mt) {
+  int b = 0;
+  for (int nt = 1; nt <= kTpzNT; ++nt)
+    b = b > tpz_depth(nt) * tpz_step_bytes(nt, mt) ? b : tpz_depth(nt) * tpz_step_bytes(nt, mt);
+  return b;
+}
 
 template <typename T, int MT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void k_fwd_tpz(const T* __restrict__ W, FwdGeo g) {
   using M = Mma<T>;
-  constexpr int KSTEP = M::KSTEP, KPL = M::KPL, PHI = M::PHI;
-  constexpr int NKS = PHI / KSTEP;
+  using frag_t = typename M::frag;
+  typedef int intx4 __attribute__((ext_vector_type(4)));
+  constexpr int NKS = kTpzKS;
   constexpr int CW = 4 * MT;  // input columns c2 per workgroup
-  constexpr int VEC = 16 / sizeof(T);
-  constexpr int RV = PHI / VEC;
-  constexpr bool SWZ = (RV == 32);
-  constexpr int NB = kTpzBufs;
-  constexpr int WSLOT = ((16 * kTpzNT * RV + 255) / 256) * 256;  // 16-byte slots per W buffer
   extern __shared__ __align__(16) char smem[];
-  T* Wb = reinterpret_cast<T*>(smem);                                        // [NB][WSLOT*VEC]
-  // injection ring: shadow rows, kRingRow elements each
-  T* ring = reinterpret_cast<T*>(smem + (size_t)NB * WSLOT * 16);            // [NB][CW][kRingRow]
-  float* ywin = reinterpret_cast<float*>(ring + NB * CW * kRingRow);         // [4 waves][16][MT + 2r]
 
   const int nent = uni(cload(g.count));
   for (int ent = blockIdx.x; ent < nent; ent += gridDim.x) {
-    const int* s = g.sched + 4 * ent;
+    const int* s = g.sched + 5 * ent;
     const SlotDesc sd = load_slot(g.slots, uni(cload(s)));
-    const T* __restrict__ Xb = reinterpret_cast<const T*>(sd.Xb);
     const int n1 = sd.n1, n2 = sd.n2;
     const int z = uni(cload(s + 1)), b1 = uni(cload(s + 2)), b2 = uni(cload(s + 3));
     const int r = uni(cload(g.r + z));
     const int K = 2 * r + 1;
-    const int NT = (K + 15) / 16;
-    const int nrow = 16 * NT;
+    const int NTr = (K + 15) / 16;
     const int WW = MT + 2 * r;
     // w: wave index, wave-uniform (readfirstlane), so loops and bases over it run on the scalar unit
     const int tid = threadIdx.x, lane = tid & 63, w = uni(tid >> 6), lr = lane & 15, lg = lane >> 4;
@@ -403,169 +407,114 @@ void k_fwd_tpz(const T* __restrict__ W, FwdGeo g) {
         sd.partial + uni64(cload(sd.poff + z)) + (size_t)(b2 * ceil_div(n1, 16) + b1) * 16 * (CW + 2 * r);
     float unscale = 1.f;
     if constexpr (is_f16<T>()) unscale = cload(g.finv + z) * sd.xs_inv;
-    const T* Xbz = Xb + (size_t)z * n2 * n1 * kShadowRow;  // shadow plane
-    // the shadow plane as a buffer (a plane is below 2^31 bytes, checked at patch creation)
-    const __amdgpu_buffer_rsrc_t shr = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<T*>(Xbz), 0, (int)((size_t)n2 * n1 * kShadowRow * sizeof(T)), kBufferDword3);
-    float* yw = ywin + w * 16 * WW;  // every cell is written by the flush
-    for (int o = tid; o < NB * CW * kRingRow; o += 256) ring[o] = (T)0.f;  // pads stay zero
+    // the shadow plane (below 2^31 bytes, checked at patch creation) and the
+    // plane's taps as buffers: reads past the end return zeros
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+        reinterpret_cast<T*>(sd.Xb) + (size_t)z * n2 * n1 * kShadowRow, 0,
+        (int)((size_t)n2 * n1 * kShadowRow * sizeof(T)), kBufferDword3);
+    const int col_bytes = NTr * NKS * kFrag;
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<T*>(W + uni64(cload(g.woff + z))), 0, K * col_bytes, kBufferDword3);
+    const unsigned tap_lane = 16 * lane;
 
-    // A operand at e1 = 0 (d1 = -r): lane row lr holds lenslet i1 = 16*b1 + lr + r
-    typename M::frag a[MT][NKS];
-  #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int c2 = c2_0 + MT * w + mt;
-      const int i1 = 16 * b1 + lr + r;
-      const bool ok = c2 < n2 && i1 < n1;
-      const size_t lens = ((size_t)z * n2 + (ok ? c2 : 0)) * n1 + (ok ? i1 : 0);
-  #pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) {
-        // shadow rows are 256 phases (zero beyond 225), 16-byte aligned
-        const typename M::frag v =
-            gload(reinterpret_cast<const typename M::frag*>(Xb + lens * kShadowRow + ks * KSTEP + lg * KPL));
-        a[mt][ks] = ok ? v : typename M::frag{};
-      }
-    }
-    __syncthreads();  // ring zeroed before any DMA lands
-
-    const T* Wz = W + uni64(cload(g.woff + z));  // [K][nrow][PHI]
-    // Only the K tap rows e2 < K are copied: rows K..16*NT-1 of the buffer feed
-    // accumulator columns that the flush drops, so whatever they hold does not
-    // matter.
-    const int nslot = K * RV;
-    const int nw_inst = (nslot + 255) / 256;
-    // Copy addresses: a wave-uniform (scalar) base plus the lane's 32-bit byte
-    // offset, which for the W copies does not depend on the step and is
-    // computed once per entry.
-    constexpr int kWInst = (16 * kTpzNT * RV + 255) / 256;  // copies per wave for the widest plane
-    int woff[kWInst];
-  #pragma unroll
-    for (int i = 0; i < kWInst; ++i) {
-      const int slot = min(256 * i + 64 * w + lane, nslot - 1);  // tail slots re-read the last vector
-      const int row = (unsigned)slot / RV, pos = (unsigned)slot % RV;
-      const int col = SWZ ? (pos ^ (row & 31)) : pos;
-      woff[i] = (row * PHI + col * VEC) * (int)sizeof(T);
-    }
-    auto issue_w = [&](int t, int buf) {
-      const char* src = reinterpret_cast<const char*>(Wz + (size_t)t * nrow * PHI);
-      char* dst = reinterpret_cast<char*>(Wb) + (size_t)buf * WSLOT * 16;
-  #pragma unroll
-      for (int i = 0; i < kWInst; ++i) {
-        if (i >= nw_inst) break;
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + woff[i]),
-                                         (__attribute__((address_space(3))) void*)(dst + (256 * i + 64 * w) * 16),
-                                         16, 0, 0);
-      }
-    };
-    constexpr int RPASS = 2;  // passes of 64 dwords per 512-byte shadow row
+    frag_t a[MT][NKS];
     floatx4 acc[MT][kTpzNT];
   #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
   #pragma unroll
       for (int nt = 0; nt < kTpzNT; ++nt) acc[mt][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    // batch t = W column t and, for t >= 1, injection row t (i1 = 16 b1 + r - t)
-    issue_w(0, 0);
-    wait_vm<0>();  // batch 0 landed
-    __syncthreads();
-    // The copies of batch t + 1 are spread over tile 0's K-steps
-    // (one injection copy and at most one W copy per K-step, no branches), so
-    // the eight waves of a CU do not queue their copies at the address unit
-    // all at once.  The last step re-copies the last column and a row past the
-    // grid (zeros) into the free buffer, which nothing reads.
-    constexpr int kInj = CW * RPASS / 4;  // injection copies per wave and step
-    static_assert(kInj <= NKS && kWInst <= NKS, "one copy of each kind per K-step");
-    for (int t = 0; t < K; ++t) {
-      const int tn = min(t + NB - 1, K - 1), bn = (t + NB - 1) % NB;
-      const char* w_src = reinterpret_cast<const char*>(Wz + (size_t)tn * nrow * PHI);
-      char* w_dst = reinterpret_cast<char*>(Wb) + (size_t)bn * WSLOT * 16;
-      const int i1r_n = 16 * b1 + r - tn;
-      const bool rowok_n = i1r_n >= 0 && i1r_n < n1;
-      const int i1_n = min(max(i1r_n, 0), n1 - 1);
-      char* inj_dst = reinterpret_cast<char*>(ring + bn * CW * kRingRow);
-      auto issue_piece = [&](int k) __attribute__((always_inline)) {
-        if (k < kWInst)
-          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(w_src + woff[k]),
-                                           (__attribute__((address_space(3))) void*)(w_dst + (256 * k + 64 * w) * 16),
-                                           16, 0, 0);
-        if (k < kInj) {
-          // rows outside the grid: an offset past the plane, which the
-          // buffer load returns as zeros (no branch, no zero-row pointer)
-          const int q = w + 4 * k, c = q / RPASS, part = q - c * RPASS;
-          const bool ok = rowok_n && c2_0 + c < n2;
-          const int c2 = min(c2_0 + c, n2 - 1);
-          const unsigned voff = ok ? (unsigned)(((c2 * n1 + i1_n) * kShadowRow + part * 128) * 2) + 4u * lane
-                                   : 0x80000000u;
+    auto walk = [&](auto ntc) __attribute__((always_inline)) {
+      constexpr int NT = decltype(ntc)::value, D = tpz_depth(NT);
+      constexpr int kW = NT * NKS * kFrag;                 // a column's taps
+      constexpr int kRow = kShadowRow * (int)sizeof(T);     // a lenslet's row
+      constexpr int kPiecesW = NT * NKS / 4, kPiecesX = MT / 2;  // copies per wave and step
+      char* const ring = smem + D * kW + w * D * MT * kRow;  // [D][MT][row] of this wave
+      // piece q of step t's copies: taps (fragment 4 q + w), then two lenslet rows
+      auto issue = [&](int t, int q) __attribute__((always_inline)) {
+        if (q < kPiecesW) {
+          // tap rows e2 >= K of the last tile stay zero without being read
+          const unsigned vo = 16 * ((4 * q) / NKS) + lr < K ? tap_lane : 0x80000000u;
           __builtin_amdgcn_raw_ptr_buffer_load_lds(
-              shr, (__attribute__((address_space(3))) void*)(inj_dst + (c * kRingRow) * (int)sizeof(T) + 4 * part * 64),
-              4, voff, 0, 0, 0);
-        }
-      };
-      const T* Wc = Wb + (size_t)(t % NB) * WSLOT * VEC;
-      auto load_b = [&](int ks, int nt) {
-        const int row = nt * 16 + lr;
-        if constexpr (SWZ) {
-          const int col = (ks * KSTEP + lg * KPL) / VEC;
-          return M::load(Wc + row * PHI + ((col ^ (row & 31)) * VEC));
+              wr, (__attribute__((address_space(3))) void*)(smem + (t % D) * kW + (4 * q + w) * kFrag), 16, vo,
+              t * kW + (4 * q + w) * kFrag, 0, 0);
         } else {
-          return M::load(Wc + row * PHI + ks * KSTEP + lg * KPL);
+          // the lenslets that enter at step t: i1 = 16 b1 + r - t, columns 2 k, 2 k + 1 of the wave
+          const int k = q - kPiecesW, i1 = 16 * b1 + r - t, c2 = c2_0 + MT * w + 2 * k + (lane >> 5);
+          const unsigned vo = i1 >= 0 && i1 < n1 && c2 < n2
+                                  ? (unsigned)((c2 * n1 + i1) * kRow + 16 * (lane & 31)) : 0x80000000u;
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(
+              xr, (__attribute__((address_space(3))) void*)(ring + ((t % D) * MT + 2 * k) * kRow), 16, vo, 0, 0, 0);
         }
       };
-      // N-tile outer, K-step inner: each tile's loads and MFMAs are
-      // straight-line code, and the tile count is tested twice per step
-      // rather than once per group of MFMAs (a branch makes the MFMAs after
-      // it wait for every LDS read issued before it)
-      // B fragments are read two K-steps ahead (crossing into the next
-      // N-tile's first steps), so their LDS latency hides behind the MFMAs of
-      // the two steps before; reading a tile that the plane does not use is
-      // harmless (the buffer holds kTpzNT tiles).
-      auto load_seq = [&](int q) {  // q-th step of the tile sequence
-        return load_b(q % NKS, min(q / NKS, kTpzNT - 1));
-      };
-      typename M::frag bq0 = load_seq(0), bq1 = load_seq(1);
-      auto tile = [&](auto ntc) __attribute__((always_inline)) {
-        constexpr int nt = decltype(ntc)::value;
+      constexpr int kPieces = kPiecesW + kPiecesX;
+      static_assert(kPieces <= NT * NKS, "at most one copy per K-step");
   #pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) {
-          const typename M::frag bf = bq0;
-          bq0 = bq1;
-          bq1 = load_seq(nt * NKS + ks + 2);
+      for (int t = 0; t < D - 1; ++t)
+        if (t < K)
   #pragma unroll
-          for (int mt = 0; mt < MT; ++mt) acc[mt][nt] = M::mma(a[mt][ks], bf, acc[mt][nt]);
-          if constexpr (nt == 0) issue_piece(ks);
-        }
-      };
-      static_assert(kTpzNT == 3, "three N-tiles");
-      tile(std::integral_constant<int, 0>{});
-      if (NT > 1) tile(std::integral_constant<int, 1>{});
-      if (NT > 2) tile(std::integral_constant<int, 2>{});
-      wait_vm<0>();  // batch t + 1 landed
-      __syncthreads();
-      if (t + 1 < K) {
-        const T* rg = ring + ((t + 1) % NB) * CW * kRingRow;
+          for (int q = 0; q < kPieces; ++q) issue(t, q);
+      // A operand at e1 = 0 (d1 = -r): lane row lr holds lenslet i1 = 16*b1 + lr + r
   #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          const int c = MT * w + mt;
-          // shift every 16-lane row down by one lane, then lane 0 of each row
-          // alone reads the entering lenslet from the ring (the other lanes'
-          // LDS reads would return data nobody keeps); rows outside the grid
-          // arrived as zeros
+      for (int mt = 0; mt < MT; ++mt) {
+        const int c2 = c2_0 + MT * w + mt, i1 = 16 * b1 + lr + r;
+        const unsigned o = c2 < n2 && i1 < n1 ? (unsigned)((c2 * n1 + i1) * kRow + 16 * lg) : 0x80000000u;
+  #pragma unroll
+        for (int ks = 0; ks < NKS; ++ks)
+          a[mt][ks] = __builtin_bit_cast(frag_t, __builtin_amdgcn_raw_buffer_load_b128(xr, o, 64 * ks, 0));
+      }
+      wait_vm<0>();
+      lds_barrier();
+      for (int t = 0; t < K; ++t) {
+        const bool more = t + D - 1 < K;
+        const char* Wc = smem + (t % D) * kW + 16 * lane;
+        auto load_b = [&](int q) { return *reinterpret_cast<const frag_t*>(Wc + q * kFrag); };
+        // N-tile outer, K-step inner; B fragments are read two K-steps ahead,
+        // so their LDS latency hides behind the MFMAs of the two steps before
+        frag_t bq0 = load_b(0), bq1 = load_b(1);
+  #pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
   #pragma unroll
           for (int ks = 0; ks < NKS; ++ks) {
-            typedef int intx4 __attribute__((ext_vector_type(4)));
-            intx4 cv = __builtin_bit_cast(intx4, a[mt][ks]);
+            const int q = nt * NKS + ks;
+            const frag_t bf = bq0;
+            bq0 = bq1;
+            bq1 = load_b(q + 2 < NT * NKS ? q + 2 : NT * NKS - 1);
   #pragma unroll
-            for (int q = 0; q < 4; ++q) cv[q] = __builtin_amdgcn_mov_dpp(cv[q], 0x111, 0xF, 0xF, true);
-            a[mt][ks] = __builtin_bit_cast(typename M::frag, cv);
+            for (int mt = 0; mt < MT; ++mt) acc[mt][nt] = M::mma(a[mt][ks], bf, acc[mt][nt]);
+            if (q < kPieces && more) issue(t + D - 1, q);
           }
-          if (lr == 0) {
-            const T* rp = rg + c * kRingRow + lg * KPL;
+        // the next step's copies have landed; those of the D - 2 steps after it
+        // may still be in flight (all that are left, near the end)
+        if (D == 2 || !more) wait_vm<0>();
+        else wait_vm<(D - 2) * kPieces>();
+        lds_barrier();  // ... every wave's, and every wave is done with this step's
+        if (t + 1 < K) {
+          const char* rg = ring + ((t + 1) % D) * MT * kRow + 16 * lg;
   #pragma unroll
-            for (int ks = 0; ks < NKS; ++ks) a[mt][ks] = *reinterpret_cast<const typename M::frag*>(rp + ks * KSTEP);
+          for (int mt = 0; mt < MT; ++mt) {
+            // shift every 16-lane row down by one lane, then lane 0 of each row
+            // alone reads the entering lenslet from the ring (the other lanes'
+            // LDS reads would return data nobody keeps)
+  #pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) {
+              intx4 cv = __builtin_bit_cast(intx4, a[mt][ks]);
+  #pragma unroll
+              for (int q = 0; q < 4; ++q) cv[q] = __builtin_amdgcn_mov_dpp(cv[q], 0x111, 0xF, 0xF, true);
+              a[mt][ks] = __builtin_bit_cast(frag_t, cv);
+            }
+            if (lr == 0) {
+  #pragma unroll
+              for (int ks = 0; ks < NKS; ++ks) a[mt][ks] = *reinterpret_cast<const frag_t*>(rg + mt * kRow + 64 * ks);
+            }
           }
         }
       }
-    }
+    };
+    static_assert(kTpzNT == 3, "three N-tiles");
+    if (NTr == 1) walk(std::integral_constant<int, 1>{});
+    else if (NTr == 2) walk(std::integral_constant<int, 2>{});
+    else walk(std::integral_constant<int, 3>{});
 
     // P tiles -> this wave's window: y[i1][mt + e2] = sum_mt P_mt[i1, e2] (rows
     // i1 - 16*b1, columns c2 + d2 - (c2_0 + MT*w - r)).  Lane (lr, lg) holds
@@ -575,21 +524,24 @@ void k_fwd_tpz(const T* __restrict__ W, FwdGeo g) {
     // 16 (nt + 1) + lr and are carried into the next tile.  Columns e2 >= K
     // (padded taps) are zeroed first.  Each window cell then has one writer:
     // plain LDS stores, summed in a fixed order, and no clearing of the window.
+    // The windows reuse the rings (the last barrier has freed them).
     // FP16 undoes the PSF and volume pre-scaling here (one plane per entry).
     static_assert(MT <= 4, "row rotations of up to 3 lanes");
+    float* const ywin = reinterpret_cast<float*>(smem);  // [4 waves][16][MT + 2r]
+    float* const yw = ywin + w * 16 * WW;
     floatx4 carry = {0.f, 0.f, 0.f, 0.f};
   #pragma unroll
     for (int nt = 0; nt <= kTpzNT; ++nt) {
-      if (nt > NT) continue;
+      if (nt > NTr) continue;
       floatx4 col = carry;
       carry = floatx4{0.f, 0.f, 0.f, 0.f};
-      if (nt < kTpzNT && nt < NT) {
+      if (nt < kTpzNT && nt < NTr) {
         const bool ev = nt * 16 + lr < K;
   #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
   #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            const float v = ev ? acc[mt][nt][j] : 0.f;
+            const float v = ev ? acc[mt][nt < kTpzNT ? nt : 0][j] : 0.f;
             const float x = row_ror(v, mt);
             col[j] += lr >= mt ? x : 0.f;
             carry[j] += lr >= mt ? 0.f : x;
@@ -641,8 +593,8 @@ void k_fwd_tpz(const T* __restrict__ W, FwdGeo g) {
 // reads are free of conflicts.
 // Infinities of the volume or the taps would turn into NaN between the parts:
 // an entry that meets one is summed again directly in FP32.
-constexpr int kSplitKS = 4;       // K-steps (32 phases) per half
-constexpr int kSplitFrag = 1024;  // bytes of one fragment of a wave
+constexpr int kSplitKS = 4;  // K-steps (32 phases) per half
+constexpr int kSplitFrag = kFrag;
 
 __device__ __forceinline__ unsigned pack_bf16(float lo, float hi) {
   return (unsigned)__builtin_bit_cast(unsigned short, (__bf16)lo) |
@@ -683,7 +635,7 @@ void k_fwd_tps(const char* __restrict__ W, FwdGeo g) {
   // [MT][part][128 phases].  The flush's windows reuse the tap buffers.
   const int nent = uni(cload(g.count));
   for (int ent = blockIdx.x; ent < nent; ent += gridDim.x) {
-    const int* s = g.sched + 4 * ent;
+    const int* s = g.sched + 5 * ent;
     const SlotDesc sd = load_slot(g.slots, uni(cload(s)));
     const int n1 = sd.n1, n2 = sd.n2;
     const int z = uni(cload(s + 1)), b1 = uni(cload(s + 2)), b2 = uni(cload(s + 3));
@@ -693,8 +645,9 @@ void k_fwd_tps(const char* __restrict__ W, FwdGeo g) {
     const int WW = MT + 2 * r;
     const int tid = threadIdx.x, lane = tid & 63, w = uni(tid >> 6), lr = lane & 15, lg = lane >> 4;
     const int c2_0 = CW * b2;
-    float* const out =
-        sd.partial + uni64(cload(sd.poff + z)) + (size_t)(b2 * ceil_div(n1, 16) + b1) * 16 * (CW + 2 * r);
+    const int part = uni(cload(s + 4)), t0 = part * K / sd.fparts, t1 = (part + 1) * K / sd.fparts;  // run of e1
+    float* const out = sd.partial + uni64(cload(sd.poff + z)) +
+                       (size_t)((part * ceil_div(n2, CW) + b2) * ceil_div(n1, 16) + b1) * 16 * (CW + 2 * r);
     // one plane of the volume and one plane's taps as buffers: reads past the
     // end (lenslets outside the grid, padded tap rows) return zeros
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
@@ -709,8 +662,8 @@ void k_fwd_tps(const char* __restrict__ W, FwdGeo g) {
     auto load_a = [&](int h) {
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
-        const int c2 = c2_0 + MT * w + mt, i1 = 16 * b1 + lr + r;
-        const unsigned o = c2 < n2 && i1 < n1 ? (unsigned)(4 * ((c2 * n1 + i1) * kXRow + 128 * h + 8 * lg))
+        const int c2 = c2_0 + MT * w + mt, i1 = 16 * b1 + lr + r - t0;
+        const unsigned o = c2 < n2 && i1 >= 0 && i1 < n1 ? (unsigned)(4 * ((c2 * n1 + i1) * kXRow + 128 * h + 8 * lg))
                                               : 0x80000000u;
 #pragma unroll
         for (int ks = 0; ks < kSplitKS; ++ks) {
@@ -729,15 +682,19 @@ void k_fwd_tps(const char* __restrict__ W, FwdGeo g) {
         }
       }
     };
-    // piece q of step st's taps: this wave's share of N-tile q / 3
+    // piece q of step st's taps (st = h (t1 - t0) + t - t0): this wave's share of N-tile q / 3
     const unsigned tap_lane = 16 * lane;
+    const int nt1 = t1 - t0;
     auto issue_w = [&](int st, int q) __attribute__((always_inline)) {
+      const int col = st < nt1 ? t0 + st : K + t0 + st - nt1;  // column of [half][e1]
       const unsigned vo = 16 * (q / 3) + lr < K ? tap_lane : 0x80000000u;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           wr, (__attribute__((address_space(3))) void*)(smem + (st & 1) * WBUF + (4 * q + w) * kSplitFrag), 16, vo,
-          st * step_bytes + (4 * q + w) * kSplitFrag, 0, 0);
+          col * step_bytes + (4 * q + w) * kSplitFrag, 0, 0);
     };
-    for (int q = 0; q < 3 * NT; ++q) issue_w(0, q);
+    if (nt1 > 0) {
+      for (int q = 0; q < 3 * NT; ++q) issue_w(0, q);
+    }
     load_a(0);
 
     floatx4 acc[MT][kTpzNT];
@@ -751,10 +708,10 @@ void k_fwd_tps(const char* __restrict__ W, FwdGeo g) {
     // the lenslet that enters column `inj_mt` of this wave: 4 of its phases per lane
     const int inj_mt = MT == 2 ? lane >> 5 : 0, inj_ph = 4 * (lane & 31), inj_c2 = c2_0 + MT * w + inj_mt;
     const bool inj_on = MT == 2 || lane < 32;
-    const int nst = 2 * K;
-    int t = 0, h = 0;  // step st = h K + t
+    const int nst = 2 * nt1;
+    int t = t0, h = 0;
     for (int st = 0; st < nst; ++st) {
-      const bool last_t = t + 1 == K;
+      const bool last_t = t + 1 == t1;
       floatx4 inj = {0.f, 0.f, 0.f, 0.f};
       if (!last_t) {
         const int i1 = 16 * b1 + r - (t + 1);
@@ -811,7 +768,7 @@ void k_fwd_tps(const char* __restrict__ W, FwdGeo g) {
       wait_vm<0>();   // the next step's taps
       lds_barrier();  // ... of every wave, and every wave is done with this step's
       if (last_t) {
-        t = 0;
+        t = t0;
         ++h;
         if (h < 2) load_a(h);
         continue;
@@ -884,7 +841,7 @@ void k_fwd_tps(const char* __restrict__ W, FwdGeo g) {
       } else {
         // y[i][c] = sum over e1, columns and phases of X * taps, FP32
         for (int cc = max(0, c - K + 1); cc < CW && cc <= c; ++cc)
-          for (int e1 = 0; e1 < K; ++e1) {
+          for (int e1 = t0; e1 < t1; ++e1) {
             const int i1 = 16 * b1 + i - (e1 - r), c2 = c2_0 + cc, e2 = c - cc;
             const bool in = i1 >= 0 && i1 < n1 && c2 < n2;
             for (int ph = 0; ph < kP; ++ph) {
@@ -987,7 +944,7 @@ __global__ __launch_bounds__(256) void k_ratio_gather_tpz(FwdGeo g, RatioGeo rg,
     // The slice's planes go in chunks of kZC: the radii and offsets of a chunk
     // are read together, then up to kW windows per plane (all of them for
     // 16-column blocks, r <= 23), and only then summed, in plane then window
-    // order (an unused slot adds +0.0, which changes no sum).  A plane with
+    // order, one run of e1 after the other (an unused slot adds +0.0, which changes no sum).  A plane with
     // more windows (narrower blocks) reads the rest one by one.
     float y = 0.f;
     if (ok) {
@@ -1001,6 +958,7 @@ __global__ __launch_bounds__(256) void k_ratio_gather_tpz(FwdGeo g, RatioGeo rg,
           rr[q] = gload(g.r + zq);
           pz[q] = sd.partial + gload(sd.poff + zq);
         }
+        for (int pt = 0; pt < sd.fparts; ++pt) {
         float vv[kZC][kW];
   #pragma unroll
         for (int q = 0; q < kZC; ++q) {
@@ -1011,7 +969,7 @@ __global__ __launch_bounds__(256) void k_ratio_gather_tpz(FwdGeo g, RatioGeo rg,
           for (int wi = 0; wi < kW; ++wi) {
             const int b2 = b2l + wi;
             const bool use = zc + q < z1 && b2 <= b2h;
-            const size_t idx = use ? (size_t)(b2 * nb1 + b1) * 16 * Wc2 + (i2 - CW * b2 + r) * 16 + (i1 - 16 * b1) : 0;
+            const size_t idx = use ? (size_t)((pt * nb2 + b2) * nb1 + b1) * 16 * Wc2 + (i2 - CW * b2 + r) * 16 + (i1 - 16 * b1) : 0;
             const float t = gload(pz[q] + idx);
             vv[q][wi] = use ? t : 0.f;
           }
@@ -1025,7 +983,8 @@ __global__ __launch_bounds__(256) void k_ratio_gather_tpz(FwdGeo g, RatioGeo rg,
           const int b2h = min(nb2 - 1, (i2 + r) / CW);
           const int b2l = (i2 - r - CW + 1 <= 0) ? 0 : (i2 - r - CW + 1 + CW - 1) / CW;
           for (int b2 = b2l + kW; b2 <= b2h; ++b2)
-            y += gload(pz[q] + (size_t)(b2 * nb1 + b1) * 16 * Wc2 + (i2 - CW * b2 + r) * 16 + (i1 - 16 * b1));
+            y += gload(pz[q] + (size_t)((pt * nb2 + b2) * nb1 + b1) * 16 * Wc2 + (i2 - CW * b2 + r) * 16 + (i1 - 16 * b1));
+        }
         }
       }
     }
@@ -1041,23 +1000,26 @@ __global__ __launch_bounds__(256) void k_ratio_gather_tpz(FwdGeo g, RatioGeo rg,
   }
 }
 
-// ABI block [e2][e1][phase] -> Toeplitz pack [e1][e2 padded to 16*ceil(K/16)][PHI].
+// ABI block [e2][e1][phase] -> the fragments of k_fwd_tpz, [e1][N-tile][K-step][lane][8].
 template <typename T>
 __global__ void k_pack_fwd_tpz(const float* __restrict__ src, T* __restrict__ dst, PackGeo pg) {
   const int z = blockIdx.y, v = blockIdx.z;
   const float sc = pg.scale ? pg.scale[(size_t)v * gridDim.y + z] : 1.f;
-  const int K = 2 * pg.r[z] + 1;
-  const int nrow = 16 * ((K + 15) / 16);
-  const int PHI = Mma<T>::PHI;
+  const int K = 2 * pg.r[z] + 1, NT = (K + 15) / 16;
   const float* s = src + (size_t)v * pg.src_view + pg.src_off[z];
-  T* d = dst + (size_t)v * pg.dst_view + pg.dst_off[z];
-  const size_t total = (size_t)K * nrow * PHI;
+  typename Mma<T>::frag* d = reinterpret_cast<typename Mma<T>::frag*>(dst + (size_t)v * pg.dst_view + pg.dst_off[z]);
+  const size_t total = (size_t)K * NT * kTpzKS * 64;
   for (size_t o = blockIdx.x * (size_t)blockDim.x + threadIdx.x; o < total;
        o += (size_t)gridDim.x * blockDim.x) {
-    const int ph = (int)(o % PHI);
-    const int e2 = (int)((o / PHI) % nrow);
-    const int e1 = (int)(o / ((size_t)PHI * nrow));
-    d[o] = (T)((e2 < K && ph < kP) ? s[((size_t)e2 * K + e1) * kP + ph] * sc : 0.f);
+    const int lane = (int)(o & 63);
+    const size_t f = o >> 6;
+    const int ph = 32 * (int)(f % kTpzKS) + 8 * (lane >> 4);
+    const int e2 = 16 * (int)((f / kTpzKS) % NT) + (lane & 15), e1 = (int)(f / ((size_t)kTpzKS * NT));
+    typename Mma<T>::frag x;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      x[j] = (T)((e2 < K && ph + j < kP) ? s[((size_t)e2 * K + e1) * kP + ph + j] * sc : 0.f);
+    d[o] = x;
   }
 }
 
@@ -2097,10 +2059,7 @@ hipError_t launch_fwd_mfma(Precision p, const void* W, FwdGeo g, int grid, size_
 
 size_t tpz_smem_bytes(Precision p, int rmax, int MT) {
   if (p == Precision::kF32) return (size_t)2 * kTpzNT * kSplitKS * 3 * kSplitFrag + 4 * MT * 768;
-  const int RV = Mma<__bf16>::PHI / 8;
-  const size_t wslot = ((16 * kTpzNT * RV + 255) / 256) * 256;
-  return (size_t)kTpzBufs * wslot * 16 + elem_bytes(p) * kTpzBufs * 4 * MT * kRingRow +
-         sizeof(float) * 4 * 16 * (MT + 2 * rmax);
+  return tpz_lds(MT);
 }
 
 int64_t fwd_tpz_elems(Precision p, int r) {

@@ -967,7 +967,7 @@ static BwdGeo bwd_geo(mlf_patch_s* p, int k) {
   mlf_psf_s* ps = p->psf;
   const PrecPack& pk = ps->pack[(int)p->kp];
   return BwdGeo{p->d_slot.ptr, ps->d_rb.ptr, pk.d_boff.ptr, pk.d_epad.ptr, p->d_bsched.ptr,
-                p->d_counts.ptr + 1, k, bwd_groups_per_entry(p->bwd_nt, p->bwd_grp)};
+                p->d_counts.ptr + 1, k, p->bwd_gpe};
 }
 
 // Forward projection of view k, then the ratio (LF != null) and/or y.
@@ -1033,8 +1033,61 @@ static mlf_status patch_view_step(mlf_patch_s* p, int k) {
   return MLF_OK;
 }
 
+// Workgroups that the MFMA kernels keep on the card at a time (two per CU).
+constexpr int kSlots = 512;
+
+// Runs of e1 per block of the FP32 Toeplitz forward.  A grid with fewer blocks
+// than the card has room for is split along e1, each run writing partial
+// windows of its own: the run count with the least estimated time, the longer
+// of the average load of a slot and of the longest run, in e1 steps (every run
+// pays about 4 steps for its first operands and its flush; the kernel walks e1
+// twice).  33 x 33 lenslets, 11 planes (165 blocks), per view: forward and
+// ratio 41.7 + 5.6 us whole, 31.3 + 10.3 us split (the ratio reads every run's
+// windows).  Grids of many more than kSlots blocks stay whole.  The count
+// depends on the patch alone, so a patch's sums do not depend on the batch it
+// runs in.  The 16-bit forwards stay whole: their sums keep their order, whose
+// rounding a view step's 16-bit ratio would magnify (8e-5 of the volume after
+// 8 iterations of that patch).
+static int forward_runs(const mlf_psf_s* ps, Precision kp, int cw, int n1, int n2) {
+  if (kp != Precision::kF32) return 1;
+  const int nb = ((n1 + 15) / 16) * ((n2 + cw - 1) / cw);
+  const double per = 2.0, fixed = 4.0;
+  int best = 1;
+  double best_t = 1e300;
+  for (int runs = 1; runs <= 4; ++runs) {
+    double load = 0.0, longest = 0.0;
+    for (int z = 0; z < ps->Z; ++z) {
+      const int K = 2 * ps->rf[z] + 1;
+      load += nb * (runs * fixed + per * K) / kSlots;
+      longest = std::max(longest, fixed + per * ((K + runs - 1) / runs));
+    }
+    const double t = std::max(load, longest);
+    if (t < best_t * 0.95) {
+      best = runs;
+      best_t = t;
+    }
+  }
+  return best;
+}
+
+int mlf::backward_split(int entries, int ngrp, int want) {
+  if (want != ngrp) return want;
+  int best = ngrp;
+  double best_t = 1e300;
+  for (int gpe = ngrp; gpe >= 1; --gpe) {
+    if (ngrp % gpe) continue;
+    const double each = 0.6 + gpe;
+    const double t = std::max((double)entries * (ngrp / gpe) * each / kSlots, each) + 0.5 * each;
+    if (t < best_t * 0.95) {
+      best = gpe;
+      best_t = t;
+    }
+  }
+  return best;
+}
+
 // Forward partial-window elements of each plane for an n1 x n2 grid.
-static int64_t partial_elems(const mlf_psf_s* ps, bool tpz, int cw, int bm2, int n1, int n2,
+static int64_t partial_elems(const mlf_psf_s* ps, bool tpz, int cw, int bm2, int n1, int n2, int fparts,
                              std::vector<int64_t>* poff) {
   const int colw = tpz ? cw : bm2;  // lenslets per block along axis 1
   const int nb1 = (n1 + 15) / 16, nb2 = (n2 + colw - 1) / colw;
@@ -1042,7 +1095,7 @@ static int64_t partial_elems(const mlf_psf_s* ps, bool tpz, int cw, int bm2, int
   for (int z = 0; z < ps->Z; ++z) {
     const int r = ps->rf[z];
     if (poff) (*poff)[z] = po;
-    po += tpz ? (int64_t)nb1 * nb2 * 16 * (cw + 2 * r) : (int64_t)nb1 * nb2 * (16 + 2 * r) * (bm2 + 2 * r);
+    po += tpz ? (int64_t)fparts * nb1 * nb2 * 16 * (cw + 2 * r) : (int64_t)nb1 * nb2 * (16 + 2 * r) * (bm2 + 2 * r);
   }
   return po;
 }
@@ -1104,7 +1157,8 @@ mlf_status mlf::patch_setup_tiles(mlf_patch_s* p) {
   for (int z = 0; z < Z; ++z) order[z] = z;
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return ps->rf[a] > ps->rf[b]; });
   std::vector<int64_t> poff(Z);
-  const int64_t po = partial_elems(ps, p->tpz, p->cw, p->bm2, p->n1, p->n2, &poff);
+  const int fparts = p->tpz ? forward_runs(ps, p->kp, p->cw, p->n1, p->n2) : 1;
+  const int64_t po = partial_elems(ps, p->tpz, p->cw, p->bm2, p->n1, p->n2, fparts, &poff);
   int rfmax = 0, rbmax = 0;
   for (int z = 0; z < Z; ++z) {
     rfmax = std::max(rfmax, ps->rf[z]);
@@ -1113,23 +1167,27 @@ mlf_status mlf::patch_setup_tiles(mlf_patch_s* p) {
   p->fent.clear();
   for (int z : order)
     for (int b2 = 0; b2 < nb2; ++b2)
-      for (int b1 = 0; b1 < nb1; ++b1) {
-        p->fent.push_back(z);
-        p->fent.push_back(b1);
-        p->fent.push_back(b2);
-      }
-  p->nblk_f = (int)(p->fent.size() / 3);
+      for (int b1 = 0; b1 < nb1; ++b1)
+        for (int q = 0; q < fparts; ++q) {
+          p->fent.push_back(z);
+          p->fent.push_back(b1);
+          p->fent.push_back(b2);
+          p->fent.push_back(q);
+        }
+  p->nblk_f = (int)(p->fent.size() / 4);
   {  // one plane per XCD at a time: its blocks share the plane's taps and halo rows
     std::vector<int> grp(p->nblk_f);
-    for (int e = 0; e < p->nblk_f; ++e) grp[e] = p->fent[3 * e];
-    xcd_interleave(p->fent, 3, grp);
+    for (int e = 0; e < p->nblk_f; ++e) grp[e] = p->fent[4 * e];
+    xcd_interleave(p->fent, 4, grp);
   }
   std::vector<int> border(Z);
   for (int z = 0; z < Z; ++z) border[z] = z;
   std::stable_sort(border.begin(), border.end(), [&](int a, int b) { return ps->rb[a] > ps->rb[b]; });
   const int mb1 = (p->n1 + 15) / 16, mb2 = (p->n2 + 15) / 16;
   const int ngrp = kPhiPadBwd / (16 * p->bwd_nt);
-  const int gpe = bwd_groups_per_entry(p->bwd_nt, p->bwd_grp);  // groups per entry share its window
+  // groups per entry share its window
+  const int gpe = backward_split(Z * mb1 * mb2, ngrp, bwd_groups_per_entry(p->bwd_nt, p->bwd_grp));
+  p->bwd_gpe = gpe;
   p->bent.clear();
   for (int z : border)
     for (int b2 = 0; b2 < mb2; ++b2)
@@ -1148,7 +1206,7 @@ mlf_status mlf::patch_setup_tiles(mlf_patch_s* p) {
   }
   p->nblk_r = (p->n1 * p->n2 + kRatioLens - 1) / kRatioLens;
   std::vector<int32_t> fs, bs, rs;
-  append_entries(p->fent, 3, 0, &fs);
+  append_entries(p->fent, 4, 0, &fs);
   append_entries(p->bent, 4, 0, &bs);
   for (int i = 0; i < p->nblk_r; ++i) {
     rs.push_back(0);
@@ -1183,6 +1241,7 @@ mlf_status mlf::patch_setup_tiles(mlf_patch_s* p) {
   sd.n2 = p->n2;
   sd.xs = p->xs;
   sd.xs_inv = 1.f / p->xs;
+  sd.fparts = fparts;
   MLF_CHECK(upload_vec(p->d_slot, std::vector<SlotDesc>{sd}));
   p->smem_f = p->tpz ? tpz_smem_bytes(p->kp, rfmax, p->fwd_mt) : fwd_smem_bytes(p->kp, rfmax, p->bm2);
   p->fwd_nbuf = fwd_nbuf(p->kp, rfmax, p->bm2);
@@ -1248,7 +1307,8 @@ size_t mlf::patch_bytes_estimate(mlf_psf_s* ps, mlf_precision prec, int n1, int 
   const size_t n = (size_t)n1 * n2, Z = (size_t)ps->Z;
   size_t b = 4 * n * Z * kXRow * 2;  // volume + sample_filter temporary
   b += 4 * n * kP + 4 * n * Z + 8 * n;
-  b += 4 * (size_t)partial_elems(ps, tpz, cw, fwd_bm2(kp), n1, n2, nullptr);
+  b += 4 * (size_t)partial_elems(ps, tpz, cw, fwd_bm2(kp), n1, n2, tpz ? forward_runs(ps, kp, cw, n1, n2) : 1,
+                                 nullptr);
   if (kp != Precision::kF32 && tpz) b += 2 * n * Z * kShadowRow;
   if (kp == Precision::kBF16 && tpz) b += 2 * n * Z * kShadowRow;  // lower plane of the split volume
   // entry lists and filter taps: < 1 MB

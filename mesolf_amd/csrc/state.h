@@ -115,7 +115,8 @@ struct mlf_patch_s {
   mlf::DevBuf<int64_t> d_poff;
   // work entries of this patch: host (without slot index) for batch assembly,
   // device (slot 0) for single-patch launches
-  std::vector<int32_t> fent, bent;     // (z, b1, b2), (z, b1, b2, group)
+  std::vector<int32_t> fent, bent;     // (z, b1, b2, run of e1), (z, b1, b2, first group)
+  int bwd_gpe = 1;                     // phase groups per entry of bent (backward_split)
   mlf::DevBuf<int32_t> d_fsched, d_bsched, d_rsched, d_counts;  // counts: fwd, bwd, ratio
   mlf::SlotDesc slot{};
   mlf::DevBuf<mlf::SlotDesc> d_slot;
@@ -183,6 +184,14 @@ struct TileShape {
 std::vector<TileShape> tile_candidates(Precision kp);
 // Phase groups per backprojection entry that a shape asks for (0 -> all).
 int bwd_groups_per_entry(int nt, int grp);
+// Phase groups per backprojection entry for `entries` lenslet tiles: `want`, or
+// fewer where all groups of a tile in one entry would leave the card idle (a
+// divisor of ngrp with the least estimated time, an entry costing its groups
+// and 0.6 of a group for its ratio window).  33 x 33 lenslets, 11 planes (99
+// tiles), per view: BF16 31.6 us, as 396 entries 16.9 us; FP32 59.0 us, as 297
+// entries 26.4 us.  Beyond about 450 tiles all groups stay in one entry.  The results do
+// not depend on it.
+int backward_split(int entries, int ngrp, int want);
 // Tile shape cache (per process, optionally persisted in the file named by
 // MLF_TUNE_CACHE): key = precision, grid(s), PSF radii.
 bool tune_cache_get(const std::string& key, Precision kp, TileShape* shape);
