@@ -682,18 +682,18 @@ void k_fwd_tps(const char* __restrict__ W, FwdGeo g) {
         }
       }
     };
-    // piece q of step st's taps (st = h (t1 - t0) + t - t0): this wave's share of N-tile q / 3
+    // piece q of a step's taps at byte `at` of the plane's: this wave's share of N-tile q / 3
     const unsigned tap_lane = 16 * lane;
     const int nt1 = t1 - t0;
-    auto issue_w = [&](int st, int q) __attribute__((always_inline)) {
-      const int col = st < nt1 ? t0 + st : K + t0 + st - nt1;  // column of [half][e1]
+    auto issue_w = [&](int buf, int at, int q) __attribute__((always_inline)) {
       const unsigned vo = 16 * (q / 3) + lr < K ? tap_lane : 0x80000000u;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          wr, (__attribute__((address_space(3))) void*)(smem + (st & 1) * WBUF + (4 * q + w) * kSplitFrag), 16, vo,
-          col * step_bytes + (4 * q + w) * kSplitFrag, 0, 0);
+          wr, (__attribute__((address_space(3))) void*)(smem + buf * WBUF + (4 * q + w) * kSplitFrag), 16, vo,
+          at + (4 * q + w) * kSplitFrag, 0, 0);
     };
+    int w_at = t0 * step_bytes;  // of the step whose taps are copied next
     if (nt1 > 0) {
-      for (int q = 0; q < 3 * NT; ++q) issue_w(0, q);
+      for (int q = 0; q < 3 * NT; ++q) issue_w(0, w_at, q);
     }
     load_a(0);
 
@@ -722,6 +722,7 @@ void k_fwd_tps(const char* __restrict__ W, FwdGeo g) {
       }
       const char* Wc = smem + (st & 1) * WBUF + 16 * lane;
       const bool more = st + 1 < nst;
+      w_at = last_t ? (K + t0) * step_bytes : w_at + step_bytes;
       bf16x8 bn[3];
 #pragma unroll
       for (int p = 0; p < 3; ++p) bn[p] = *reinterpret_cast<const bf16x8*>(Wc + p * kSplitFrag);
@@ -740,7 +741,7 @@ void k_fwd_tps(const char* __restrict__ W, FwdGeo g) {
           // the next K-step's fragments (past the plane's tiles: unused)
 #pragma unroll
           for (int p = 0; p < 3; ++p) bn[p] = *reinterpret_cast<const bf16x8*>(Wc + (3 * qn + p) * kSplitFrag);
-          if (more && q < 3 * NT) issue_w(st + 1, q);
+          if (more && q < 3 * NT) issue_w((st + 1) & 1, w_at, q);
           // smallest products first
           constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
