@@ -942,24 +942,26 @@ __global__ __launch_bounds__(256) void k_ratio_gather_tpz(FwdGeo g, RatioGeo rg,
     const int i1 = ok ? i % n1 : 0, i2 = ok ? i / n1 : 0;
     const int nb1 = ceil_div(n1, 16), nb2 = ceil_div(n2, CW);
     const int b1 = i1 / 16;
-    // The slice's planes go in chunks of kZC: the radii and offsets of a chunk
-    // are read together, then up to kW windows per plane (all of them for
-    // 16-column blocks, r <= 23), and only then summed, in plane then window
-    // order, one run of e1 after the other (an unused slot adds +0.0, which changes no sum).  A plane with
-    // more windows (narrower blocks) reads the rest one by one.
+    // The slice's (plane, run of e1) pairs go in chunks of kZC: the radii and
+    // offsets of a chunk are read together, then up to kW windows per pair (all
+    // of them for 16-column blocks, r <= 23), and only then summed, in plane, run
+    // and window order (an unused slot adds +0.0, which changes no sum).  A pair
+    // with more windows (narrower blocks) reads the rest one by one.
     float y = 0.f;
     if (ok) {
       constexpr int kZC = 8, kW = 4;
-      for (int zc = z0; zc < z1; zc += kZC) {
-        int rr[kZC];
+      const int runs = sd.fparts, q1 = z1 * runs;
+      for (int qc = z0 * runs; qc < q1; qc += kZC) {
+        int rr[kZC], row[kZC];  // radius; b2 = 0 row of the run's windows
         const float* pz[kZC];
   #pragma unroll
         for (int q = 0; q < kZC; ++q) {
-          const int zq = min(zc + q, z1 - 1);  // the plane slice differs between the half-waves
+          const int v = min(qc + q, q1 - 1);  // the plane slice differs between the half-waves
+          const int zq = runs == 1 ? v : v / runs;
           rr[q] = gload(g.r + zq);
           pz[q] = sd.partial + gload(sd.poff + zq);
+          row[q] = (v - zq * runs) * nb2;
         }
-        for (int pt = 0; pt < sd.fparts; ++pt) {
         float vv[kZC][kW];
   #pragma unroll
         for (int q = 0; q < kZC; ++q) {
@@ -969,23 +971,22 @@ __global__ __launch_bounds__(256) void k_ratio_gather_tpz(FwdGeo g, RatioGeo rg,
   #pragma unroll
           for (int wi = 0; wi < kW; ++wi) {
             const int b2 = b2l + wi;
-            const bool use = zc + q < z1 && b2 <= b2h;
-            const size_t idx = use ? (size_t)((pt * nb2 + b2) * nb1 + b1) * 16 * Wc2 + (i2 - CW * b2 + r) * 16 + (i1 - 16 * b1) : 0;
+            const bool use = qc + q < q1 && b2 <= b2h;
+            const size_t idx = use ? (size_t)((row[q] + b2) * nb1 + b1) * 16 * Wc2 + (i2 - CW * b2 + r) * 16 + (i1 - 16 * b1) : 0;
             const float t = gload(pz[q] + idx);
             vv[q][wi] = use ? t : 0.f;
           }
         }
   #pragma unroll
         for (int q = 0; q < kZC; ++q) {
-          if (zc + q >= z1) break;
+          if (qc + q >= q1) break;
   #pragma unroll
           for (int wi = 0; wi < kW; ++wi) y += vv[q][wi];
           const int r = rr[q], Wc2 = CW + 2 * r;
           const int b2h = min(nb2 - 1, (i2 + r) / CW);
           const int b2l = (i2 - r - CW + 1 <= 0) ? 0 : (i2 - r - CW + 1 + CW - 1) / CW;
           for (int b2 = b2l + kW; b2 <= b2h; ++b2)
-            y += gload(pz[q] + (size_t)((pt * nb2 + b2) * nb1 + b1) * 16 * Wc2 + (i2 - CW * b2 + r) * 16 + (i1 - 16 * b1));
-        }
+            y += gload(pz[q] + (size_t)((row[q] + b2) * nb1 + b1) * 16 * Wc2 + (i2 - CW * b2 + r) * 16 + (i1 - 16 * b1));
         }
       }
     }
