@@ -25,32 +25,23 @@ constexpr int kPhiPadBwd = 256;   // phase rows of a backward plane block: 3 gro
 // registers and LDS per workgroup, so three workgroups share a CU.
 constexpr int kBwdStages = 6;
 inline __host__ __device__ constexpr int bwd_stages(int occ) { return occ >= 3 ? 4 : kBwdStages; }
-// Bytes before the 16-bit backprojection's shifted window: the FP32 staging
-// window [Wd][Wd] and the tap ring (bwd_stages slices of [16 nt][32] taps),
-// which alias (the staging window is dead once the shifted one is built).
-inline __host__ __device__ int bwd_ring_bytes(int Wd, int nt, int elem_bytes, int occ) {
-  const int rs = 4 * ((Wd * Wd + 3) & ~3);
-  const int ring = bwd_stages(occ) * nt * 16 * 32 * elem_bytes;
-  return rs > ring ? rs : ring;
-}
 // 16-bit backprojection tap order.  Row length K is padded to Kp8 (a multiple
 // of 8) and the row count to a multiple of 4; K-step ks (32 taps) holds the
 // 8-tap pieces (e2 = 4 (ks / nch) + q, e1 = 8 (ks % nch) + 0..7), q = 0..3,
 // nch = Kp8 / 8.  The four pieces of a step then sit at one window column in
-// four consecutive rows, so with window rows of a multiple of 16 cells the
-// four 16-lane groups of an A-fragment read hit the same LDS bank groups.
+// four consecutive rows.
 inline __host__ __device__ int bwd_quad_steps(int K) { return ((K + 7) / 8) * ((K + 3) / 4); }
 inline __host__ __device__ void bwd_quad_tap(int t, int K, int* e2, int* e1) {
   const int nch = (K + 7) / 8, ks = t / 32, w = t % 32, b = ks / nch;
   *e2 = 4 * b + w / 8;
   *e1 = 8 * (ks - b * nch) + w % 8;
 }
-// Window row stride (cells) of the 16-bit backprojection: a multiple of 16
-// when the workgroup's LDS still fits (otherwise Wd, with bank conflicts).
-inline __host__ __device__ int bwd_row_cells(int Wd, int nt, int occ) {
-  const int a = (Wd + 15) & ~15;
-  return bwd_ring_bytes(Wd, nt, 2, occ) + 16 * Wd * a <= 160 * 1024 ? a : Wd;
-}
+// Dwords per row and copy of the 16-bit backprojection's window: room for the
+// 8-tap pieces past the last column, and 8 modulo 16, so that the four rows and
+// two copies that a fragment read touches fall on different banks.
+inline __host__ __device__ constexpr int bwd_pair_row(int Wd) { return 8 + 16 * ((Wd / 2 + 3 - 8 + 15) / 16); }
+// largest radius of the backprojection
+inline constexpr int bwd_max_radius(Precision p) { return p == Precision::kF32 ? 67 : 37; }
 constexpr int kRatioLens = 32;    // lenslets per ratio work entry
 constexpr int kRatioSlices = 8;   // plane slices summed in parallel per entry (x kRatioLens = 256 threads)
 constexpr int kBwdTapPad = 64;    // an even number of K-steps of 32 taps (the K loop runs in pairs)

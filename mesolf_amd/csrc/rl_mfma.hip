@@ -1069,40 +1069,6 @@ __global__ __launch_bounds__(256) void k_ratio_gather(FwdGeo g, RatioGeo rg, int
 }
 
 // --------------------------------------------------------------- backward
-// dst[y][x] = R(a1_0 + x, a2_0 + y) for a Wd x Wd window (0 outside the
-// grid), 256 threads.  The reads of up to 16 cells per thread are issued
-// before any is waited for (clamped addresses, the zero applied by a select),
-// so a window costs about one L2 round trip instead of one per 256 cells.
-__device__ __forceinline__ void gather_window(const float* __restrict__ R, int n1, int n2, int a1_0,
-                                              int a2_0, int Wd, float* __restrict__ dst) {
-  constexpr int kPer = 16;
-  const int tid = threadIdx.x, ncell = Wd * Wd;
-  // global (not flat) loads: a pending flat load makes the compiler wait for
-  // every memory operation at the next use of any loaded register
-  const __attribute__((address_space(1))) float* Rg = (const __attribute__((address_space(1))) float*)R;
-  for (int c0 = 0; c0 < ncell; c0 += 256 * kPer) {
-    float v[kPer];
-  #pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-      const int o = min(c0 + tid + 256 * q, ncell - 1);
-      const int y = o / Wd, x = o - y * Wd;
-      const int a1 = a1_0 + x, a2 = a2_0 + y;
-      const bool in = a1 >= 0 && a1 < n1 && a2 >= 0 && a2 < n2;
-      const float t = Rg[min(max(a1, 0), n1 - 1) + n1 * min(max(a2, 0), n2 - 1)];
-      v[q] = in ? t : 0.f;
-    }
-    // every load waited for here, on every path: a load the compiler still
-    // counts as in flight later (its register reused) would make it wait at
-    // the reuse for the memory operations issued since, stores included
-    wait_vm<0>();
-  #pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-      const int o = c0 + tid + 256 * q;
-      if (o < ncell) dst[o] = v[q];
-    }
-  }
-}
-
 __device__ __forceinline__ int norm_class(int a, int n, int r) {
   if (n < 2 * r + 1) return a;  // small grid: one class per lenslet
   return a < r ? a : (a > n - 1 - r ? 2 * r - (n - 1 - a) : r);
@@ -1180,48 +1146,114 @@ void k_bwd_mfma(const T* __restrict__ Wb, BwdGeo g, float wgt) {
     const bool ok1 = a1 < n1;
     const int a1c = ok1 ? a1 : n1 - 1;
     const int c1 = norm_class(a1c, n1, r);
-    // window cell of this lane's lenslet in M-tile mt: base + mt * Wr
-    const int Wr = bwd_row_cells(Wd, NT, OCC);
-    const int base = (lr + r) + (4 * w + r) * Wr;
-
-    // ratio window
+    // Ratio window as 16-bit operands, two copies per row: cell x of row y (R(16
+    // b1 - r + x, 16 b2 - r + y)) lies at position p = Wd - 1 - x, copy 0 holds the pairs (p, p
+    // + 1) from even p, copy 1 from odd p.  A lane's 8 taps of a K-step are 8
+    // consecutive e1 in one row (bwd_quad_tap), i.e. 8 ascending positions, read
+    // as four dwords of the copy of their parity.  Eight shifted copies, one
+    // 16-byte read per fragment, need twice the LDS and a second pass over a
+    // staged FP32 window, behind which the first tap slices had to wait: with
+    // two copies a view step went from 17.1 to 15.6 us at 33x33x11 (entries of few
+    // K-steps, where the window is most of the time), 154.5 to 151.0 us at
+    // 81x73x31 (FP16) and 332.3 to 330.1 us at 101x101x51.
     using frag_t = typename M::frag;
-    // [Wd][Wr] after the staging window Rs / tap ring (which alias)
-    frag_t* Rv = reinterpret_cast<frag_t*>(smem + bwd_ring_bytes(Wd, NT, (int)sizeof(T), OCC));
+    const int Wr = bwd_pair_row(Wd);
+    unsigned* const Rp = reinterpret_cast<unsigned*>(smem);  // [Wd][2][Wr]
+    const unsigned* const Rl = Rp + (2 * (4 * w + 2 * r) + ((15 - lr) & 1)) * Wr + ((15 - lr) >> 1);
+    constexpr bool PAIR = SPL;
+    // SPB K-steps per barrier: a step's copies are waited for, and the
+    // ring refilled, once per SPB steps; the ring then runs STG - SPB
+    // steps ahead.  nks is even (taps padded to 64).
+    constexpr int SPB = OCC >= 3 ? 1 : 2;
+    static_assert(STG >= 2 * SPB, "ring too shallow");
+    // Taps go global -> LDS by DMA (global_load_lds, one copy per
+    // workgroup instead of one per wave through the L1) into a ring of
+    // STG K-step slices [16 NT rows][32 taps], STG - SPB steps ahead;
+    // no slice past the last step is copied, and the waits count only
+    // the copies issued.  The window offset of a lane's 8 taps follows the step's row
+    // block and column chunk (bwd_quad_tap), stepped without divisions.
+    const int nch = (K + 7) / 8;
+    T* Bq = reinterpret_cast<T*>(smem + 8 * Wd * Wr);  // ring
+    constexpr int kSlice = NT * 16 * 32;  // elements per K-step slice
+    const int ncopy = w < NT ? (NT - w + 3) / 4 : 0;  // copies per step issued by this wave
+    // A copy moves one N-tile's slice (16 rows x 32 taps) as 64 16-byte
+    // pieces, DMA lane s landing at byte 16 s.  Piece (row, 8-tap group q)
+    // goes to s = 16 q + row, so the 16 lanes reading group q at rows
+    // 0..15 read 16 consecutive pieces and the four groups the same bank
+    // groups (the pattern ds_read_b128 serves without conflicts).
+    // SPL: slice row j of a paired N-tile (half h) is phase row
+    // 8 (j / 4) + 4 h + j % 4 of the pair (lph).
+    // 16-bit tables are stored tile-major (bwd_tap_index): a 16-row tile's
+    // K-step is 1 KB of contiguous memory, [16 rows][32 taps].  Element
+    // offset of (row R of the tile pair starting at row0, tap tq of the step):
+    // (R / 16) * 16 epad + (R % 16) * 32 + tq, for R < 32.
+    const int jr = lane & 15, tq = (lane >> 4) * 8;
+    auto tap_off = [&](int R) { return ((R >> 4) * 16 * epad + (R & 15) * 32 + tq) * (int)sizeof(T); };
+    const int tap_lane_s = tap_off(jr);                                  // unpaired tile
+    const int tap_lane_p0 = tap_off(8 * (jr >> 2) + (jr & 3));           // pair, half 0
+    const int tap_lane_p1 = tap_off(8 * (jr >> 2) + 4 + (jr & 3));       // pair, half 1
+    const int tap_slot = (16 * lg + lr) * 8;  // element offset of (row lr, 8-tap group lg) in an N-tile slice
+    // copies of K-step ks of phase group gx into ring slot `slot`: buffer
+    // loads to LDS (MUBUF) over the plane's table, [kPhiPadBwd rows][epad]
+    // taps.  A FLAT-encoded global_load_lds would count as an access that
+    // may reach LDS out of order, and the compiler then turns every wait for
+    // a load issued before it into a wait for all memory operations,
+    // stores included.
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<T*>(Wb + boffz), 0, kPhiPadBwd * epad * (int)sizeof(T), kBufferDword3);
+    auto issue_taps_g = [&](int gx, int ks, int slot) {
+      if (ks >= nks) return;  // past the last step (wave-uniform)
+      const int kc = ks;
+      const int oddx = PAIR && NT % 2 == 1 ? (gx & 1) : 0;
+      char* dst = reinterpret_cast<char*>(Bq + slot * kSlice);
+      for (int nt = w; nt < NT; nt += 4) {
+        const bool pr = PAIR && nt < 2 * NPR;
+        // first packed row relative to the group
+        const int row0 = !PAIR ? 16 * nt : pr ? 16 * oddx + 16 * (nt & ~1) : (oddx ? 0 : 16 * (NT - 1));
+        const int tl = pr ? ((nt & 1) ? tap_lane_p1 : tap_lane_p0) : tap_lane_s;
+        const int so = ((gx * 16 * NT + row0) * epad + kc * 512) * (int)sizeof(T);  // wave-uniform
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (__attribute__((address_space(3))) void*)(dst + nt * 1024),
+                                                 16, tl, so, 0, 0);
+      }
+    };
+    // the first group's first slices are under way while the window is built
+  #pragma unroll
+    for (int q = 0; q < STG - SPB; ++q) issue_taps_g(grp0, q, q);
     {
-      // a lane's 8 taps of a K-step are 8 consecutive e1 in one row
-      // (bwd_quad_tap).  Cell (x, y) of the pre-shifted window holds R(x-j, y)
-      // for j = 0..7, so each A fragment is a single 16-byte LDS read.
-      float* Rs = reinterpret_cast<float*>(smem);  // [Wd][Wd]
-      gather_window(R, n1, n2, 16 * b1 - r, 16 * b2 - r, Wd, Rs);
-      lds_barrier();
-      // four cells per thread per pass, their 32 reads issued together
-      for (int c0 = 0; c0 < Wd * Wd; c0 += 4 * 256) {
-        float rv[4][8];
+      const __amdgpu_buffer_rsrc_t rr =
+          __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(R), 0, (int)(nlp * 4), kBufferDword3);
+      constexpr int kPer = 4;
+      for (int c0 = 0; c0 < Wd * Wr; c0 += 256 * kPer) {
+        float v[kPer][3];
   #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int o = min(c0 + tid + 256 * q, Wd * Wd - 1);
-          const int x = o % Wd;
+        for (int q = 0; q < kPer; ++q) {
+          const int o = c0 + tid + 256 * q, y = o / Wr, i2 = 16 * b2 - r + y;
+          const int x0 = Wd - 1 - 2 * (o - y * Wr);  // cell of the first position
   #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const float t = Rs[max(o - j, 0)];
-            rv[q][j] = x - j >= 0 ? t : 0.f;
+          for (int j = 0; j < 3; ++j) {
+            const int i1 = 16 * b1 - r + x0 - j;
+            const bool in = x0 - j >= 0 && y < Wd && i1 >= 0 && i1 < n1 && i2 >= 0 && i2 < n2;
+            v[q][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                    rr, in ? 4u * (unsigned)(i2 * n1 + i1) : 0x80000000u, 0, 0));
           }
         }
+        // every load waited for here, on every path: a load the compiler still
+        // counts as in flight later (its register reused) would make it wait at
+        // the reuse for the memory operations issued since, stores included
+        wait_vm<0>();
   #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int o = c0 + tid + 256 * q;
-          if (o < Wd * Wd) {
-            frag_t v;
+        for (int q = 0; q < kPer; ++q) {
+          const int o = c0 + tid + 256 * q, y = o / Wr;
+          unsigned short h[3];
   #pragma unroll
-            for (int j = 0; j < 8; ++j)
-              v[j] = (T)(is_f16<T>() ? fminf(rv[q][j], 65504.f) : rv[q][j]);  // FP16: clamp to the largest finite value
-            const int y = o / Wd;
-            Rv[o + y * (Wr - Wd)] = v;  // cell (o % Wd, y)
+          for (int j = 0; j < 3; ++j)  // FP16: cut to the largest finite value
+            h[j] = to_bits16<T>(is_f16<T>() ? fminf(v[q][j], 65504.f) : v[q][j]);
+          if (o < Wd * Wr) {
+            Rp[o + y * Wr] = (unsigned)h[0] | ((unsigned)h[1] << 16);
+            Rp[o + (y + 1) * Wr] = (unsigned)h[1] | ((unsigned)h[2] << 16);
           }
         }
       }
-      lds_barrier();  // Rv written, Rs read by every wave (the ring copies overwrite Rs)
     }
 
     bool pref = false;  // the group's first tap slices were issued by the previous group
@@ -1243,7 +1275,6 @@ void k_bwd_mfma(const T* __restrict__ Wb, BwdGeo g, float wgt) {
       // N-tile NT - 1 covers 16 phases in order, after the pairs in even
       // groups and before them in odd ones (whose first phase is 16 past a
       // 32-aligned one).  The tap copies below place the rows to match.
-      constexpr bool PAIR = SPL;
       const int gbase = grp * 16 * NT;
       // with an odd tile count, a group starts 16 phases past a 32-aligned
       // phase when its index is odd
@@ -1328,61 +1359,6 @@ void k_bwd_mfma(const T* __restrict__ Wb, BwdGeo g, float wgt) {
       static_assert(kEpiLoads + kUpdOps + (bwd_stages(OCC) - 2 * (OCC >= 3 ? 1 : 2)) * ((NT + 3) / 4) <= 63,
                     "wait_vm_le covers at most 63 operations in flight");
 
-      // SPB K-steps per barrier: a step's copies are waited for, and the
-      // ring refilled, once per SPB steps; the ring then runs STG - SPB
-      // steps ahead.  nks is even (taps padded to 64).
-      constexpr int SPB = OCC >= 3 ? 1 : 2;
-      static_assert(STG >= 2 * SPB, "ring too shallow");
-      // Taps go global -> LDS by DMA (global_load_lds, one copy per
-      // workgroup instead of one per wave through the L1) into a ring of
-      // STG K-step slices [16 NT rows][32 taps], STG - SPB steps ahead;
-      // no slice past the last step is copied, and the waits count only
-      // the copies issued.  The window offset of a lane's 8 taps follows the step's row
-      // block and column chunk (bwd_quad_tap), stepped without divisions.
-      const int nch = (K + 7) / 8;
-      T* Bq = reinterpret_cast<T*>(smem);  // ring (aliases the dead staging window Rs)
-      constexpr int kSlice = NT * 16 * 32;  // elements per K-step slice
-      const int ncopy = w < NT ? (NT - w + 3) / 4 : 0;  // copies per step issued by this wave
-      // A copy moves one N-tile's slice (16 rows x 32 taps) as 64 16-byte
-      // pieces, DMA lane s landing at byte 16 s.  Piece (row, 8-tap group q)
-      // goes to s = 16 q + row, so the 16 lanes reading group q at rows
-      // 0..15 read 16 consecutive pieces and the four groups the same bank
-      // groups (the pattern ds_read_b128 serves without conflicts).
-      // SPL: slice row j of a paired N-tile (half h) is phase row
-      // 8 (j / 4) + 4 h + j % 4 of the pair (lph).
-      // 16-bit tables are stored tile-major (bwd_tap_index): a 16-row tile's
-      // K-step is 1 KB of contiguous memory, [16 rows][32 taps].  Element
-      // offset of (row R of the tile pair starting at row0, tap tq of the step):
-      // (R / 16) * 16 epad + (R % 16) * 32 + tq, for R < 32.
-      const int jr = lane & 15, tq = (lane >> 4) * 8;
-      auto tap_off = [&](int R) { return ((R >> 4) * 16 * epad + (R & 15) * 32 + tq) * (int)sizeof(T); };
-      const int tap_lane_s = tap_off(jr);                                  // unpaired tile
-      const int tap_lane_p0 = tap_off(8 * (jr >> 2) + (jr & 3));           // pair, half 0
-      const int tap_lane_p1 = tap_off(8 * (jr >> 2) + 4 + (jr & 3));       // pair, half 1
-      const int tap_slot = (16 * lg + lr) * 8;  // element offset of (row lr, 8-tap group lg) in an N-tile slice
-      // copies of K-step ks of phase group gx into ring slot `slot`: buffer
-      // loads to LDS (MUBUF) over the plane's table, [kPhiPadBwd rows][epad]
-      // taps.  A FLAT-encoded global_load_lds would count as an access that
-      // may reach LDS out of order, and the compiler then turns every wait for
-      // a load issued before it into a wait for all memory operations,
-      // stores included.
-      const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
-          const_cast<T*>(Wb + boffz), 0, kPhiPadBwd * epad * (int)sizeof(T), kBufferDword3);
-      auto issue_taps_g = [&](int gx, int ks, int slot) {
-        if (ks >= nks) return;  // past the last step (wave-uniform)
-        const int kc = ks;
-        const int oddx = PAIR && NT % 2 == 1 ? (gx & 1) : 0;
-        char* dst = reinterpret_cast<char*>(Bq + slot * kSlice);
-        for (int nt = w; nt < NT; nt += 4) {
-          const bool pr = PAIR && nt < 2 * NPR;
-          // first packed row relative to the group
-          const int row0 = !PAIR ? 16 * nt : pr ? 16 * oddx + 16 * (nt & ~1) : (oddx ? 0 : 16 * (NT - 1));
-          const int tl = pr ? ((nt & 1) ? tap_lane_p1 : tap_lane_p0) : tap_lane_s;
-          const int so = ((gx * 16 * NT + row0) * epad + kc * 512) * (int)sizeof(T);  // wave-uniform
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (__attribute__((address_space(3))) void*)(dst + nt * 1024),
-                                                   16, tl, so, 0, 0);
-        }
-      };
       auto issue_taps = [&](int ks, int slot) { issue_taps_g(grp, ks, slot); };
       // the first STG - SPB slices of the next phase group of the entry,
       // issued once every wave is done with the ring, so that they land
@@ -1399,10 +1375,6 @@ void k_bwd_mfma(const T* __restrict__ Wb, BwdGeo g, float wgt) {
         // the first slices came from the previous group's prefetch: the
         // update's operations issued since are younger than them
         const int upd = pref ? kUpdOps : 0;
-        if (!pref) {
-  #pragma unroll
-          for (int q = 0; q < STG - SPB; ++q) issue_taps(q, q);
-        }
         pref = false;
         if constexpr (PRE > 0) {
           load_x(0, PRE);  // after the first slices: their waits need not cover these loads
@@ -1440,7 +1412,7 @@ void k_bwd_mfma(const T* __restrict__ Wb, BwdGeo g, float wgt) {
             // piece lg: row e2 = 4 qb + lg, taps e1 = 8 qc .. 8 qc + 7; rows
             // past K (zero weights) read row K - 1, which keeps the bank pattern
             const int e2 = min(4 * qb + lg, K - 1);
-            const int o = (r - 8 * qc) - (e2 - r) * Wr;
+            const unsigned* R0 = Rl - 2 * e2 * Wr + 4 * qc;
             if (++qc == nch) {
               qc = 0;
               ++qb;
@@ -1452,7 +1424,10 @@ void k_bwd_mfma(const T* __restrict__ Wb, BwdGeo g, float wgt) {
             // to the top, which would leave no registers for the A fragments)
             frag_t af[MT];
   #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) af[mt] = Rv[base + mt * Wr + o];
+            for (int mt = 0; mt < MT; ++mt) {
+              const unsigned* p = R0 + 2 * mt * Wr;
+              af[mt] = __builtin_bit_cast(frag_t, uintx4{p[0], p[1], p[2], p[3]});
+            }
             frag_t bq[3];
             bq[0] = *reinterpret_cast<const frag_t*>(Bs + tap_slot);
             if (NT > 1) bq[1] = *reinterpret_cast<const frag_t*>(Bs + 512 + tap_slot);
@@ -1690,8 +1665,12 @@ void k_bwd_mfma(const T* __restrict__ Wb, BwdGeo g, float wgt) {
 // three groups; groups of 48 measured 580 us (each group splits the window again).
 constexpr int kBwdSplitStages = 4;
 // Floats per window row: room for the 8-tap pieces past the last column, and
-// 16 modulo 32 so that the four rows of a fragment read fall on different banks.
-inline __host__ __device__ constexpr int bwd_split_row(int Wd) { return 16 + 32 * ((Wd + 7 - 16 + 31) / 32); }
+// 16 modulo 32 so that the four rows of a fragment read fall on different banks
+// (where the workgroup's LDS still fits).
+inline __host__ __device__ constexpr int bwd_split_row(int Wd, int nt) {
+  const int row = 16 + 32 * ((Wd + 7 - 16 + 31) / 32);
+  return 4 * Wd * row + kBwdSplitStages * nt * 3 * kSplitFrag <= 160 * 1024 ? row : Wd + 8;
+}
 
 template <int NT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
@@ -1710,7 +1689,7 @@ void k_bwd_split(const char* __restrict__ Wb, BwdGeo g, float wgt) {
     const int r = uni(cload(g.r + z));
     const int K = 2 * r + 1, nch = (K + 7) / 8;
     const int nks = uni(cload(g.epad + z)) / 32;
-    const int Wd = 16 + 2 * r, Wr = bwd_split_row(Wd);
+    const int Wd = 16 + 2 * r, Wr = bwd_split_row(Wd, NT);
     const int tid = threadIdx.x, lane = tid & 63, w = uni(tid >> 6), lr = lane & 15, lg = lane >> 4;
     float* const Rw = reinterpret_cast<float*>(smem);  // [Wd][Wr]
     char* const ring = smem + 4 * Wd * Wr;
@@ -2036,8 +2015,8 @@ size_t fwd_smem_bytes(Precision p, int rmax, int bm2) {
 size_t bwd_smem_bytes(Precision p, int rmax, int nt, int occ) {
   const int Wd = 16 + 2 * rmax;
   if (p == Precision::kF32)
-    return sizeof(float) * (size_t)Wd * bwd_split_row(Wd) + (size_t)kBwdSplitStages * nt * 3 * kSplitFrag;
-  return bwd_ring_bytes(Wd, nt, 2, occ) + 16 * (size_t)Wd * bwd_row_cells(Wd, nt, occ);
+    return sizeof(float) * (size_t)Wd * bwd_split_row(Wd, nt) + (size_t)kBwdSplitStages * nt * 3 * kSplitFrag;
+  return 8 * (size_t)Wd * bwd_pair_row(Wd) + (size_t)bwd_stages(occ) * nt * kFrag;
 }
 
 hipError_t launch_fwd_mfma(Precision p, const void* W, FwdGeo g, int grid, size_t smem, int nbuf,

@@ -1215,7 +1215,7 @@ mlf_status mlf::patch_setup_tiles(mlf_patch_s* p) {
   p->smem_f = p->tpz ? tpz_smem_bytes(p->kp, rfmax, p->fwd_mt) : fwd_smem_bytes(p->kp, rfmax, p->bm2);
   p->fwd_nbuf = fwd_nbuf(p->kp, rfmax, p->bm2);
   p->smem_b = bwd_smem_bytes(p->kp, rbmax, p->bwd_nt, p->bwd_occ);
-  if (p->smem_f > 160 * 1024 || p->smem_b > 160 * 1024)
+  if (p->smem_f > 160 * 1024 || p->smem_b > 160 * 1024 || rbmax > bwd_max_radius(p->kp))
     return set_error(MLF_ERR_UNSUPPORTED,
                      "PSF radius too large for the LDS tiles (rf_max=%d, rb_max=%d)", rfmax, rbmax);
   return MLF_OK;
