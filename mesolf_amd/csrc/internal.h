@@ -155,10 +155,16 @@ hipError_t launch_summary(const float* Y, size_t npix, int T, int w1, int w2, in
 // whether launch_summary keeps a detrended movie in dbuf [npix, T] ('pixelwise')
 bool summary_needs_movie(size_t npix, int T);
 const double* summary_temporal(const double* scratch);
+// Query coordinates along one axis: point i is grid point m = q0 + i, at
+// center - step (first - 1 - m) below m = first, then (center + step) + step (m - first).
+struct RectAxis {
+  double center, step;
+  int64_t first, q0, size;
+};
 // Bilinear (griddedInterpolant 'linear', extrapolating) resample of n frames
-// [H, W] at yq [Hq] x xq [Wq] (device arrays, 1-based pixel coordinates).
-hipError_t launch_rectify(const float* in, int H, int W, int n, const double* yq, int Hq, const double* xq,
-                          int Wq, float* out, hipStream_t st);
+// [H, W] at yq x xq (1-based pixel coordinates).
+hipError_t launch_rectify(const float* in, int H, int W, int n, RectAxis yq, RectAxis xq, float* out,
+                          hipStream_t st);
 // out [h, w, T] = in(top : top+h-1, left : left+w-1, :) of in [H, W, T], 0-based corner.
 hipError_t launch_crop_movie(const float* in, int64_t H, int64_t W, int64_t top, int64_t left, int h,
                              int w, int T, float* out, hipStream_t st);

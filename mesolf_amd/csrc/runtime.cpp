@@ -1923,24 +1923,19 @@ mlf_status mlf_lfm_convolution_vec(const float* bitmap, int64_t width, int64_t h
 // coordinates along one axis, step dx/M through `center`, from -dx/M to
 // size + 0.9, started at a whole lenslet and cut to whole lenslets.  MATLAB's
 // a:d:b is taken as a + k*d.
-static std::vector<double> rectify_axis(double center, int64_t size, int M, double dx) {
+static RectAxis rectify_axis(double center, int64_t size, int M, double dx) {
   const double s = dx / M;
-  auto colon = [](double a, double d, double b) {
-    const int64_t n = (int64_t)std::floor((b - a) / d + 1e-10) + 1;
-    std::vector<double> v;
-    for (int64_t k = 0; k < n; ++k) v.push_back(a + d * (double)k);
-    return v;
+  auto count = [](double a, double d, double b) {
+    return std::max<int64_t>(0, (int64_t)std::floor((b - a) / d + 1e-10) + 1);
   };
-  std::vector<double> first = colon(center, -s, -s);
-  std::reverse(first.begin(), first.end());
-  const std::vector<double> second = colon(center + s, s, (double)size + 0.9);
-  std::vector<double> grid(first);
-  grid.insert(grid.end(), second.begin(), second.end());
-  const int64_t qc = (int64_t)first.size() - M / 2;  // find(grid == center) - floor(M/2)
-  const int64_t q0 = qc - (int64_t)M * (int64_t)std::floor((double)qc / M);
-  std::vector<double> q;
-  if (q0 < (int64_t)grid.size()) q.assign(grid.begin() + q0, grid.end());
-  q.resize(q.size() / M * M);
+  RectAxis q;
+  q.center = center;
+  q.step = s;
+  q.first = count(center, -s, -s);
+  const int64_t total = q.first + count(center + s, s, (double)size + 0.9);
+  const int64_t qc = q.first - M / 2;  // find(grid == center) - floor(M/2)
+  q.q0 = qc - (int64_t)M * (int64_t)std::floor((double)qc / M);
+  q.size = std::max<int64_t>(0, total - q.q0) / M * M;
   return q;
 }
 
@@ -1957,8 +1952,8 @@ mlf_status mlf_rectify_size(int64_t H, int64_t W, double x_center, double y_cent
   clear_error();
   if (!out_h || !out_w) return set_error(MLF_ERR_INVALID_ARGUMENT, "NULL argument");
   MLF_CHECK(rectify_check(H, W, x_center, y_center, M, dx));
-  *out_h = (int64_t)rectify_axis(y_center, H, M, dx).size();
-  *out_w = (int64_t)rectify_axis(x_center, W, M, dx).size();
+  *out_h = rectify_axis(y_center, H, M, dx).size;
+  *out_w = rectify_axis(x_center, W, M, dx).size;
   return MLF_OK;
 }
 
@@ -1969,18 +1964,12 @@ mlf_status mlf_rectify_device(mlf_context ctx, const float* d_in, int64_t H, int
   MLF_CHECK(rectify_check(H, W, x_center, y_center, M, dx));
   if (frames < 1 || H > 0x7fffffff || W > 0x7fffffff || frames > 0x7fffffff)
     return set_error(MLF_ERR_INVALID_ARGUMENT, "bad frame count or size");
-  const std::vector<double> yq = rectify_axis(y_center, H, M, dx), xq = rectify_axis(x_center, W, M, dx);
-  if (yq.empty() || xq.empty() || xq.size() > 65535)
-    return set_error(MLF_ERR_INVALID_ARGUMENT, "rectified size %zu x %zu", yq.size(), xq.size());
+  const RectAxis yq = rectify_axis(y_center, H, M, dx), xq = rectify_axis(x_center, W, M, dx);
+  if (yq.size < 1 || xq.size < 1 || xq.size > 65535 || yq.size > 0x7fffffff - 4096)
+    return set_error(MLF_ERR_INVALID_ARGUMENT, "rectified size %lld x %lld", (long long)yq.size, (long long)xq.size);
   MLF_CHECK(ctx_activate(ctx));
-  DevBuf<double> dq;
-  MLF_CHECK(dq.alloc(yq.size() + xq.size()));
-  MLF_HIP(hipMemcpyAsync(dq.ptr, yq.data(), sizeof(double) * yq.size(), hipMemcpyHostToDevice, ctx->stream));
-  MLF_HIP(hipMemcpyAsync(dq.ptr + yq.size(), xq.data(), sizeof(double) * xq.size(), hipMemcpyHostToDevice,
-                         ctx->stream));
-  MLF_LAUNCH(launch_rectify(d_in, (int)H, (int)W, (int)frames, dq.ptr, (int)yq.size(), dq.ptr + yq.size(),
-                            (int)xq.size(), d_out, ctx->stream));
-  MLF_HIP(hipStreamSynchronize(ctx->stream));  // before the grid buffer is released
+  MLF_LAUNCH(launch_rectify(d_in, (int)H, (int)W, (int)frames, yq, xq, d_out, ctx->stream));
+  MLF_HIP(hipStreamSynchronize(ctx->stream));
   return MLF_OK;
 }
 
