@@ -84,8 +84,9 @@ struct DevBuf {
 
 // MATLAB [I1,I2,Z] (column-major) <-> lenslet-blocked [z][L2][L1][s2][s1].
 hipError_t launch_to_blocked(const float* src, float* dst, int n1, int n2, int Z, hipStream_t st);
-hipError_t launch_from_blocked_f32(const float* src, float* dst, int n1, int n2, int Z, hipStream_t st);
-hipError_t launch_from_blocked_f64(const float* src, double* dst, int n1, int n2, int Z, hipStream_t st);
+// Elements [first, first + count) of the MATLAB array, as single or double.
+hipError_t launch_from_blocked(const float* src, void* dst, bool f64, int n1, int n2, size_t first, size_t count,
+                               hipStream_t st);
 hipError_t launch_fill(float* dst, size_t n, float value, hipStream_t st);
 // parts[2k], parts[2k+1] = FP64 sums of (a-b)^2 and b^2 over block k's share.
 hipError_t launch_diff_norms(const float* a, const float* b, size_t n, double* parts, int nblk,

@@ -33,18 +33,19 @@ __global__ void k_to_blocked(const float* __restrict__ src, float* __restrict__ 
   }
 }
 
+// dst[o - first] = element o of the MATLAB array, o in [first, first + count).
 template <typename T>
 __global__ void k_from_blocked(const float* __restrict__ src, T* __restrict__ dst, int n1, int n2,
-                               int Z) {
+                               size_t first, size_t count) {
   const int I1 = n1 * kN, I2 = n2 * kN;
-  const size_t total = (size_t)I1 * I2 * Z;
-  for (size_t o = blockIdx.x * (size_t)blockDim.x + threadIdx.x; o < total;
-       o += (size_t)gridDim.x * blockDim.x) {
+  for (size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x; k < count;
+       k += (size_t)gridDim.x * blockDim.x) {
+    const size_t o = first + k;
     const int p1 = o % I1;
     const size_t r = o / I1;
     const int p2 = r % I2;
     const int z = (int)(r / I2);
-    dst[o] = (T)src[blk_index(p1, p2, z, n1, n2)];
+    dst[k] = (T)src[blk_index(p1, p2, z, n1, n2)];
   }
 }
 
@@ -346,19 +347,14 @@ hipError_t launch_to_blocked(const float* src, float* dst, int n1, int n2, int Z
   return hipGetLastError();
 }
 
-hipError_t launch_from_blocked_f32(const float* src, float* dst, int n1, int n2, int Z,
-                                   hipStream_t st) {
-  const size_t n = (size_t)n1 * n2 * Z * kP;
-  hipLaunchKernelGGL(k_from_blocked<float>, dim3(grid_for(n, 256)), dim3(256), 0, st, src, dst, n1,
-                     n2, Z);
-  return hipGetLastError();
-}
-
-hipError_t launch_from_blocked_f64(const float* src, double* dst, int n1, int n2, int Z,
-                                   hipStream_t st) {
-  const size_t n = (size_t)n1 * n2 * Z * kP;
-  hipLaunchKernelGGL(k_from_blocked<double>, dim3(grid_for(n, 256)), dim3(256), 0, st, src, dst,
-                     n1, n2, Z);
+hipError_t launch_from_blocked(const float* src, void* dst, bool f64, int n1, int n2, size_t first,
+                               size_t count, hipStream_t st) {
+  if (f64)
+    hipLaunchKernelGGL(k_from_blocked<double>, dim3(grid_for(count, 256)), dim3(256), 0, st, src, (double*)dst, n1,
+                       n2, first, count);
+  else
+    hipLaunchKernelGGL(k_from_blocked<float>, dim3(grid_for(count, 256)), dim3(256), 0, st, src, (float*)dst, n1,
+                       n2, first, count);
   return hipGetLastError();
 }
 

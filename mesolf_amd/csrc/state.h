@@ -14,11 +14,21 @@
 #include "internal.h"
 #include "rl_mfma.h"
 
+// Pinned buffers of one thread that reads a volume back (read_volume).
+struct ReadSlot {
+  void* buf[2] = {nullptr, nullptr};
+  hipEvent_t ev[2] = {nullptr, nullptr};
+};
+constexpr int kReadThreads = 8;
+constexpr size_t kReadChunk = (size_t)4 << 20;  // bytes per buffer
+
 struct mlf_context_s {
   int device = 0;
   hipStream_t stream = nullptr;
   mlf::DevBuf<float> mex_kq;  // MEX operator operand scratch, reused across calls (guarded by mu)
   std::mutex mu;
+  ReadSlot read[kReadThreads];  // guarded by read_mu; made on first use, freed with the context
+  std::mutex read_mu;
   int refs = 0;         // live PSFs created on this context
   bool closed = false;  // destroy requested; freed when refs reaches 0
 };
@@ -81,6 +91,8 @@ struct mlf_psf_s {
   mlf::PrecPack pack[mlf::kPrecisions];
   std::vector<std::unique_ptr<mlf::NormTable>> norms[mlf::kPrecisions];
   std::mutex mu;
+  ReadSlot read[kReadThreads];  // guarded by read_mu; made on first use, freed with the context
+  std::mutex read_mu;
   int refs = 0;         // live patches
   bool closed = false;
 };
