@@ -339,7 +339,7 @@ mlf_status mlf_lfm_convolution_vec_device(mlf_context ctx, const float* d_bitmap
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory (code under graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): mlf_lfm_convolution_vec_device with no allocation of
- * any kind.  Its GEMM operand lives in a 64 MiB device array of the library
+ * any kind.  Its GEMM operands live in a 116 MiB device array of the library
  * that every GPU it runs on holds until the process ends; odd kernels are
  * limited to kw <= 257 by that array (MLF_ERR_INVALID_ARGUMENT beyond), even
  * kernels need no scratch.  Results equal mlf_lfm_convolution_vec_device's

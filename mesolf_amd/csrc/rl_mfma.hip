@@ -10,8 +10,8 @@
 //
 // Backprojection + multiplicative update (recon:121-137), per plane z:
 //     B[a, phase] = sum_e R[a - e] * Wt[z][e][phase]             (GEMM, K = taps)
-//   A operand = im2col of the ratio image (LDS window), B operand = the
-//   transposed PSF table (global, taps contiguous).  The backprojection of
+//   One operand = im2col of the ratio image (LDS window), the other = the
+//   transposed PSF table (copied to an LDS ring).  The backprojection of
 //   ones (the normaliser B1) is read from a precomputed table of 1 / B1
 //   (summed and inverted in FP64).
 //

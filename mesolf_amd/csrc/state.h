@@ -51,8 +51,8 @@ mlf_status upload_vec(DevBuf<T>& d, const std::vector<T>& h) {
 // PSF tables re-laid out for the MFMA kernels of one precision.
 struct PrecPack {
   bool built = false;
-  bool tpz = false;                   // forward tables for the Toeplitz kernels (16-bit: [z][e1][e2pad][PHI],
-                                      // FP32: split fragments, k_pack_fwd_split)
+  bool tpz = false;                   // forward tables for the Toeplitz kernels: ready fragments (16-bit:
+                                      // k_pack_fwd_tpz, FP32: split, k_pack_fwd_split)
   DevBuf<uint8_t> fwd, bwd;           // [V][z][e_pad64][PHI], [V][z][kPhiPadBwd][e_pad32]
   int64_t pvf = 0, pvb = 0;           // elements per view
   std::vector<int64_t> woff, boff;    // per-plane element offsets inside a view
