@@ -1454,10 +1454,11 @@ mlf_status mlf_patch_set_volume(mlf_patch p, const float* X) {
 // copy from a temporary array moves and touches them with one thread: reading back after a
 // reconstruction took 32 ms longer for 468 MB (101 x 101 x 51: 834 -> 802 ms
 // in all), 13 ms for 165 MB (81 x 73 x 31: 135 -> 122 ms).  Smaller volumes take
-// that copy: a context that reads one of them once would pay more for pinning
-// the 64 MB of buffers than it saves.  Returns false, with nothing pending, if
+// that copy: pinning and freeing the 64 MB of buffers takes 5 ms of a context's life,
+// what one read of 64 MB saves (98 MB: 10.1 -> 2.7 ms, 3.4 the first time and
+// 2 more to free; 32 MB: 3.3 -> 1.2, 5.1 the first time).  Returns false, with nothing pending, if
 // the buffers are not to be had.
-constexpr size_t kReadMin = (size_t)32 << 20;
+constexpr size_t kReadMin = (size_t)64 << 20;
 
 static bool read_volume(mlf_context ctx, const float* X, void* out, bool f64, int n1, int n2, size_t numel) {
   const size_t es = f64 ? 8 : 4, per = kReadChunk / es;

@@ -416,7 +416,7 @@ __global__ __launch_bounds__(kThreads) void k_rectify(const float* __restrict__ 
 // movie once instead of twice, the first pass takes the maximum along, and the
 // last round's Y t, the detrend, the smoothing and the std image share one
 // read with no detrended movie in memory: 6 reads of the movie for 5 rounds
-// instead of 13 and a write.  765 x 750 x 400: 2.26 ms a call (the passes above:
+// instead of 13 and a write.  765 x 750 x 400: 2.11 ms a call (the passes above:
 // 4.15), 0.24 ms per round (3.8 TB/s; k_r1_tdot + k_r1_sdot 0.48).  A workgroup
 // requests its next tile into registers before it computes on the one in LDS
 // (tiles of 64 pixels x 400 frames leave room for one workgroup per CU; 1024

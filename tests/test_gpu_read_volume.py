@@ -1,5 +1,5 @@
 """Reading volumes back below and above the size from which several threads
-copy them out (32 MB, chunks of 4 MB): the values that were set, exactly."""
+copy them out (64 MiB, chunks of 4 MiB): the values that were set, exactly."""
 import threading
 
 import numpy as np
@@ -20,8 +20,9 @@ def psf():
     ctx.close()
 
 
-# float32 MiB: 0.03, 32.006 (a last chunk of few elements), 31.996 and 47.9; float64 twice that
-@pytest.mark.parametrize("n1,n2", [(3, 4), (113, 110), (109, 114), (131, 142)])
+# float32 MiB: 0.03, 32.006, 31.996 (their float64: just above, with a last chunk of few
+# elements, and just below the line) and 65.9
+@pytest.mark.parametrize("n1,n2", [(3, 4), (113, 110), (109, 114), (160, 160)])
 def test_set_and_read_back(psf, n1, n2):
     p = mesolf_amd.Patch(psf, n1, n2, "fp32")
     X = np.random.default_rng(n1).random(p.shape).astype(np.float32)
@@ -32,7 +33,7 @@ def test_set_and_read_back(psf, n1, n2):
 
 
 def test_two_threads_read_at_once(psf):
-    patches = [mesolf_amd.Patch(psf, 120, 111 + k, "fp32") for k in range(2)]
+    patches = [mesolf_amd.Patch(psf, 170, 160 + k, "fp32") for k in range(2)]
     want = [np.random.default_rng(k).random(p.shape).astype(np.float32) for k, p in enumerate(patches)]
     for p, x in zip(patches, want):
         p.set_volume(x)
