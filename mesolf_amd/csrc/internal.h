@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "../../include/mesolf.h"
+#include "mex_marks.h"
 
 namespace mlf {
 
@@ -177,37 +178,36 @@ hipError_t launch_mex_conv(const float* in, int64_t W, int64_t H, int64_t n, con
                            float* out, hipStream_t st);
 // MFMA forms of the MEX operator for odd kw (clipping == zero padding): the
 // BF16 split form (mex_split.hip) where its 32-bit offsets reach, with the FP32
-// form behind it for bitmaps or kernels holding values that it leaves, or the
-// FP32 form alone.  One call has one scratch of mex_scratch_floats(kw) floats,
-// whose first kMexFlagFloats floats were zero when it was allocated and are
-// written by these launches only.
+// form behind it for the bitmaps and kernel sets holding values that it leaves, or
+// the FP32 form alone.  A call of the split form has a scratch of
+// mex_scratch_floats(kw, images) floats, whose first mex_mark_words(images)
+// were zero when it was allocated and are written by these launches only.
 constexpr int kMexMfmaMaxKw = 511;
-constexpr int kMexFlagFloats = 64;
-size_t mex_scratch_floats(int kw);
+size_t mex_mark_words(int64_t images);
+size_t mex_scratch_floats(int kw, int64_t images);
+bool mex_split_takes(int64_t W, int64_t H, int64_t images, int kw);
 struct MexCall {
-  float* scratch = nullptr;     // operand table of the kernel set in use
   int kw = 0;
+  int64_t images = 0;           // bitmaps of the call
   const float* scan = nullptr;  // bitmaps still to be looked through
-  size_t nscan = 0;
-  int* flag = nullptr;          // null: the FP32 form alone
-  int gen = 0;                  // number of the call, stored in *flag to leave it to the FP32 form
+  void* table = nullptr;        // the split form's operand of the kernel set in use
+  MexMarks marks;               // none: the FP32 form alone
+  int sets = 0;                 // kernel sets used so far
 };
-// A call on `images` bitmaps [W, H] at `in`.
-MexCall mex_begin(int64_t W, int64_t H, int64_t images, int kw, const float* in, float* scratch);
+// A call on `images` bitmaps [W, H] at `in`.  scratch (null: the FP32 form alone)
+// has room for the marks of `room` >= images bitmaps.
+MexCall mex_begin(int64_t images, int kw, const float* in, float* scratch, int64_t room);
 // out[j] = MEX(in[j], K) for j < n, or with lists out[dst[j]] += MEX(in[src[j]], K)
-// (dst distinct within a launch); new_kernel: K differs from the launch before.
+// (dst distinct within a launch); new_kernel: K differs from the launch before;
+// last: the call's last launch.
 hipError_t launch_mex_mfma(MexCall& c, const float* in, int64_t W, int64_t H, int64_t n, const float* K,
-                           bool new_kernel, const int32_t* src, const int32_t* dst, float* out,
+                           bool new_kernel, bool last, const int32_t* src, const int32_t* dst, float* out,
                            hipStream_t st);
 // The split form (mex_split.hip).
-bool mex_split_takes(int64_t W, int64_t H, int64_t images, int kw);
 size_t mex_split_bytes(int kw);
-int mex_next_call();
-hipError_t launch_mex_split_prep(const float* K, int kw, void* Bt, const float* scan, size_t nscan, int* flag,
-                                 int gen, hipStream_t st);
-hipError_t launch_mex_split(const float* in, int64_t W, int64_t H, int64_t n, const void* Bt, int kw,
-                            const int32_t* src, const int32_t* dst, float* out, const int* flag, int gen,
-                            hipStream_t st);
+hipError_t launch_mex_split_prep(const MexCall& c, const float* K, size_t image, hipStream_t st);
+hipError_t launch_mex_split(const MexCall& c, const float* in, int64_t W, int64_t H, int64_t n,
+                            const int32_t* src, const int32_t* dst, float* out, hipStream_t st);
 // Device address of the no-allocation MEX scratch on `device` (the device
 // must be current), resolved once per device at context creation.
 mlf_status noalloc_scratch_init(int device);

@@ -5,8 +5,6 @@
 // h = kw/2, zero outside the bitmap; the tap window is clipped exactly as
 // mex_lfm_convolution_vec.cu:55-78 clips it (for even kw the last column/row
 // tap is dropped near the right/bottom edge).
-#include <algorithm>
-
 #include "internal.h"
 
 namespace mlf {
@@ -122,15 +120,13 @@ __global__ __launch_bounds__(kTileX* kTileY) void k_mex_conv_segments(
 // i.e. M = lenslet columns i, N = the 15 phases p (padded to 16), K = (ky, t).
 // A workgroup takes one output row and kMexImg images (kMexImgW per wave) over
 // 32 lenslet columns (two M-tiles).  Per chunk of kMexCK input rows it stages
-// the images' rows and the chunk's Kq rows (T4 x 16 floats per row, read with
-// 16-byte loads, shared by every wave) in LDS; each Kq fragment read from LDS
+// the images' rows and the chunk's Kq rows (T4 x 16 floats per row, gathered from K,
+// shared by every wave) in LDS; each Kq fragment read from LDS
 // feeds the MFMAs of both M-tiles.  This is the form for values that the BF16
 // split form (mex_split.hip) leaves and for bitmaps beyond its 32-bit offsets.
-// Measured on the seed-library loop
-// (396 x 396, kw = 241): 7.37 s with these settings (11.8 + 16 KB of LDS per
-// workgroup at kw = 241); Kq fragments from L2 instead: 9.60 s with one image
-// per wave, 8.27 s with two (three 9.52, four 10.76 s); two input rows per
-// chunk, Kq from L2: 10.59 s.
+// A call whose 96 bitmaps of 396 x 396 are all marked (kw = 241) takes 27.9 ms, one
+// with a single marked bitmap 12.7 ms; Kq rows copied from a prepared table,
+// which takes a launch and 59 MB of scratch of its own, 27.0 ms.
 typedef float mex_floatx4 __attribute__((ext_vector_type(4)));
 constexpr int kMexImgW = 1;
 constexpr int kMexImg = 8 * kMexImgW;
@@ -138,35 +134,28 @@ constexpr int kMexThreads = 64 * kMexImg / kMexImgW;  // one wave per kMexImgW i
 constexpr int kMexCK = 1;
 constexpr int kMexCols = 32;  // lenslet columns per workgroup (2 M-tiles)
 
-// flag != null: the launch does its work only if *flag == gen (the split form
-// of mex_split.hip has left the call to this one).
-__global__ void k_mex_kq(const float* __restrict__ K, int kw, int T4, float* __restrict__ Kq,
-                         const int* __restrict__ flag, int gen) {
-  if (flag && *flag != gen) return;
-  const size_t total = (size_t)kN * kw * T4 * 16;
-  for (size_t o = blockIdx.x * (size_t)blockDim.x + threadIdx.x; o < total;
-       o += (size_t)gridDim.x * blockDim.x) {
-    const int p = (int)(o % 16);
-    const int t = (int)((o / 16) % T4);
-    const int ky = (int)((o / (16 * (size_t)T4)) % kw);
-    const int q = (int)(o / (16 * (size_t)T4 * kw));
-    const int kx = t - p;
-    Kq[o] = (p < kN && kx >= 0 && kx < kw)
-                ? K[(size_t)kx + (size_t)kw * ky + (size_t)kw * kw * (p + kN * q)]
-                : 0.f;
-  }
-}
-
 // List mode (seed-library batches): image j of the launch is input image
 // src[j] and its projection is added to output image dst[j] (the dst of one
 // launch are distinct, so no two workgroups add to the same pixel).
+// With marks, the launch makes the images that k_mex_split has left to it.
 __global__ __launch_bounds__(kMexThreads) void k_mex_mfma(const float* __restrict__ in, int W, int H, int n,
-                                                  const float* __restrict__ Kq, int kw, int T4,
+                                                  const float* __restrict__ K, int kw, int T4,
                                                   float* __restrict__ out,
                                                   const int32_t* __restrict__ src,
-                                                  const int32_t* __restrict__ dst,
-                                                  const int* __restrict__ flag, int gen) {
-  if (flag && *flag != gen) return;
+                                                  const int32_t* __restrict__ dst, MexMarks marks,
+                                                  int set, bool last) {
+  uint32_t call = 0;
+  bool all = true;
+  if (marks.w) {
+    call = *marks.current();
+    if (last && threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) *marks.finished() = call;
+    if (*marks.any() != call) return;
+    all = marks.set_marked(call, set);
+    bool some = all;
+    for (int i = blockIdx.y * kMexImg; i < min((int)(blockIdx.y + 1) * kMexImg, n); ++i)
+      some = some || marks.image_marked(call, src ? src[i] : i);
+    if (!some) return;
+  }
   extern __shared__ float xs[];  // [kMexCK][kMexImg][XL], then the chunk's Kq rows [kMexCK][T4][16]
   const int y = blockIdx.x, ng = blockIdx.y, ib = blockIdx.z;
   const int q = y % kN, h = kw / 2;
@@ -178,7 +167,11 @@ __global__ __launch_bounds__(kMexThreads) void k_mex_mfma(const float* __restric
   mex_floatx4 acc[kMexImgW][2];
 #pragma unroll
   for (int m = 0; m < kMexImgW; ++m) acc[m][0] = acc[m][1] = mex_floatx4{0.f, 0.f, 0.f, 0.f};
-  const float* Kqq = Kq + (size_t)q * kw * T4 * 16;
+  // this thread's phase of the Kq rows (the 16th column repeats the 15th: its
+  // sums are dropped), elements t = tid / 16 + 32 i
+  static_assert(kMexThreads % 16 == 0, "one phase per thread");
+  const int kp = tid & 15, kt = tid >> 4;
+  const float* Kp = K + (size_t)kw * kw * (min(kp, kN - 1) + kN * q);
   for (int c0 = 0; c0 < kw; c0 += kMexCK) {
     __syncthreads();  // previous chunk consumed
     for (int o = tid; o < kMexCK * kMexImg * XL; o += kMexThreads) {
@@ -191,11 +184,15 @@ __global__ __launch_bounds__(kMexThreads) void k_mex_mfma(const float* __restric
         v = in[(size_t)(src ? src[nn] : nn) * W * H + (size_t)r * W + x];
       xs[o] = v;
     }
-    {
-      float* Bs = xs + kMexCK * kMexImg * XL;
-      const mex_floatx4* src4 = reinterpret_cast<const mex_floatx4*>(Kqq + (size_t)c0 * T4 * 16);
-      for (int o = tid; o < kMexCK * T4 * 4; o += kMexThreads)
-        reinterpret_cast<mex_floatx4*>(Bs)[o] = (c0 + o / (T4 * 4) < kw) ? src4[o] : mex_floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int kk = 0; kk < kMexCK && c0 + kk < kw; ++kk) {
+      float* Bs = xs + kMexCK * kMexImg * XL + kk * T4 * 16 + kp;
+      const float* row = Kp + (size_t)kw * (c0 + kk);
+#pragma unroll 4
+      for (int t = kt; t < T4; t += kMexThreads / 16) {
+        const unsigned kx = t - kp;
+        const float v = row[min(kx, (unsigned)kw - 1)];
+        Bs[t * 16] = kx < (unsigned)kw ? v : 0.f;
+      }
     }
     __syncthreads();
     for (int kk = 0; kk < kMexCK && c0 + kk < kw; ++kk) {
@@ -217,6 +214,7 @@ __global__ __launch_bounds__(kMexThreads) void k_mex_mfma(const float* __restric
   for (int m = 0; m < kMexImgW; ++m) {
     const int img = img0 + m;
     if (img >= n) break;
+    if (!all && !marks.image_marked(call, src ? src[img] : img)) continue;
     float* o = out + (size_t)(dst ? dst[img] : img) * W * H + (size_t)y * W;
 #pragma unroll
     for (int it = 0; it < 2; ++it)
@@ -233,21 +231,9 @@ __global__ __launch_bounds__(kMexThreads) void k_mex_mfma(const float* __restric
 
 }  // namespace
 
-static size_t mex_kq_floats(int kw) {
-  const int T4 = (kw + kN - 1 + 3) / 4 * 4;
-  return (size_t)kN * kw * T4 * 16;
-}
-
-static hipError_t launch_kq(const float* K, int kw, float* Kq, const int* flag, int gen, hipStream_t st) {
-  const int T4 = (kw + kN - 1 + 3) / 4 * 4;
-  hipLaunchKernelGGL(k_mex_kq, dim3(1024), dim3(256), 0, st, K, kw, T4, Kq, flag, gen);
-  return hipGetLastError();
-}
-
-static hipError_t launch_mfma(const float* in, int64_t W, int64_t H, int64_t n, const float* Kq, int kw,
-                              const int32_t* src, const int32_t* dst, float* out, const int* flag, int gen,
-                              hipStream_t st) {
-  const int T4 = (kw + kN - 1 + 3) / 4 * 4;
+static hipError_t launch_mfma(const MexCall& c, const float* in, int64_t W, int64_t H, int64_t n, const float* K,
+                              bool last, const int32_t* src, const int32_t* dst, float* out, hipStream_t st) {
+  const int T4 = (c.kw + kN - 1 + 3) / 4 * 4;
   const int XL = kN * kMexCols + T4;
   const size_t shmem = sizeof(float) * kMexCK * (kMexImg * XL + T4 * 16);
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_mex_mfma),
@@ -255,47 +241,41 @@ static hipError_t launch_mfma(const float* in, int64_t W, int64_t H, int64_t n, 
   if (attr != hipSuccess) return attr;
   dim3 grid((unsigned)H, (unsigned)((n + kMexImg - 1) / kMexImg),
             (unsigned)((W / kN + 1 + kMexCols - 1) / kMexCols));
-  hipLaunchKernelGGL(k_mex_mfma, grid, dim3(kMexThreads), shmem, st, in, (int)W, (int)H, (int)n, Kq, kw, T4,
-                     out, src, dst, flag, gen);
+  hipLaunchKernelGGL(k_mex_mfma, grid, dim3(kMexThreads), shmem, st, in, (int)W, (int)H, (int)n, K, c.kw, T4,
+                     out, src, dst, c.marks, c.sets, last);
   return hipGetLastError();
 }
 
-size_t mex_scratch_floats(int kw) {
-  return kMexFlagFloats + std::max(mex_kq_floats(kw), mex_split_bytes(kw) / sizeof(float));
-}
+size_t mex_mark_words(int64_t images) { return kMexHeadWords + ((size_t)images + 63) / 64 * 64; }
 
-MexCall mex_begin(int64_t W, int64_t H, int64_t images, int kw, const float* in, float* scratch) {
+size_t mex_scratch_floats(int kw, int64_t images) { return mex_mark_words(images) + mex_split_bytes(kw) / sizeof(float); }
+
+MexCall mex_begin(int64_t images, int kw, const float* in, float* scratch, int64_t room) {
   MexCall c;
-  c.scratch = scratch + kMexFlagFloats;
   c.kw = kw;
-  c.scan = in;
-  c.nscan = (size_t)W * H * images;
-  if (mex_split_takes(W, H, images, kw)) {
-    c.flag = reinterpret_cast<int*>(scratch);
-    c.gen = mex_next_call();
+  c.images = images;
+  if (scratch) {
+    c.scan = in;
+    c.table = scratch + mex_mark_words(room);
+    c.marks.w = reinterpret_cast<uint32_t*>(scratch);
   }
   return c;
 }
 
 hipError_t launch_mex_mfma(MexCall& c, const float* in, int64_t W, int64_t H, int64_t n, const float* K,
-                           bool new_kernel, const int32_t* src, const int32_t* dst, float* out,
+                           bool new_kernel, bool last, const int32_t* src, const int32_t* dst, float* out,
                            hipStream_t st) {
-  if (c.flag) {
+  if (c.marks.w) {
     if (new_kernel) {
-      const hipError_t e = launch_mex_split_prep(K, c.kw, c.scratch, c.scan, c.nscan, c.flag, c.gen, st);
+      ++c.sets;
+      const hipError_t e = launch_mex_split_prep(c, K, (size_t)W * H, st);
       if (e != hipSuccess) return e;
-      c.nscan = 0;  // the bitmaps are looked through once per call
+      c.scan = nullptr;  // the bitmaps are looked through once per call
     }
-    const hipError_t e = launch_mex_split(in, W, H, n, c.scratch, c.kw, src, dst, out, c.flag, c.gen, st);
+    const hipError_t e = launch_mex_split(c, in, W, H, n, src, dst, out, st);
     if (e != hipSuccess) return e;
   }
-  // the whole call without the split form, and behind it for values that it
-  // leaves (the operand then takes the place of the split form's table)
-  if (new_kernel) {
-    const hipError_t e = launch_kq(K, c.kw, c.scratch, c.flag, c.gen, st);
-    if (e != hipSuccess) return e;
-  }
-  return launch_mfma(in, W, H, n, c.scratch, c.kw, src, dst, out, c.flag, c.gen, st);
+  return launch_mfma(c, in, W, H, n, K, last, src, dst, out, st);
 }
 
 hipError_t launch_mex_conv_segments(const float* in, int64_t W, int64_t H, const int32_t* plane,

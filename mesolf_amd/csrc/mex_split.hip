@@ -28,10 +28,10 @@
 //
 // A value that BF16 cannot round without overflow (infinities, NaN, the last
 // 2^-9 below FLT_MAX) would turn the products of its parts into NaN: the prep
-// kernel looks for one and stores the call's number in *flag, and then this
-// kernel leaves the call to k_mex_mfma, launched behind it.
+// kernel marks the bitmap or the kernel set that holds one (mex_marks.h), and this
+// kernel leaves a marked bitmap, or every bitmap of a marked set, to k_mex_mfma,
+// launched behind it.  The other bitmaps of the call stay here.
 #include <algorithm>
-#include <atomic>
 
 #include "internal.h"
 
@@ -77,13 +77,15 @@ struct SplitGeo {
 };
 
 // Fragment table Bt[q][ky][ks][part][lane][8]: lane (p = lane % 16, lg = lane / 16)
-// holds slots 8 (lg % 2) .. + 7 of lenslet L = 2 ks + lg / 2.  The blocks past
-// nbt look through `nscan` input values.
+// holds slots 8 (lg % 2) .. + 7 of lenslet L = 2 ks + lg / 2.  Past the nbt blocks that
+// make it, nbi blocks look through each bitmap of `image` values.
 __global__ __launch_bounds__(256) void k_mex_split_prep(const float* __restrict__ K, int kw, int b, int nks,
                                                         uintx4* __restrict__ Bt, int nbt,
-                                                        const float* __restrict__ scan, size_t nscan,
-                                                        int* __restrict__ flag, int gen) {
+                                                        const float* __restrict__ scan, size_t image, int nbi,
+                                                        MexMarks marks, int set) {
+  const uint32_t call = *marks.finished() + 1;
   bool bad = false;
+  int img = -1;  // bitmap of this block, or the kernel set
   if ((int)blockIdx.x < nbt) {
     const size_t total = (size_t)kN * kw * nks * 64;
     for (size_t o = blockIdx.x * (size_t)256 + threadIdx.x; o < total; o += (size_t)nbt * 256) {
@@ -109,16 +111,20 @@ __global__ __launch_bounds__(256) void k_mex_split_prep(const float* __restrict_
       for (int k = 0; k < 3; ++k) Bt[(blk * 3 + k) * 64 + lane] = uintx4{w[0][k], w[1][k], w[2][k], w[3][k]};
     }
   } else {
-    const size_t nb = gridDim.x - nbt;
-    const size_t step = nb * 256;
-    size_t o = (blockIdx.x - nbt) * (size_t)256 + threadIdx.x;
-    for (; o + 3 * step < nscan; o += 4 * step) {
-      const float v0 = scan[o], v1 = scan[o + step], v2 = scan[o + 2 * step], v3 = scan[o + 3 * step];
+    img = (int)(blockIdx.x - nbt) / nbi;
+    const float* s = scan + img * image;
+    const size_t step = (size_t)nbi * 256;
+    size_t o = ((blockIdx.x - nbt) % nbi) * (size_t)256 + threadIdx.x;
+    for (; o + 3 * step < image; o += 4 * step) {
+      const float v0 = s[o], v1 = s[o + step], v2 = s[o + 2 * step], v3 = s[o + 3 * step];
       bad = bad || too_large(v0) || too_large(v1) || too_large(v2) || too_large(v3);
     }
-    for (; o < nscan; o += step) bad = bad || too_large(scan[o]);
+    for (; o < image; o += step) bad = bad || too_large(s[o]);
   }
-  if (bad) *flag = gen;
+  if (!bad) return;
+  *marks.any() = call;
+  if (img < 0) *marks.set() = MexMarks::set_mark(call, set);
+  else *marks.image(img) = call;
 }
 
 // WM waves along M times WK groups that share the input rows (row j goes to
@@ -143,13 +149,16 @@ template <int WM, int WK, int MT, int G, int SPB>
 __global__ __launch_bounds__(64 * WM * WK) void k_mex_split(const float* __restrict__ in, SplitGeo g,
                                                             const uintx4* __restrict__ Bt, float* __restrict__ out,
                                                             const int32_t* __restrict__ src,
-                                                            const int32_t* __restrict__ dst,
-                                                            const int* __restrict__ flag, int gen) {
+                                                            const int32_t* __restrict__ dst, MexMarks marks,
+                                                            int set) {
   using S = SplitShape<WM, WK, MT, G, SPB>;
   constexpr int NTH = 64 * WM;  // threads of a group
   constexpr int NU = (S::kSlots * 8 + NTH - 1) / NTH;  // pixel pairs staged per thread and row
   extern __shared__ __align__(16) char sm[];
-  if (uni(*flag) == gen) return;
+  const uint32_t call = uni(*marks.finished()) + 1;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *marks.current() = call;
+  const bool any = (uint32_t)uni(*marks.any()) == call;
+  if (any && marks.set_marked(call, set)) return;
   const int W = g.W, H = g.H, nL = g.nL;
   const int tid = threadIdx.x, lane = tid & 63, w = uni(tid >> 6), lr = lane & 15, lg = lane >> 4;
   const int wk = w / WM, wm = w % WM, gt = tid - wk * NTH;
@@ -164,6 +173,12 @@ __global__ __launch_bounds__(64 * WM * WK) void k_mex_split(const float* __restr
   const int yg = (rank & 1) ? g.nyg / 2 - (rank + 1) / 2 : g.nyg / 2 + rank / 2;
   const int y0 = G * yg;
   const int M0 = mb * S::kRows, NC = g.n * nL;
+  if (any) {  // nothing to do if every bitmap of the block is marked
+    bool live = false;
+    for (int i = M0 / nL; i <= (min(M0 + S::kRows, NC) - 1) / nL; ++i)
+      live = live || !marks.image_marked(call, src ? src[i] : i);
+    if (!live) return;
+  }
 
   // staged pairs: pixels 15 lens + 2 k, + 1 (k = 7: pixel 14 and the zero slot)
   const int pk8 = gt & 7;
@@ -317,7 +332,7 @@ __global__ __launch_bounds__(64 * WM * WK) void k_mex_split(const float* __restr
       const int c = M0 + 16 * (wm * MT + m) + 4 * lg + j;
       if (c >= NC) continue;
       const int img = c / nL, x = kN * (c - img * nL) + lr;
-      if (x >= W) continue;
+      if (x >= W || (any && marks.image_marked(call, src ? src[img] : img))) continue;
       float* o = out + (size_t)(dst ? dst[img] : img) * W * H + x;
 #pragma unroll
       for (int i = 0; i < G; ++i) {
@@ -328,7 +343,7 @@ __global__ __launch_bounds__(64 * WM * WK) void k_mex_split(const float* __restr
     }
 }
 
-typedef void (*SplitKernel)(const float*, SplitGeo, const uintx4*, float*, const int32_t*, const int32_t*, const int*,
+typedef void (*SplitKernel)(const float*, SplitGeo, const uintx4*, float*, const int32_t*, const int32_t*, MexMarks,
                             int);
 struct SplitVariant {
   SplitKernel fn;
@@ -360,21 +375,17 @@ bool mex_split_takes(int64_t W, int64_t H, int64_t images, int kw) {
 
 size_t mex_split_bytes(int kw) { return (size_t)kN * kw * split_nks(kw) * 3 * 1024; }
 
-int mex_next_call() {
-  static std::atomic<int> calls{0};
-  return ++calls;
-}
-
-hipError_t launch_mex_split_prep(const float* K, int kw, void* Bt, const float* scan, size_t nscan, int* flag,
-                                 int gen, hipStream_t st) {
+hipError_t launch_mex_split_prep(const MexCall& c, const float* K, size_t image, hipStream_t st) {
   int a, b;
-  split_lenslets(kw, &a, &b);
-  const int nks = split_nks(kw);
-  const size_t total = (size_t)kN * kw * nks * 64;
+  split_lenslets(c.kw, &a, &b);
+  const int nks = split_nks(c.kw);
+  const size_t total = (size_t)kN * c.kw * nks * 64;
   const int nbt = (int)std::min<size_t>((total + 255) / 256, 4096);
-  const int nbs = nscan ? (int)std::min<size_t>((nscan + 1023) / 1024, 2048) : 0;
-  hipLaunchKernelGGL(k_mex_split_prep, dim3(nbt + nbs), dim3(256), 0, st, K, kw, b, nks, (uintx4*)Bt, nbt, scan,
-                     nscan, flag, gen);
+  const int nbi = (int)std::max<size_t>(1, std::min<size_t>((image + 1023) / 1024, 2048 / c.images));
+  const int64_t grid = nbt + (c.scan ? nbi * c.images : 0);
+  if (grid > 0x7fffffff) return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL(k_mex_split_prep, dim3((unsigned)grid), dim3(256), 0, st, K, c.kw, b, nks, (uintx4*)c.table, nbt,
+                     c.scan, image, nbi, c.marks, c.sets);
   return hipGetLastError();
 }
 
@@ -384,9 +395,9 @@ hipError_t launch_mex_split_prep(const float* K, int kw, void* Bt, const float* 
 // M-tiles in blocks of 24: 693 workgroups, 2.7 rounds; blocks of 32 would pad
 // them by a fifth), 17 bitmaps <2, 4, 2, 2, 1> or <4, 2, 2, 4, 1>, one small
 // bitmap <1, 8, 1, 1, 1> (eight waves share the kernel's rows).
-hipError_t launch_mex_split(const float* in, int64_t W, int64_t H, int64_t n, const void* Bt, int kw,
-                            const int32_t* src, const int32_t* dst, float* out, const int* flag, int gen,
-                            hipStream_t st) {
+hipError_t launch_mex_split(const MexCall& c, const float* in, int64_t W, int64_t H, int64_t n,
+                            const int32_t* src, const int32_t* dst, float* out, hipStream_t st) {
+  const int kw = c.kw;
   static const SplitVariant variants[] = {
       variant<8, 1, 4, 4, 2>(), variant<8, 1, 3, 4, 2>(), variant<8, 1, 2, 4, 2>(), variant<4, 2, 4, 4, 1>(),
       variant<4, 2, 3, 4, 1>(), variant<4, 2, 2, 4, 1>(), variant<2, 4, 2, 2, 1>(), variant<1, 8, 2, 1, 1>(),
@@ -429,7 +440,7 @@ hipError_t launch_mex_split(const float* in, int64_t W, int64_t H, int64_t n, co
   const int64_t grid = (int64_t)((g.nyg + 7) / 8) * 8 * g.nmb;
   if (grid > 0x7fffffff) return hipErrorInvalidConfiguration;
   hipLaunchKernelGGL(best->fn, dim3((unsigned)grid), dim3(64 * best->wm * best->wk), best->lds, st, in, g,
-                     (const uintx4*)Bt, out, src, dst, flag, gen);
+                     (const uintx4*)c.table, out, src, dst, c.marks, c.sets);
   return hipGetLastError();
 }
 

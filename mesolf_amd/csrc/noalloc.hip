@@ -1,10 +1,10 @@
 // MEX operator without device allocation: mlf_lfm_convolution_vec_noalloc.
 //
-// mlf_lfm_convolution_vec_device keeps the MFMA forms' kernel operand
-// (mex_scratch_floats(kw) floats, 100 MB at the production kernel width 241) in
-// a buffer the library allocates on first use.  Callers that cannot allocate
-// device memory (code under graph capture, tight serving loops) use this
-// variant instead: the operand lives in `scratch`, a file-scope device array of
+// mlf_lfm_convolution_vec_device keeps the split form's kernel operand and the
+// marks of its bitmaps (mex_scratch_floats(kw, n) floats, 100 MB at the production
+// kernel width 241) in a buffer the library allocates on first use.  Callers that
+// cannot allocate device memory (code under graph capture, tight serving loops)
+// use this variant instead: they live in `scratch`, a file-scope device array of
 // kNoAllocFloats floats (116 MiB, odd kw <= 257) that every GPU the library
 // runs on holds until the process ends.
 //
@@ -13,10 +13,10 @@
 // context creation (mlf_context_create, with that device current) and only
 // that address is passed to kernels.  Every call on one GPU shares its
 // array, which keeps the last call's contents: the operand build writes every
-// element a launch reads, and the flag words at its start (zero at load) hold
-// numbers of past calls, which no later call has; so nothing needs clearing.  Calls on one context
-// are ordered by its stream; calls that overlap on one GPU from different
-// contexts race on the array.
+// element a launch reads, and the marks (zero at load) hold the numbers of the calls
+// that made them, counted on the device (mex_marks.h); so nothing needs
+// clearing.  Calls on one context are ordered by its stream; calls that overlap
+// on one GPU from different contexts race on the array.
 #include <mutex>
 
 #include "internal.h"
@@ -27,6 +27,7 @@ namespace mlf {
 namespace {
 constexpr size_t kNoAllocFloats = (size_t)29 << 20;  // 116 MiB
 constexpr int kNoAllocMaxKw = 257;                   // largest odd kw whose operand fits
+constexpr int64_t kNoAllocImages = 65536;            // bitmaps whose marks fit beside it
 constexpr int kMaxDevices = 64;
 
 static __device__ __align__(256) float scratch[kNoAllocFloats];
@@ -76,17 +77,17 @@ extern "C" mlf_status mlf_lfm_convolution_vec_noalloc(mlf_context ctx, const flo
                      (long long)kw, kNoAllocMaxKw, kNoAllocFloats * sizeof(float));
   MLF_CHECK(ctx_activate(ctx));
   if (kw % 2 == 1) {
-    // resolved by mlf_context_create on this device
-    float* kq = nullptr;
-    {
+    float* mem = nullptr;
+    if (mex_split_takes(width, height, n, (int)kw)) {
+      // resolved by mlf_context_create on this device
       std::lock_guard<std::mutex> lk(g_scratch_mu);
-      kq = ctx->device >= 0 && ctx->device < kMaxDevices ? g_scratch_ptr[ctx->device] : nullptr;
+      mem = ctx->device >= 0 && ctx->device < kMaxDevices ? g_scratch_ptr[ctx->device] : nullptr;
+      if (!mem) return set_error(MLF_ERR_INTERNAL, "scratch of device %d not resolved", ctx->device);
+      if (n > kNoAllocImages || mex_scratch_floats((int)kw, kNoAllocImages) > kNoAllocFloats)
+        return set_error(MLF_ERR_INTERNAL, "scratch too small for kw %lld", (long long)kw);
     }
-    if (!kq) return set_error(MLF_ERR_INTERNAL, "scratch of device %d not resolved", ctx->device);
-    if (mex_scratch_floats((int)kw) > kNoAllocFloats)
-      return set_error(MLF_ERR_INTERNAL, "scratch too small for kw %lld", (long long)kw);
-    MexCall c = mex_begin(width, height, n, (int)kw, d_bitmap, kq);
-    MLF_LAUNCH(launch_mex_mfma(c, d_bitmap, width, height, n, d_kernels, true, nullptr, nullptr, d_out,
+    MexCall c = mex_begin(n, (int)kw, d_bitmap, mem, kNoAllocImages);
+    MLF_LAUNCH(launch_mex_mfma(c, d_bitmap, width, height, n, d_kernels, true, true, nullptr, nullptr, d_out,
                                ctx->stream));
     return MLF_OK;
   }

@@ -1930,13 +1930,24 @@ mlf_status mlf_recon_phase_space(const float* lfimg, int64_t I1, int64_t I2, con
   return MLF_OK;
 }
 
-// Operand scratch of the context for kernels kw wide (called with ctx->mu held).
-static mlf_status ctx_mex_scratch(mlf_context ctx, int kw) {
-  const size_t need = mex_scratch_floats(kw);
-  if (ctx->mex_kq.count >= need) return MLF_OK;
-  MLF_HIP(hipStreamSynchronize(ctx->stream));  // earlier calls may still read it
-  MLF_CHECK(ctx->mex_kq.alloc(need));
-  MLF_LAUNCH(launch_fill(ctx->mex_kq.ptr, kMexFlagFloats, 0.f, ctx->stream));
+// Begins a MEX call of odd kw on `images` bitmaps (called with ctx->mu held):
+// the context's scratch is grown to it.
+static mlf_status ctx_mex_begin(mlf_context ctx, int64_t W, int64_t H, int64_t images, int kw, const float* in,
+                                MexCall* c) {
+  if (!mex_split_takes(W, H, images, kw)) {
+    *c = mex_begin(images, kw, in, nullptr, 0);
+    return MLF_OK;
+  }
+  const int64_t room = std::max<int64_t>(std::max(images, ctx->mex_room), 4096);
+  const size_t need = mex_scratch_floats(kw, room);
+  if (ctx->mex_scratch.count < need || room != ctx->mex_room) {
+    MLF_HIP(hipStreamSynchronize(ctx->stream));  // earlier calls may still read it
+    ctx->mex_room = 0;
+    MLF_CHECK(ctx->mex_scratch.alloc(std::max(need, ctx->mex_scratch.count)));
+    MLF_LAUNCH(launch_fill(ctx->mex_scratch.ptr, mex_mark_words(room), 0.f, ctx->stream));
+    ctx->mex_room = room;
+  }
+  *c = mex_begin(images, kw, in, ctx->mex_scratch.ptr, room);
   return MLF_OK;
 }
 
@@ -1957,9 +1968,9 @@ mlf_status mlf_lfm_convolution_vec_device(mlf_context ctx, const float* d_bitmap
   if (kw % 2 == 1 && kw <= kMexMfmaMaxKw) {
     // odd kernels: the MFMA form; its operand scratch lives in the context
     std::lock_guard<std::mutex> lk(ctx->mu);
-    MLF_CHECK(ctx_mex_scratch(ctx, (int)kw));
-    MexCall c = mex_begin(width, height, n, (int)kw, d_bitmap, ctx->mex_kq.ptr);
-    MLF_LAUNCH(launch_mex_mfma(c, d_bitmap, width, height, n, d_kernels, true, nullptr, nullptr, d_out,
+    MexCall c;
+    MLF_CHECK(ctx_mex_begin(ctx, width, height, n, (int)kw, d_bitmap, &c));
+    MLF_LAUNCH(launch_mex_mfma(c, d_bitmap, width, height, n, d_kernels, true, true, nullptr, nullptr, d_out,
                                ctx->stream));
     return MLF_OK;
   }
@@ -2420,11 +2431,11 @@ static mlf_status segments_device(mlf_context ctx, const float* d_in, int64_t W,
     MLF_CHECK(upload_vec(d_dst, dst));
     MLF_LAUNCH(launch_fill(d_out, img * nseg, 0.f, st));
     std::lock_guard<std::mutex> lk(ctx->mu);
-    MLF_CHECK(ctx_mex_scratch(ctx, kw));
-    MexCall c = mex_begin(W, H, nslices, kw, d_in, ctx->mex_kq.ptr);
+    MexCall c;
+    MLF_CHECK(ctx_mex_begin(ctx, W, H, nslices, kw, d_in, &c));
     int64_t zprev = -1;
     for (const Launch& l : launches) {
-      MLF_LAUNCH(launch_mex_mfma(c, d_in, W, H, l.n, d_K + (size_t)l.z * kplane, l.z != zprev,
+      MLF_LAUNCH(launch_mex_mfma(c, d_in, W, H, l.n, d_K + (size_t)l.z * kplane, l.z != zprev, &l == &launches.back(),
                                  d_src.ptr + l.off, d_dst.ptr + l.off, d_out, st));
       zprev = l.z;
     }

@@ -25,7 +25,8 @@ constexpr size_t kReadChunk = (size_t)4 << 20;  // bytes per buffer
 struct mlf_context_s {
   int device = 0;
   hipStream_t stream = nullptr;
-  mlf::DevBuf<float> mex_kq;  // MEX operator operand scratch, reused across calls (guarded by mu)
+  mlf::DevBuf<float> mex_scratch;  // MEX operator scratch, reused across calls (guarded by mu)
+  int64_t mex_room = 0;            // bitmaps whose marks it holds
   std::mutex mu;
   ReadSlot read[kReadThreads];  // guarded by read_mu; made on first use, freed with the context
   std::mutex read_mu;
