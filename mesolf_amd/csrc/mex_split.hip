@@ -3,8 +3,9 @@
 // As in k_mex_mfma (mex_kernels.hip), outputs grouped by phase make the operator a
 // GEMM: for output row y (q = y % 15), image n and x = 15 i + p
 //   out = sum_{ky, t} in[15 i + t - h, y - h + ky, n] * K[t - p, ky, p, q].
-// Every FP32 operand is split into three BF16 parts, x = x0 + x1 + x2 exactly
-// (8 + 8 + 8 significand bits, each part rounded to nearest), and a product
+// Every FP32 operand is split into three BF16 parts (8 + 8 + 8 significand bits, each
+// part rounded to nearest), x = x0 + x1 + x2 exactly for |x| from 2^-110 (8e-34): below,
+// x2 ends at BF16's last bit, 2^-133, and leaves up to 2^-134 out.  A product
 // takes the six MFMAs x0 k0, x0 k1, x1 k0, x1 k1, x0 k2, x2 k0, all into one
 // FP32 accumulator; the three left out are below 2^-24 of the product.  Six
 // 16x16x32 BF16 MFMAs take 96 cycles where the FP32 pipe takes 256, and the

@@ -574,11 +574,12 @@ void k_fwd_tpz(const T* __restrict__ W, FwdGeo g) {
 
 // ------------------------------------------- forward (Toeplitz, split FP32)
 // The FP32 forward on the BF16 matrix pipe.  Same GEMM, register window over
-// i1 and partial windows as k_fwd_tpz; every operand is split exactly into
-// three BF16 parts (x = x0 + x1 + x2, each rounded to nearest) and a product
-// takes the six MFMAs of the parts whose orders add up to at most two (left
-// out: below 2^-24 of the product).  Six 16x16x32 BF16 MFMAs take 96 cycles
-// where the FP32 pipe takes 256.  The matrix pipe cuts low bits of what it
+// i1 and partial windows as k_fwd_tpz; every operand is split into three BF16 parts
+// (x = x0 + x1 + x2, each rounded to nearest; exactly for |x| from 2^-110, up to 2^-134
+// off below, where the products with a normalised kernel's taps fall out of the
+// normal numbers anyway) and a product takes the six MFMAs of the parts whose
+// orders add up to at most two (left out: below 2^-24 of the product).  Six
+// 16x16x32 BF16 MFMAs take 96 cycles where the FP32 pipe takes 256.  The matrix pipe cuts low bits of what it
 // adds to a large accumulator, so a step's 24 MFMAs per tile start from zero
 // and their sum is added to the accumulator by the vector unit: with one chain
 // over all steps the sums came out 1.2e-6 low, with one per step the error
@@ -1650,7 +1651,7 @@ void k_bwd_mfma(const T* __restrict__ Wb, BwdGeo g, float wgt) {
 // ------------------------------------------------ backward (split FP32)
 // The FP32 backprojection and update on the BF16 matrix pipe: the GEMM, tap
 // order (bwd_quad_tap) and entries of k_bwd_mfma, with every operand split
-// exactly into three BF16 parts and six MFMAs per product as in k_fwd_tps.
+// into three BF16 parts and six MFMAs per product as in k_fwd_tps (exactly from 2^-110).
 // The ratio window stays FP32 in LDS, mirrored along axis 0 so that a lane's 8
 // taps are 8 ascending floats, and is split in registers: a window of ready
 // parts would need eight shifted copies to be read 16 bytes at a time (125 KB
