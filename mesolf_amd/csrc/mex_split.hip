@@ -370,8 +370,12 @@ static int split_nks(int kw) {
 }
 
 bool mex_split_takes(int64_t W, int64_t H, int64_t images, int kw) {
-  // 32-bit element offsets into the bitmaps and the M row count
-  return kw % 2 == 1 && kw <= kMexMfmaMaxKw && (double)W * H * images < 2147483648.0 && split_nks(kw) * 2 <= kMaxL;
+  // Kernels 1 and 3 pixels wide have too few products to pay for the operand table,
+  // the look through the bitmaps and the two launches: the FP32 form alone takes 17
+  // and 22 us for 150 x 137 (split form 23 and 28), 126 us for 396 x 396 x 96 at 3 (142);
+  // at 5 it takes 26 and 192 us (25 and 126).  32-bit element offsets into the
+  // bitmaps and the M row count.
+  return kw % 2 == 1 && kw > 3 && kw <= kMexMfmaMaxKw && (double)W * H * images < 2147483648.0 && split_nks(kw) * 2 <= kMaxL;
 }
 
 size_t mex_split_bytes(int kw) { return (size_t)kN * kw * split_nks(kw) * 3 * 1024; }
