@@ -328,7 +328,8 @@ mlf_status mlf_recon_phase_space(const float* lfimg, int64_t I1, int64_t I2,
  * with zero outside the bitmap (taps clipped as mex:55-78 clips them).
  * bitmap [width, height, n] single, kernels [kw, kw, 15, 15] single, out like
  * bitmap.  Host pointers, synchronous.  No kernel-width limit (the reference
- * stops at 341, mex:41). */
+ * stops at 341, mex:41).  A bitmap's result does not depend on the others of
+ * its call, bit for bit (calls of less than 2^31 pixels). */
 mlf_status mlf_lfm_convolution_vec(const float* bitmap, int64_t width, int64_t height, int64_t n,
                                    const float* kernels, int64_t kw, int64_t nphase,
                                    float* out, int32_t device);

@@ -10,11 +10,12 @@
 // FP32 accumulator; the three left out are below 2^-24 of the product.  Six
 // 16x16x32 BF16 MFMAs take 96 cycles where the FP32 pipe takes 256, and the
 // accumulator is rounded 6 times per 32 taps instead of 8 or more times.
-// Bound by the matrix pipe.  396 x 396 x 96, kw = 241: 8.85 ms, 1.19e15 BF16
+// Bound by the matrix pipe.  396 x 396 x 96, kw = 241: 8.44 ms, 1.25e15 BF16
 // flop/s issued for the products alone (FP32 MFMA, k_mex_mfma: 26.8 ms); 24
-// segments over 5 planes of that size: 7.9 ms (23.9); one 150 x 137 bitmap,
-// kw = 61: 35 us (229: one wave in eight had work).  Relative L2 error against
-// FP64 there: 5.7e-7 / 2.2e-7 / 7.2e-8 (FP32 MFMA 8.2e-7 / 7.9e-7 / 6.1e-7).
+// segments over 5 planes of that size: 6.3 to 8.5 ms by their slices (24.5 for the
+// former); one 150 x 137 bitmap, kw = 61: 34 us (229: one wave in eight had work).
+// Relative L2 error against FP64 there: 9.5e-8 / 8.7e-8 / 6.5e-8 (FP32 MFMA 8.2e-7 / 7.9e-7
+// / 6.1e-7; in one chain over all rows, whose low bits the pipe cuts, 5.6e-7 / 1.8e-7 / 6.6e-8).
 //
 // Operand layout.  A lenslet's 15 pixels take 16 slots (slot 15 zero), so tap
 // t = 15 L + s - b sits at slot s of lenslet i - a + L (h = 15 a - b) and the
@@ -128,9 +129,16 @@ __global__ __launch_bounds__(256) void k_mex_split_prep(const float* __restrict_
   else *marks.image(img) = call;
 }
 
-// WM waves along M times WK groups that share the input rows (row j goes to
-// group j % WK; the groups' accumulators are added in group order at the
-// end), MT M-tiles per wave, G output rows, SPB K-steps per barrier.
+// Input row r is of class r % kClasses.  Each class is summed from zero, row by
+// row, and the sums of the classes are added in class order, whatever the shape
+// of the workgroups: an output's bits do not depend on the shape, and so not on
+// how many bitmaps share the call (a call may take any of the shapes below).
+constexpr int kClasses = 8;
+
+// WM waves along M times WK groups that share the input rows (class c goes to
+// group c % WK in lap c / WK; every group keeps the sums of its laps to the end, or
+// adds them up as it goes if it is the only one), MT M-tiles per wave, G output rows,
+// SPB K-steps per barrier.
 template <int WM, int WK, int MT, int G, int SPB>
 struct SplitShape {
   static constexpr int kThreads = 64 * WM * WK;
@@ -141,17 +149,19 @@ struct SplitShape {
   static constexpr int kA = 3 * kPart;              // one input row, three parts
   static constexpr int kB = SPB * G * 3 * 1024;     // one stage of kernel fragments
   static constexpr int kGroup = 2 * kA + 2 * kB;
-  static constexpr int kLds = WK * kGroup;
-  static_assert(kLds <= 160 * 1024, "LDS");
-  static_assert((WK - 1) * WM * MT * G * 1024 <= kLds, "reduction buffer");
+  static constexpr int kLaps = kClasses / WK;
+  static constexpr int kSums = WK == 1 ? 1 : kLaps;  // sums kept
+  static constexpr int kRed = (WK - 1) * kSums * WM * MT * G * 1024;  // the other groups' sums, at the end
+  static constexpr int kLds = WK * kGroup > kRed ? WK * kGroup : kRed;
+  static_assert(kClasses % WK == 0 && kLds <= 160 * 1024, "LDS");
+  static constexpr int kPerCu = 160 * 1024 / kLds;  // workgroups that share a CU
 };
 
 template <int WM, int WK, int MT, int G, int SPB>
-__global__ __launch_bounds__(64 * WM * WK) void k_mex_split(const float* __restrict__ in, SplitGeo g,
-                                                            const uintx4* __restrict__ Bt, float* __restrict__ out,
-                                                            const int32_t* __restrict__ src,
-                                                            const int32_t* __restrict__ dst, MexMarks marks,
-                                                            int set) {
+__global__ __launch_bounds__(64 * WM * WK)
+__attribute__((amdgpu_waves_per_eu(SplitShape<WM, WK, MT, G, SPB>::kPerCu * WM * WK / 4)))
+void k_mex_split(const float* __restrict__ in, SplitGeo g, const uintx4* __restrict__ Bt, float* __restrict__ out,
+                 const int32_t* __restrict__ src, const int32_t* __restrict__ dst, MexMarks marks, int set) {
   using S = SplitShape<WM, WK, MT, G, SPB>;
   constexpr int NTH = 64 * WM;  // threads of a group
   constexpr int NU = (S::kSlots * 8 + NTH - 1) / NTH;  // pixel pairs staged per thread and row
@@ -225,14 +235,14 @@ __global__ __launch_bounds__(64 * WM * WK) void k_mex_split(const float* __restr
   for (int m = 0; m < MT; ++m) lens[m] = (M0 + 16 * (wm * MT + m) + lr) % nL - g.a + (lg >> 1);
   const int slot0 = 16 * wm * MT + lr + (lg >> 1);
 
-  floatx4 acc[MT][G];
+  floatx4 acc[MT][G], sum[S::kSums][MT][G];
 #pragma unroll
   for (int m = 0; m < MT; ++m)
 #pragma unroll
-    for (int i = 0; i < G; ++i) acc[m][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < G; ++i) acc[m][i] = sum[0][m][i] = floatx4{0.f, 0.f, 0.f, 0.f};
 
   const int rlo = max(0, y0 - g.h), rhi = min(H - 1, y0 + G - 1 + g.h);
-  const int nj = (rhi - rlo + WK) / WK;       // rows per group
+  const int nj = (rhi - rlo) / kClasses + 1;  // rows of a class, at most
   const int ns = (g.nks + SPB - 1) / SPB;     // stages per row
   const __amdgpu_buffer_rsrc_t br = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uintx4*>(Bt), 0, kN * g.kw * g.nks * 3 * 1024, kDword3);
@@ -253,13 +263,27 @@ __global__ __launch_bounds__(64 * WM * WK) void k_mex_split(const float* __restr
     }
   };
 
-  issue_b(rlo + wk, 0, Bb);
-  load_row(min(rlo + wk, H - 1));
+  // The rows of this group, class by class.  Several groups walk nj rows of
+  // each class together (past the last one a row is not used); a group alone takes
+  // the rows there are.
+  auto first = [&](int lap) { return rlo + ((lap * WK + wk - rlo) & (kClasses - 1)); };
+  int lap = 0, j = 0, r = first(0);
+  if (WK == 1)
+    while (r > rhi) r = first(++lap);
+  issue_b(r, 0, Bb);
+  load_row(min(r, H - 1));
   store_row(Ab);
   int t = 0;
-  for (int j = 0; j < nj; ++j) {
-    const int r = rlo + j * WK + wk;
-    const char* A = Ab + (j & 1) * S::kA;
+  for (int n = 0;; ++n) {
+    int lap2 = lap, r2 = r + kClasses;  // the row after this one
+    if (WK == 1) {
+      while (r2 > rhi && ++lap2 < S::kLaps) r2 = first(lap2);
+    } else if (++j == nj) {
+      j = 0;
+      r2 = first(++lap2);
+    }
+    const bool lastrow = lap2 == S::kLaps;
+    const char* A = Ab + (n & 1) * S::kA;
     unsigned use = 0;  // output rows whose kernel holds this input row
 #pragma unroll
     for (int i = 0; i < G; ++i) {
@@ -272,10 +296,9 @@ __global__ __launch_bounds__(64 * WM * WK) void k_mex_split(const float* __restr
       // wave is done with the buffers that are written next
       __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();
-      const bool lastrow = j + 1 >= nj;
-      if (!(lastrow && s + 1 >= ns)) issue_b(s + 1 < ns ? r : r + WK, s + 1 < ns ? s + 1 : 0, Bb + ((t + 1) & 1) * S::kB);
-      if (s == 0 && !lastrow) load_row(min(r + WK, H - 1));
-      if (s == 1 && !lastrow) store_row(Ab + ((j + 1) & 1) * S::kA);
+      if (!(lastrow && s + 1 >= ns)) issue_b(s + 1 < ns ? r : r2, s + 1 < ns ? s + 1 : 0, Bb + ((t + 1) & 1) * S::kB);
+      if (s == 0 && !lastrow) load_row(min(r2, H - 1));
+      if (s == 1 && !lastrow) store_row(Ab + ((n + 1) & 1) * S::kA);
       const char* B = Bb + (t & 1) * S::kB + lane * 16;
 #pragma unroll
       for (int kk = 0; kk < SPB; ++kk) {
@@ -303,27 +326,53 @@ __global__ __launch_bounds__(64 * WM * WK) void k_mex_split(const float* __restr
               acc[m][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m][pa[q]], b[pb[q]], acc[m][i], 0, 0, 0);
         }
       }
-      if (ns == 1 && !lastrow) store_row(Ab + ((j + 1) & 1) * S::kA);
+      if (ns == 1 && !lastrow) store_row(Ab + ((n + 1) & 1) * S::kA);
     }
-  }
-
-  if constexpr (WK > 1) {
-    __syncthreads();
-    floatx4* red = reinterpret_cast<floatx4*>(sm);
-    if (wk > 0) {
+    if (lap2 != lap && (WK == 1 || !lastrow)) {  // the class is complete
+#pragma unroll
+      for (int p = 0; p < (WK == 1 ? 1 : S::kSums - 1); ++p)
+        if (WK == 1 || p == lap)
+#pragma unroll
+          for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int i = 0; i < G; ++i) sum[p][m][i] = WK == 1 ? sum[p][m][i] + acc[m][i] : acc[m][i];
 #pragma unroll
       for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int i = 0; i < G; ++i) red[((((wk - 1) * WM + wm) * MT + m) * G + i) * 64 + lane] = acc[m][i];
+        for (int i = 0; i < G; ++i) acc[m][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    if (lastrow) break;
+    lap = lap2;
+    r = r2;
+  }
+
+  if constexpr (WK > 1) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int i = 0; i < G; ++i) sum[S::kSums - 1][m][i] = acc[m][i];  // the last lap's
+    __syncthreads();
+    // [group - 1][lap][wave][MT][G][lane]
+    floatx4* red = reinterpret_cast<floatx4*>(sm) + wm * MT * G * 64 + lane;
+    constexpr int kOne = WM * MT * G * 64;
+    if (wk > 0) {
+#pragma unroll
+      for (int p = 0; p < S::kSums; ++p)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+          for (int i = 0; i < G; ++i) red[((wk - 1) * S::kSums + p) * kOne + (m * G + i) * 64] = sum[p][m][i];
     }
     __syncthreads();
     if (wk > 0) return;
 #pragma unroll
-    for (int k = 0; k < WK - 1; ++k)
+    for (int c = 1; c < kClasses; ++c)
 #pragma unroll
       for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int i = 0; i < G; ++i) acc[m][i] += red[(((k * WM + wm) * MT + m) * G + i) * 64 + lane];
+        for (int i = 0; i < G; ++i)
+          sum[0][m][i] += c % WK == 0 ? sum[c / WK % S::kSums][m][i]
+                                      : red[((c % WK - 1) * S::kSums + c / WK) * kOne + (m * G + i) * 64];
   }
   if (lr >= kN) return;
 #pragma unroll
@@ -339,7 +388,7 @@ __global__ __launch_bounds__(64 * WM * WK) void k_mex_split(const float* __restr
       for (int i = 0; i < G; ++i) {
         if (y0 + i >= H) continue;
         float* d = o + (size_t)(y0 + i) * W;
-        *d = dst ? *d + acc[m][i][j] : acc[m][i][j];
+        *d = dst ? *d + sum[0][m][i][j] : sum[0][m][i][j];
       }
     }
 }
@@ -348,11 +397,13 @@ typedef void (*SplitKernel)(const float*, SplitGeo, const uintx4*, float*, const
                             int);
 struct SplitVariant {
   SplitKernel fn;
-  int wm, wk, mt, g, spb, lds;
+  int wm, wk, mt, g, spb, lds, per_cu;
+  double step;  // matrix and LDS cycles of a K-step
 };
 template <int WM, int WK, int MT, int G, int SPB>
-SplitVariant variant() {
-  return {&k_mex_split<WM, WK, MT, G, SPB>, WM, WK, MT, G, SPB, SplitShape<WM, WK, MT, G, SPB>::kLds};
+SplitVariant variant(double step) {
+  using S = SplitShape<WM, WK, MT, G, SPB>;
+  return {&k_mex_split<WM, WK, MT, G, SPB>, WM, WK, MT, G, SPB, S::kLds, S::kPerCu, step};
 }
 
 }  // namespace
@@ -394,19 +445,41 @@ hipError_t launch_mex_split_prep(const MexCall& c, const float* K, size_t image,
   return hipGetLastError();
 }
 
-// The shape with the least estimated time: matrix or LDS cycles of a
-// workgroup's longest group, times the rounds that 256 CUs need (every shape
-// fills a CU's LDS).  396 x 396, kw = 241: 96 bitmaps take <8, 1, 3, 4, 2> (162
-// M-tiles in blocks of 24: 693 workgroups, 2.7 rounds; blocks of 32 would pad
-// them by a fifth), 17 bitmaps <2, 4, 2, 2, 1> or <4, 2, 2, 4, 1>, one small
-// bitmap <1, 8, 1, 1, 1> (eight waves share the kernel's rows).
+// Estimated cycles of a shape: the rounds that the XCD with the most row groups
+// takes on its 32 CUs, the groups with the most input rows first.  A CU
+// that holds e workgroups takes for a row the longer of all their K-steps and of
+// one workgroup's chain, its own K-steps with a latency of 630 cycles each and
+// 500 per barrier; a round 20000 more.  The cycles of each shape's K-step and these
+// constants are fitted to 110 sizes (90 to 500 pixels, 1 to 128 bitmaps, kw 31 to 251): the
+// estimates are 6 % off in the mean, and the shape chosen by them is 1.4 % slower than the
+// best of 19.  396 x 396, kw = 241: 96 bitmaps take <8, 1, 2, 2, 2>, two workgroups per
+// CU (8.4 ms; <8, 1, 3, 4, 2>, one per CU, 9.0), 10 bitmaps <2, 4, 2, 3, 1> (1.49; 1.95 to 2.1 with one
+// group of waves), one small bitmap <1, 8, 1, 1, 1> (eight waves share the kernel's rows).
+static double split_cycles(const SplitVariant& v, const SplitGeo& g, int64_t cells) {
+  const int64_t nyg = (g.H + v.g - 1) / v.g, nmb = (cells + 16 * v.mt * v.wm - 1) / (16 * v.mt * v.wm);
+  const int64_t wgs = (nyg + 7) / 8 * nmb, slots = 32 * v.per_cu, rounds = (wgs + slots - 1) / slots;
+  const double own = g.nks * v.step, chain = own + 630.0 * g.nks + 500.0 * ((g.nks + v.spb - 1) / v.spb);
+  const int64_t skip = (rounds + 63) / 64;  // of many rounds, 64 are looked at
+  double t = 0.0;
+  for (int64_t k = 0; k < rounds; k += skip) {
+    const int64_t rank = std::min(nyg - 1, k * slots / nmb * 8);
+    const int64_t y0 = v.g * ((rank & 1) ? nyg / 2 - (rank + 1) / 2 : nyg / 2 + rank / 2);
+    const int64_t most = std::min<int64_t>(g.H - 1, y0 + v.g - 1 + g.h) - std::max<int64_t>(0, y0 - g.h) + 1;
+    const double rows = v.wk == 1 ? (double)most : (double)(kClasses / v.wk) * ((most - 1) / kClasses + 1);
+    const int64_t share = std::min<int64_t>(v.per_cu, (wgs - k * slots + 31) / 32);
+    t += std::min(skip, rounds - k) * (rows * std::max(share * own, chain) + 20000.0);
+  }
+  return t;
+}
+
 hipError_t launch_mex_split(const MexCall& c, const float* in, int64_t W, int64_t H, int64_t n,
                             const int32_t* src, const int32_t* dst, float* out, hipStream_t st) {
   const int kw = c.kw;
   static const SplitVariant variants[] = {
-      variant<8, 1, 4, 4, 2>(), variant<8, 1, 3, 4, 2>(), variant<8, 1, 2, 4, 2>(), variant<4, 2, 4, 4, 1>(),
-      variant<4, 2, 3, 4, 1>(), variant<4, 2, 2, 4, 1>(), variant<2, 4, 2, 2, 1>(), variant<1, 8, 2, 1, 1>(),
-      variant<1, 8, 1, 1, 1>(),
+      variant<8, 1, 2, 2, 2>(1190), variant<8, 1, 1, 2, 2>(600),  variant<4, 1, 3, 3, 2>(1500),
+      variant<4, 1, 2, 4, 2>(1245), variant<4, 2, 2, 2, 1>(840),  variant<2, 4, 2, 3, 1>(1460),
+      variant<2, 4, 3, 2, 1>(1715), variant<2, 4, 2, 2, 1>(890),  variant<1, 8, 2, 1, 1>(505),
+      variant<1, 8, 1, 1, 1>(75),
   };
   static const hipError_t attr = [] {
     for (const SplitVariant& v : variants) {
@@ -431,10 +504,7 @@ hipError_t launch_mex_split(const MexCall& c, const float* in, int64_t W, int64_
   const SplitVariant* best = nullptr;
   double best_t = 0.0;
   for (const SplitVariant& v : variants) {
-    const int64_t wgs = (H + v.g - 1) / v.g * ((cells + 16 * v.mt * v.wm - 1) / (16 * v.mt * v.wm));
-    const double rows = (double)std::min<int64_t>(H, kw + v.g - 1) / v.wk;
-    const double mfma = 2.0 * 6 * 16 * v.mt * v.g, lds = 8.0 * 8 * 3 * (v.mt + v.g);
-    const double t = (double)((wgs + 255) / 256) * (rows * (g.nks * std::max(mfma, lds) + 400.0 * ((g.nks + v.spb - 1) / v.spb)) + 4000.0);
+    const double t = split_cycles(v, g, cells);
     if (!best || t < best_t) {
       best = &v;
       best_t = t;

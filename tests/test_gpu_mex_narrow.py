@@ -32,7 +32,4 @@ def test_narrow_kernels(W, H, n, kw):
             for i in range(ptr[s], ptr[s + 1]):
                 if plane[i] == z:
                     sum_ = sum_ + mesolf_amd.mex_lfm_convolution_vec(b[:, :, i:i + 1], K2[..., z])[:, :, 0]
-        if kw <= 3:  # one shape for any count: bit for bit
-            assert np.array_equal(seg[:, :, s], sum_)
-        else:
-            assert np.abs(seg[:, :, s] - sum_).max() <= 2.9e-6 * n * size.max()
+        assert np.array_equal(seg[:, :, s], sum_)
