@@ -214,6 +214,12 @@ void batch_mark_dirty(mlf_batch_s* b) {
   b->dirty = true;
 }
 
+// The lives' mutex keeps the batch from being destroyed until its own is held.
+std::unique_lock<std::mutex> batch_hold(mlf_patch_s* p) {
+  std::lock_guard<std::mutex> life(g_life_mu);
+  return p->batch ? std::unique_lock<std::mutex>(p->batch->mu) : std::unique_lock<std::mutex>();
+}
+
 // Called by mlf_patch_destroy.
 mlf_status batch_forget_patch(mlf_patch_s* p) {
   mlf_batch_s* b = p->batch;

@@ -197,6 +197,11 @@ void mlf::ctx_free(mlf_context ctx) {
     (void)hipStreamSynchronize(ctx->stream);
     (void)hipStreamDestroy(ctx->stream);
   }
+  if (ctx->read_stream) {
+    (void)hipStreamSynchronize(ctx->read_stream);
+    (void)hipStreamDestroy(ctx->read_stream);
+  }
+  if (ctx->read_ready) (void)hipEventDestroy(ctx->read_ready);
   for (ReadSlot& s : ctx->read)
     for (int b = 0; b < 2; ++b) {
       if (s.ev[b]) (void)hipEventDestroy(s.ev[b]);
@@ -1456,24 +1461,31 @@ mlf_status mlf_patch_set_volume(mlf_patch p, const float* X) {
 // in all), 13 ms for 165 MB (81 x 73 x 31: 135 -> 122 ms).  Smaller volumes take
 // that copy: pinning and freeing the 64 MB of buffers takes 5 ms of a context's life,
 // what one read of 64 MB saves (98 MB: 10.1 -> 2.7 ms, 3.4 the first time and
-// 2 more to free; 32 MB: 3.3 -> 1.2, 5.1 the first time).  Returns false, with nothing pending, if
-// the buffers are not to be had.
+// 2 more to free; 32 MB: 3.3 -> 1.2, 5.1 the first time).  The chunks go through a stream of their
+// own, behind what the context's holds now: on the context's, each would wait for
+// the work that other threads enqueue between two of them (240 MB while another patch
+// runs three iterations at a time: 99 ms and six of them, with the chunks' own stream
+// 6 to 50 and three).  Returns false, with nothing pending, if the buffers are not to be had.
 constexpr size_t kReadMin = (size_t)64 << 20;
 
 static bool read_volume(mlf_context ctx, const float* X, void* out, bool f64, int n1, int n2, size_t numel) {
   const size_t es = f64 ? 8 : 4, per = kReadChunk / es;
   const int64_t nchunk = (int64_t)((numel + per - 1) / per);
   std::lock_guard<std::mutex> lk(ctx->read_mu);
+  bool have = ctx->read_stream || hipStreamCreateWithFlags(&ctx->read_stream, hipStreamNonBlocking) == hipSuccess;
+  have = have && (ctx->read_ready || hipEventCreateWithFlags(&ctx->read_ready, hipEventDisableTiming) == hipSuccess);
   for (ReadSlot& s : ctx->read)
     for (int b = 0; b < 2; ++b) {
-      if (!s.buf[b] && hipHostMalloc(&s.buf[b], kReadChunk, hipHostMallocDefault) != hipSuccess) s.buf[b] = nullptr;
-      if (!s.ev[b] && hipEventCreateWithFlags(&s.ev[b], hipEventDisableTiming) != hipSuccess) s.ev[b] = nullptr;
-      if (!s.buf[b] || !s.ev[b]) {
-        (void)hipGetLastError();
-        return false;
-      }
+      have = have && (s.buf[b] || hipHostMalloc(&s.buf[b], kReadChunk, hipHostMallocDefault) == hipSuccess);
+      have = have && (s.ev[b] || hipEventCreateWithFlags(&s.ev[b], hipEventDisableTiming) == hipSuccess);
     }
-  if (hipStreamSynchronize(ctx->stream) != hipSuccess) return false;  // one thread waits for the volume, not all
+  const hipStream_t st = ctx->read_stream;
+  // one thread waits for the volume, not all
+  if (!have || hipEventRecord(ctx->read_ready, ctx->stream) != hipSuccess ||
+      hipStreamWaitEvent(st, ctx->read_ready, 0) != hipSuccess || hipEventSynchronize(ctx->read_ready) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
   std::atomic<bool> ok{true};
   std::atomic<int64_t> next{0};
   auto work = [&](int t) {
@@ -1487,9 +1499,9 @@ static bool read_volume(mlf_context ctx, const float* X, void* out, bool f64, in
       const int64_t c = ok ? next.fetch_add(1) : nchunk;
       if (c < nchunk) {
         const size_t first = (size_t)c * per;
-        if (launch_from_blocked(X, s.buf[b], f64, n1, n2, first, std::min(per, numel - first), ctx->stream) ==
+        if (launch_from_blocked(X, s.buf[b], f64, n1, n2, first, std::min(per, numel - first), st) ==
                 hipSuccess &&
-            hipEventRecord(s.ev[b], ctx->stream) == hipSuccess)
+            hipEventRecord(s.ev[b], st) == hipSuccess)
           at[b] = c;
         else
           ok = false;
@@ -1516,7 +1528,7 @@ static bool read_volume(mlf_context ctx, const float* X, void* out, bool f64, in
   work(0);
   for (std::thread& t : th) t.join();
   if (!ok) {
-    (void)hipStreamSynchronize(ctx->stream);
+    (void)hipStreamSynchronize(st);
     (void)hipGetLastError();
   }
   return ok;
@@ -1529,7 +1541,11 @@ static mlf_status get_volume_impl(mlf_patch p, void* out, bool f64) {
   MLF_CHECK(ctx_activate(p->psf->ctx));
   hipStream_t st = p->psf->ctx->stream;
   const size_t numel = patch_numel(p), bytes = numel * (f64 ? 8 : 4);
-  if (bytes >= kReadMin && read_volume(p->psf->ctx, p->X.ptr, out, f64, p->n1, p->n2, numel)) return MLF_OK;
+  if (bytes >= kReadMin) {
+    // p->mu keeps the patch as it is while its chunks are read; so does this for its batch
+    const std::unique_lock<std::mutex> held = batch_hold(p);
+    if (read_volume(p->psf->ctx, p->X.ptr, out, f64, p->n1, p->n2, numel)) return MLF_OK;
+  }
   DevBuf<uint8_t> tmp;
   MLF_CHECK(tmp.alloc(bytes));
   MLF_LAUNCH(launch_from_blocked(p->X.ptr, tmp.ptr, f64, p->n1, p->n2, 0, numel, st));

@@ -29,6 +29,8 @@ struct mlf_context_s {
   int64_t mex_room = 0;            // bitmaps whose marks it holds
   std::mutex mu;
   ReadSlot read[kReadThreads];  // guarded by read_mu; made on first use, freed with the context
+  hipStream_t read_stream = nullptr;
+  hipEvent_t read_ready = nullptr;  // what is read is complete
   std::mutex read_mu;
   int refs = 0;         // live PSFs created on this context
   bool closed = false;  // destroy requested; freed when refs reaches 0
@@ -172,6 +174,7 @@ void batch_mark_dirty(mlf_batch_s* b);  // a patch's slot descriptor changed
 size_t patch_device_bytes(const mlf_patch_s* p);
 size_t patch_bytes_estimate(mlf_psf_s* ps, mlf_precision prec, int n1, int n2);
 mlf_status batch_forget_patch(mlf_patch_s* p);  // detach before destruction
+std::unique_lock<std::mutex> batch_hold(mlf_patch_s* p);  // keeps p's batch, if any, from running
 // (Re)build a patch's work entries, partial buffers and slot descriptor for
 // its tile shape (fwd_mt, bwd_nt, bwd_grp, bwd_occ); the caller synchronises the
 // stream first.
