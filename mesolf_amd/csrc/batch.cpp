@@ -38,7 +38,6 @@ struct mlf_batch_s {
   int cus = 0;
   size_t smem_f = 0, smem_b = 0;
   int fwd_nbuf = 2;
-  int bwd_gpe = 1;  // phase groups per backprojection entry (backward_split)
   // one RL iteration's view loop as a graph
   bool use_graph = true;
   hipGraph_t graph = nullptr;
@@ -93,8 +92,6 @@ mlf_status rebuild(mlf_batch_s* b) {
   int tiles = 0;
   for (const mlf_patch_s* p : b->slots) tiles += (int)(p->bent.size() / 4) * p->bwd_gpe / ngrp;
   const int gpe = backward_split(tiles, ngrp, bwd_groups_per_entry(b->bwd_nt, b->bwd_grp));
-  if (gpe != b->bwd_gpe) drop_graph(b);
-  b->bwd_gpe = gpe;
   for (size_t i = 0; i < b->slots.size(); ++i) {
     mlf_patch_s* p = b->slots[i];
     sd.push_back(p->slot);
@@ -132,17 +129,21 @@ mlf_status rebuild(mlf_batch_s* b) {
   // with an uneven last round (three patches of 45 x 52 to 75 x 75 x 51, per view:
   // forward 242 -> 220 us, backprojection 384 -> 366 us).  A captured
   // launch keeps its grid: it serves fewer entries as it is, and more
-  // entries replace it.
-  if (b->n_f > b->grid_f || b->n_b > b->grid_b) drop_graph(b);
-  b->grid_f = std::max(b->grid_f, b->n_f);
-  b->grid_b = std::max(b->grid_b, b->n_b);
+  // entries replace it, with room for half as many again (capturing 177 views
+  // takes 1 ms, more than a view of a small batch gains; the workgroups without an
+  // entry take 1 us per launch).
+  const bool grow = b->n_f > b->grid_f || b->n_b > b->grid_b;
+  const int room = grow && b->exec ? 3 : 2;
+  if (grow) drop_graph(b);
+  if (b->n_f > b->grid_f) b->grid_f = b->n_f * room / 2;
+  if (b->n_b > b->grid_b) b->grid_b = b->n_b * room / 2;
   if (!sd.empty())
     MLF_HIP(hipMemcpy(b->d_slots.ptr, sd.data(), sd.size() * sizeof(SlotDesc), hipMemcpyHostToDevice));
   MLF_CHECK(upload_table(b, b->d_fsched, fs));
   MLF_CHECK(upload_table(b, b->d_bsched, bs));
   MLF_CHECK(upload_table(b, b->d_rsched, rs));
-  const std::vector<int32_t> counts{b->n_f, b->n_b, b->n_r};
-  MLF_HIP(hipMemcpy(b->d_counts.ptr, counts.data(), 3 * sizeof(int32_t), hipMemcpyHostToDevice));
+  const std::vector<int32_t> counts{b->n_f, b->n_b, b->n_r, gpe};
+  MLF_HIP(hipMemcpy(b->d_counts.ptr, counts.data(), counts.size() * sizeof(int32_t), hipMemcpyHostToDevice));
   b->dirty = false;
   return MLF_OK;
 }
@@ -169,7 +170,7 @@ mlf_status enqueue_views(mlf_batch_s* b, hipStream_t st, int nviews = 0) {
       MLF_LAUNCH(launch_ratio_gather(g, rg, b->grid_r, ps->Z, b->bm2, u, v, 1, nullptr, st));
     }
     const BwdGeo bg{b->d_slots.ptr, ps->d_rb.ptr, pk.d_boff.ptr, pk.d_epad.ptr, b->d_bsched.ptr,
-                    b->d_counts.ptr + 1, k, b->bwd_gpe};
+                    b->d_counts.ptr + 1, k, b->d_counts.ptr + 3};
     // every slot of a BF16 Toeplitz batch holds its volume in the split form
     const bool split = b->tpz && b->kp == Precision::kBF16;
     MLF_LAUNCH(launch_bwd_mfma(b->kp, b->bwd_nt, b->bwd_occ, split, pk.bwd.ptr + (size_t)k * pk.pvb * eb, bg,
@@ -259,9 +260,9 @@ mlf_status mlf_batch_create(mlf_psf psf, mlf_precision prec, int32_t capacity, m
   b->kp = kernel_precision(prec);
   b->capacity = capacity;
   MLF_CHECK(b->d_slots.alloc((size_t)capacity));
-  MLF_CHECK(b->d_counts.alloc(3));
-  const std::vector<int32_t> zero{0, 0, 0};
-  MLF_HIP(hipMemcpy(b->d_counts.ptr, zero.data(), 3 * sizeof(int32_t), hipMemcpyHostToDevice));
+  const std::vector<int32_t> none{0, 0, 0, 1};  // entries of each kernel; groups per backprojection entry
+  MLF_CHECK(b->d_counts.alloc(none.size()));
+  MLF_HIP(hipMemcpy(b->d_counts.ptr, none.data(), none.size() * sizeof(int32_t), hipMemcpyHostToDevice));
   int cus = 0;
   MLF_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, psf->ctx->device));
   // two workgroups per CU for the MFMA kernels (their LDS and register
@@ -308,8 +309,11 @@ mlf_status mlf_batch_attach(mlf_batch b, mlf_patch p) {
     return set_error(MLF_ERR_BUDGET, "batch is full (%d patches)", b->capacity);
   MLF_CHECK(ctx_activate(b->psf->ctx));
   if (b->slots.empty()) {
-    if (b->fwd_mt != p->fwd_mt || b->bwd_nt != p->bwd_nt || b->bwd_grp != p->bwd_grp || b->bwd_occ != p->bwd_occ)
+    if (b->fwd_mt != p->fwd_mt || b->bwd_nt != p->bwd_nt || b->bwd_grp != p->bwd_grp || b->bwd_occ != p->bwd_occ) {
       drop_graph(b);
+      b->grid_f = 2 * b->cus;
+      b->grid_b = p->bwd_occ * b->cus;
+    }
     b->tpz = p->tpz;
     b->cw = p->cw;
     b->bm2 = p->bm2;
@@ -317,7 +321,6 @@ mlf_status mlf_batch_attach(mlf_batch b, mlf_patch p) {
     b->bwd_nt = p->bwd_nt;
     b->bwd_grp = p->bwd_grp;
     b->bwd_occ = p->bwd_occ;
-    b->grid_b = b->bwd_occ * b->cus;
     b->smem_f = p->smem_f;
     b->smem_b = p->smem_b;
     b->fwd_nbuf = p->fwd_nbuf;

@@ -106,7 +106,7 @@ struct BwdGeo {
   const int32_t* sched;   // [entries][5] = (slot, z, b1, b2, first phase group)
   const int32_t* count;
   int view;               // selects the normaliser table of the view
-  int groups;             // phase groups per entry (they share its ratio window)
+  const int32_t* groups;  // phase groups per entry (they share its ratio window)
 };
 
 struct PackGeo {

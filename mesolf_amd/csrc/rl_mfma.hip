@@ -1097,7 +1097,7 @@ void k_bwd_mfma(const T* __restrict__ Wb, BwdGeo g, float wgt) {
   // SPL N-tiles: NPR pairs, then (odd NT) one unpaired tile
   constexpr int NPR = NT / 2;
   extern __shared__ __align__(16) char smem[];
-  const int nent = uni(cload(g.count));
+  const int nent = uni(cload(g.count)), ngroups = uni(cload(g.groups));
   for (int ent = blockIdx.x; ent < nent; ent += gridDim.x) {
     const int* s = g.sched + 5 * ent;
     const SlotDesc sd = load_slot(g.slots, uni(cload(s)));
@@ -1258,7 +1258,7 @@ void k_bwd_mfma(const T* __restrict__ Wb, BwdGeo g, float wgt) {
     }
 
     bool pref = false;  // the group's first tap slices were issued by the previous group
-    for (int gi = 0; gi < g.groups; ++gi) {  // phase group grp: 16 * NT phases from 16 * NT * grp
+    for (int gi = 0; gi < ngroups; ++gi) {  // phase group grp: 16 * NT phases from 16 * NT * grp
       const int grp = grp0 + gi;
       const T* Bz = Wb + boffz + (size_t)(grp * 16 * NT) * epad;
       floatx4 acc[MT][NT];
@@ -1365,7 +1365,7 @@ void k_bwd_mfma(const T* __restrict__ Wb, BwdGeo g, float wgt) {
       // issued once every wave is done with the ring, so that they land
       // while this group's update runs (16-bit)
       auto prefetch_next = [&]() {
-        if (gi + 1 < g.groups) {
+        if (gi + 1 < ngroups) {
           lds_barrier();
   #pragma unroll
           for (int q = 0; q < STG - SPB; ++q) issue_taps_g(grp + 1, q, q);
@@ -1681,7 +1681,7 @@ void k_bwd_split(const char* __restrict__ Wb, BwdGeo g, float wgt) {
   constexpr int PRE = NT == 3 ? MT : 2;  // M-tiles whose X is loaded before the K loop (registers)
   constexpr int kSlice = NT * 3 * kSplitFrag;
   extern __shared__ __align__(16) char smem[];
-  const int nent = uni(cload(g.count));
+  const int nent = uni(cload(g.count)), ngroups = uni(cload(g.groups));
   for (int ent = blockIdx.x; ent < nent; ent += gridDim.x) {
     const int* s = g.sched + 5 * ent;
     const SlotDesc sd = load_slot(g.slots, uni(cload(s)));
@@ -1747,7 +1747,7 @@ void k_bwd_split(const char* __restrict__ Wb, BwdGeo g, float wgt) {
       }
     }
 
-    for (int gi = 0; gi < g.groups; ++gi) {
+    for (int gi = 0; gi < ngroups; ++gi) {
       const int grp = grp0 + gi;
       const int gbase = grp * 16 * NT;
       floatx4 acc[MT][NT];
@@ -1862,7 +1862,7 @@ void k_bwd_split(const char* __restrict__ Wb, BwdGeo g, float wgt) {
 #pragma unroll
       for (int mt = 0; mt < 2; ++mt) load_t(mt, bt[mt]);
       lds_barrier();  // every wave is done with the ring (and, after the last group, the window)
-      if (gi + 1 < g.groups) {
+      if (gi + 1 < ngroups) {
         issue_taps(grp + 1, 0);
         issue_taps(grp + 1, 1);
       }

@@ -978,7 +978,7 @@ static BwdGeo bwd_geo(mlf_patch_s* p, int k) {
   mlf_psf_s* ps = p->psf;
   const PrecPack& pk = ps->pack[(int)p->kp];
   return BwdGeo{p->d_slot.ptr, ps->d_rb.ptr, pk.d_boff.ptr, pk.d_epad.ptr, p->d_bsched.ptr,
-                p->d_counts.ptr + 1, k, p->bwd_gpe};
+                p->d_counts.ptr + 1, k, p->d_counts.ptr + 3};
 }
 
 // Forward projection of view k, then the ratio (LF != null) and/or y.
@@ -1196,7 +1196,7 @@ mlf_status mlf::patch_setup_tiles(mlf_patch_s* p) {
   MLF_CHECK(upload_vec(p->d_fsched, fs));
   MLF_CHECK(upload_vec(p->d_bsched, bs));
   MLF_CHECK(upload_vec(p->d_rsched, rs));
-  MLF_CHECK(upload_vec(p->d_counts, std::vector<int32_t>{p->nblk_f, p->nblk_b, p->nblk_r}));
+  MLF_CHECK(upload_vec(p->d_counts, std::vector<int32_t>{p->nblk_f, p->nblk_b, p->nblk_r, p->bwd_gpe}));
   MLF_CHECK(p->partial.alloc((size_t)po));
   if (p->tpz && p->kp != Precision::kF32)
     MLF_CHECK(p->Xb.alloc((size_t)p->n1 * p->n2 * Z * kShadowRow));

@@ -132,7 +132,7 @@ struct mlf_patch_s {
   // device (slot 0) for single-patch launches
   std::vector<int32_t> fent, bent;     // (z, b1, b2, run of e1), (z, b1, b2, first group)
   int bwd_gpe = 1;                     // phase groups per entry of bent (backward_split)
-  mlf::DevBuf<int32_t> d_fsched, d_bsched, d_rsched, d_counts;  // counts: fwd, bwd, ratio
+  mlf::DevBuf<int32_t> d_fsched, d_bsched, d_rsched, d_counts;  // counts: fwd, bwd, ratio; bwd_gpe
   mlf::SlotDesc slot{};
   mlf::DevBuf<mlf::SlotDesc> d_slot;
   int nblk_f = 0, nblk_b = 0, nblk_r = 0;
