@@ -1480,9 +1480,9 @@ static bool read_volume(mlf_context ctx, const float* X, void* out, bool f64, in
       have = have && (s.ev[b] || hipEventCreateWithFlags(&s.ev[b], hipEventDisableTiming) == hipSuccess);
     }
   const hipStream_t st = ctx->read_stream;
-  // one thread waits for the volume, not all
+  // one thread waits for the volume, not all, nor a stream
   if (!have || hipEventRecord(ctx->read_ready, ctx->stream) != hipSuccess ||
-      hipStreamWaitEvent(st, ctx->read_ready, 0) != hipSuccess || hipEventSynchronize(ctx->read_ready) != hipSuccess) {
+      hipEventSynchronize(ctx->read_ready) != hipSuccess) {
     (void)hipGetLastError();
     return false;
   }
