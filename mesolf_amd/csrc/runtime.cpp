@@ -157,13 +157,15 @@ std::vector<double> filter_kernel_1d(int I, double omega) {
 }
 
 // Truncate kappa (circular) to the smallest symmetric support whose dropped
-// mass is <= 1e-10 of the total; returns (n0, taps) with taps[j] = kappa[n0+j].
+// mass is <= 1e-10 of the total, or keep the whole period if none is (an even period
+// has a middle tap that no symmetric support holds; with 30 and 60 pixels it is
+// 4e-4 and 5e-8 of the total); returns (n0, taps) with taps[j] = kappa[n0+j].
 static void truncate_kernel(const std::vector<double>& k, int* n0, std::vector<float>* taps) {
   const int I = (int)k.size();
   double total = 0.0;
   for (double v : k) total += std::fabs(v);
   const int half = (I - 1) / 2;
-  int T = half;
+  int T = I;
   double kept = std::fabs(k[0]);
   for (int t = 1; t <= half; ++t) {
     kept += std::fabs(k[t]) + std::fabs(k[I - t]);
@@ -173,7 +175,7 @@ static void truncate_kernel(const std::vector<double>& k, int* n0, std::vector<f
     }
   }
   taps->clear();
-  if (2 * T + 1 >= I) {  // full period
+  if (2 * T + 1 >= I) {
     *n0 = -((I - 1) / 2);
     for (int j = 0; j < I; ++j) taps->push_back((float)k[((*n0 + j) % I + I) % I]);
   } else {
