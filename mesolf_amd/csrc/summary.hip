@@ -411,8 +411,9 @@ __global__ __launch_bounds__(kThreads) void k_rectify(const float* __restrict__ 
 }
 
 // ---------------------------------------------------------------- tile passes
-// Movies whose tiles fit LDS (up to about 950 frames): every pass over the movie holds one tile
-// of P pixels x T frames in LDS, so a rank-1 round (Y t, then s'Y) reads the
+// Movies whose tiles fit LDS (up to 836 frames, which the last pass takes in tiles of 16
+// pixels, from 460 on; 32 below; the rounds 32 from 549 on, 64 below): every pass over
+// the movie holds one tile of P pixels x T frames in LDS, so a rank-1 round (Y t, then s'Y) reads the
 // movie once instead of twice, the first pass takes the maximum along, and the
 // last round's Y t, the detrend, the smoothing and the std image share one
 // read with no detrended movie in memory: 6 reads of the movie for 5 rounds
@@ -798,7 +799,14 @@ int tile_pixels(size_t npix, int T, int mode) {
       return P;
   return 0;
 }
-bool tiled(size_t npix, int T) { return tile_pixels(npix, T, kTileRound) && tile_pixels(npix, T, kTileLast); }
+// A tile of few frames is little work between its barriers, and a large frame has many
+// tiles: below min(60, npix / 20000 - 2) frames the passes above are the faster ones.  Time of
+// the tile passes over theirs ('pixelwise'): 400 x 400 1.07 at 4 frames, 0.67 at 16; 600 x 600 1.47 at 8,
+// 0.91 at 16; 800 x 800 1.43 at 24, 0.92 at 32; 1000 x 1000 3.0 at 4, 1.25 at 32, 1.09 at 48, 0.89 at 64;
+// 1515 x 1515 1.39 at 48, 0.94 at 64 (global: 1.12, 0.77).
+bool tiled(size_t npix, int T) {
+  return (T >= 60 || ((size_t)T + 2) * 20000 >= npix) && tile_pixels(npix, T, kTileRound) && tile_pixels(npix, T, kTileLast);
+}
 
 template <int P>
 TileKernel pick_round(int T, int mode) {
