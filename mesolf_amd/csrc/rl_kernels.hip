@@ -218,7 +218,6 @@ __global__ void k_backward_update_fp32(float* __restrict__ X, const float* __res
 }
 
 // ---------------------------------------------------------------- filter
-constexpr int kFilterThreads = 256;
 
 __device__ __forceinline__ double block_sum_f64(double v, double* sh) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;

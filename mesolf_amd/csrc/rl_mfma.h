@@ -94,7 +94,7 @@ struct FwdGeo {
 };
 
 struct RatioGeo {
-  const int32_t* sched;   // [entries][2] = (slot, first lenslet); 256 lenslets per entry
+  const int32_t* sched;   // [entries][2] = (slot, first lenslet); kRatioLens lenslets per entry
   const int32_t* count;
 };
 

@@ -1083,7 +1083,7 @@ template <typename T, int NT, int OCC, bool SPL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC)))
 void k_bwd_mfma(const T* __restrict__ Wb, BwdGeo g, float wgt) {
   using M = Mma<T>;
-  constexpr int KSTEP = M::KSTEP, KPL = M::KPL;
+  constexpr int KSTEP = M::KSTEP;
   constexpr int MT = 4;  // NT: N-tiles (16 phases each) per workgroup
   constexpr int STG = bwd_stages(OCC);  // 16-bit tap ring depth
   // M-tiles whose X (and the first 1/B1 rows) load before the K loop; with
@@ -1108,7 +1108,7 @@ void k_bwd_mfma(const T* __restrict__ Wb, BwdGeo g, float wgt) {
     // phase groups grp0 .. grp0 + groups - 1 share the entry's ratio window
     const int z = uni(cload(s + 1)), b1 = uni(cload(s + 2)), b2 = uni(cload(s + 3)), grp0 = uni(cload(s + 4));
     const int r = uni(cload(g.r + z));
-    const int K = 2 * r + 1, ntaps = K * K;
+    const int K = 2 * r + 1;
     const int epad = uni(cload(g.epad + z));
     const int64_t boffz = uni64(cload(g.boff + z));
     const int Wd = 16 + 2 * r;
@@ -1260,7 +1260,6 @@ void k_bwd_mfma(const T* __restrict__ Wb, BwdGeo g, float wgt) {
     bool pref = false;  // the group's first tap slices were issued by the previous group
     for (int gi = 0; gi < ngroups; ++gi) {  // phase group grp: 16 * NT phases from 16 * NT * grp
       const int grp = grp0 + gi;
-      const T* Bz = Wb + boffz + (size_t)(grp * 16 * NT) * epad;
       floatx4 acc[MT][NT];
   #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
@@ -1636,8 +1635,7 @@ void k_bwd_mfma(const T* __restrict__ Wb, BwdGeo g, float wgt) {
         update(std::integral_constant<bool, false>{});
         if constexpr (kTwoUpdates) wait_vm<MT * NT>();
       }
-      // LDS is reused by the next entry (the staging window aliases the
-      // ring) once every wave is here.  After an entry's last group no tap
+      // LDS is reused by the next entry once every wave is here.  After an entry's last group no tap
       // copy is in flight: that group prefetched none, its epilogue waited
       // for loads issued after its last copies, and vector-memory operations
       // complete in order; only stores may still be in flight, and they need
@@ -1755,7 +1753,7 @@ void k_bwd_split(const char* __restrict__ Wb, BwdGeo g, float wgt) {
       for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
-      floatx4 xv[MT][NT], bv[NT];
+      floatx4 xv[MT][NT];
       auto lens_of = [&](int mt) {
         const int a2 = 16 * b2 + 4 * w + mt;
         return (a2 < n2 ? a2 : n2 - 1) * n1 + a1c;

@@ -653,7 +653,6 @@ mlf_status mlf_psf_create_dense(mlf_context ctx, const float* H, const float* Ht
   const int64_t i0 = matlab_round(S / 2.0) - (int64_t)std::trunc(IMG / 2.0) - 1;
   const int R = (int)((IMG / N - 1) / 2);
   const size_t SS = (size_t)S * S;
-  const size_t slab = SS * N * N;
   auto plane_of = [&](const float* A, int a, int b, int64_t z) {
     return A + SS * ((size_t)a + (size_t)N * ((size_t)b + (size_t)N * (size_t)z));
   };

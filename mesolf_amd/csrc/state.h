@@ -56,7 +56,10 @@ struct PrecPack {
   bool built = false;
   bool tpz = false;                   // forward tables for the Toeplitz kernels: ready fragments (16-bit:
                                       // k_pack_fwd_tpz, FP32: split, k_pack_fwd_split)
-  DevBuf<uint8_t> fwd, bwd;           // [V][z][e_pad64][PHI], [V][z][kPhiPadBwd][e_pad32]
+  // fwd: [V][z], then with tpz [e1][N-tile][K-step][lane][8] (FP32: [half] before it,
+  // [part] before the lane), else rows [e_pad64][PHI]; bwd: [V][z][16-phase tile][K-step],
+  // then [16 rows][32 taps] (FP32: [part][lane][8])
+  DevBuf<uint8_t> fwd, bwd;
   int64_t pvf = 0, pvb = 0;           // elements per view
   std::vector<int64_t> woff, boff;    // per-plane element offsets inside a view
   std::vector<int32_t> nchunk, epad;
@@ -94,8 +97,6 @@ struct mlf_psf_s {
   mlf::PrecPack pack[mlf::kPrecisions];
   std::vector<std::unique_ptr<mlf::NormTable>> norms[mlf::kPrecisions];
   std::mutex mu;
-  ReadSlot read[kReadThreads];  // guarded by read_mu; made on first use, freed with the context
-  std::mutex read_mu;
   int refs = 0;         // live patches
   bool closed = false;
 };

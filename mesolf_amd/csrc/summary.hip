@@ -506,7 +506,7 @@ __device__ __forceinline__ size_t first_tile() {
   return n % 8 == 0 ? (blockIdx.x & 7) * (n / 8) + (blockIdx.x >> 3) : blockIdx.x;
 }
 
-// tile -> LDS; `t` (null: not wanted): this thread's part of Y t
+// tile -> LDS; each(j, x): this thread's samples x of frame j
 template <int P, int R, typename F>
 __device__ __forceinline__ void tile_store(const TileRegs<P, R>& regs, float* Yt, int T, bool in, F&& each) {
   constexpr int G = kTileThreads / P, LD = P + 1;
@@ -808,11 +808,11 @@ bool tiled(size_t npix, int T) {
   return (T >= 60 || ((size_t)T + 2) * 20000 >= npix) && tile_pixels(npix, T, kTileRound) && tile_pixels(npix, T, kTileLast);
 }
 
-template <int P>
-TileKernel pick_round(int T, int mode) {
-  const bool small = T <= 16 * (kTileThreads / P);
-  if (mode == kTileFirst) return small ? &k_summary_round<P, 16, kTileFirst> : &k_summary_round<P, 40, kTileFirst>;
-  return small ? &k_summary_round<P, 16, kTileRound> : &k_summary_round<P, 40, kTileRound>;
+// 64 pixels take 16 registers for up to 256 frames, 40 up to 548; 32 pixels come
+// from 549 on and take 40
+template <int P, int R>
+TileKernel pick_round(int mode) {
+  return mode == kTileFirst ? &k_summary_round<P, R, kTileFirst> : &k_summary_round<P, R, kTileRound>;
 }
 template <int P>
 TileKernel pick_last(int mode) {
@@ -824,8 +824,9 @@ constexpr int kTileWgs = 1024;  // most workgroups of a pass
 hipError_t launch_tile(const TileArgs& g, int mode, int cus, int* nwg, hipStream_t st) {
   const int P = tile_pixels(g.npix, g.T, mode);
   const size_t lds = tile_lds(P, g.T, mode);
-  const TileKernel fn = mode <= kTileRound ? (P == 64 ? pick_round<64>(g.T, mode) : pick_round<32>(g.T, mode))
-                                           : (P == 32 ? pick_last<32>(mode) : pick_last<16>(mode));
+  const TileKernel fn = mode <= kTileRound
+                            ? (P == 32 ? pick_round<32, 40>(mode) : g.T <= 256 ? pick_round<64, 16>(mode) : pick_round<64, 40>(mode))
+                            : (P == 32 ? pick_last<32>(mode) : pick_last<16>(mode));
   const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTileLds);
   if (e != hipSuccess) return e;
