@@ -86,6 +86,7 @@ extern "C" mlf_status mlf_lfm_convolution_vec_noalloc(mlf_context ctx, const flo
       if (n > kNoAllocImages || mex_scratch_floats((int)kw, kNoAllocImages) > kNoAllocFloats)
         return set_error(MLF_ERR_INTERNAL, "scratch too small for kw %lld", (long long)kw);
     }
+    std::lock_guard<std::mutex> lk(ctx->mu);  // the call's launches follow one another
     MexCall c = mex_begin(n, (int)kw, d_bitmap, mem, kNoAllocImages);
     MLF_LAUNCH(launch_mex_mfma(c, d_bitmap, width, height, n, d_kernels, true, true, nullptr, nullptr, d_out,
                                ctx->stream));
