@@ -210,7 +210,9 @@ mlf_status mlf_patch_kernel_times(mlf_patch p, double* total_ms, int64_t* launch
  * keep their own image and volume; attach them after set_image and
  * init_volume / set_volume.  A destroyed
  * patch is detached first.  Calls on one batch are serialized; running a
- * batch and one of its patches from two threads at once is not supported. */
+ * batch and one of its patches from two threads at once is not supported.
+ * Reading a patch's volume beside it is: what is read is one state, and a run
+ * started meanwhile waits until a large volume is out. */
 typedef struct mlf_batch_s* mlf_batch;
 mlf_status mlf_batch_create(mlf_psf psf, mlf_precision prec, int32_t capacity, mlf_batch* out);
 mlf_status mlf_batch_destroy(mlf_batch b);
