@@ -21,6 +21,10 @@ def _inputs(W, H, n, kw, seed=17):
     (47, 33, 31, (1, 2, 3, 5, 9, 17, 33, 65, 160)), (150, 137, 61, (1, 2, 4, 8, 16, 48, 96)),
     (16, 5, 5, (1, 7, 60, 300)), (90, 7, 241, (1, 3, 20, 90)), (396, 110, 121, (1, 2, 4, 9, 24, 50)),
     (31, 200, 7, (1, 4, 30, 120)), (225, 60, 13, (1, 8, 64)),
+    # many rows and several lengths of batch: the shapes of three and four rows to a
+    # workgroup, and those of many cells, each against one bitmap's small shape
+    (130, 513, 61, (1, 4, 8, 16, 30, 60)), (130, 513, 17, (1, 8, 16, 30, 60)), (77, 1501, 33, (1, 16, 30)),
+    (640, 9, 5, (1, 24, 48)),
 ])
 def test_any_number_of_bitmaps(W, H, kw, counts):
     b, K = _inputs(W, H, counts[-1], kw)
